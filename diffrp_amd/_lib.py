@@ -63,6 +63,8 @@ _SIGS = {
     'drp_sample2d_fwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int, c_void_p]),
     'drp_sample2d_bwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int, c_void_p,
                                  c_void_p, c_void_p]),
+    'drp_sample2d_image_bwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int, c_int,
+                                       c_void_p, c_void_p, c_void_p]),
     'drp_sample3d_fwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int,
                                  c_void_p]),
     'drp_sample3d_bwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int,

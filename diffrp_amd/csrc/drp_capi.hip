@@ -1060,14 +1060,21 @@ int drp_sample2d_fwd(void *stream, const float *tex, int H, int W, int C, const 
     return 0;
 }
 
-int drp_sample2d_bwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n, int wrap,
-                     int mode, const float *grad_out, float *grad_tex, float *grad_uv) {
+int drp_sample2d_image_bwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n,
+                           int width, int wrap, int mode, const float *grad_out, float *grad_tex, float *grad_uv) {
     if (int e = tex_check(1, H, W, C, n, wrap, mode, true)) return e;
+    if (width < 0) return fail(-1, "negative row width");
     if (n == 0) return 0;
     if (!tex || !uv || !grad_out) return fail(-1, "null pointer argument");
-    int rc = launch_sample2d_bwd(tex, H, W, C, uv, n, wrap, mode, grad_out, grad_tex, grad_uv, (hipStream_t)stream);
+    int rc = launch_sample2d_bwd(tex, H, W, C, uv, n, width, wrap, mode, grad_out, grad_tex, grad_uv,
+                                 (hipStream_t)stream);
     if (rc) return fail(rc, "sample2d backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
+}
+
+int drp_sample2d_bwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n, int wrap,
+                     int mode, const float *grad_out, float *grad_tex, float *grad_uv) {
+    return drp_sample2d_image_bwd(stream, tex, H, W, C, uv, n, 0, wrap, mode, grad_out, grad_tex, grad_uv);
 }
 
 int drp_sample3d_fwd(void *stream, const float *tex, int D, int H, int W, int C, const float *uvw, long long n,

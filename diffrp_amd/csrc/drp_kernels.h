@@ -225,8 +225,8 @@ size_t incidence_ws_bytes(int V, int F);
 size_t stencil_partition_ws_bytes(long long npx, int n_owner);
 int launch_sample2d(const float *tex, int H, int W, int C, const float *uv, long long n, int wrap, int mode,
                     float *out, hipStream_t st);
-int launch_sample2d_bwd(const float *tex, int H, int W, int C, const float *uv, long long n, int wrap, int mode,
-                        const float *gout, float *gtex, float *guv, hipStream_t st);
+int launch_sample2d_bwd(const float *tex, int H, int W, int C, const float *uv, long long n, int width, int wrap,
+                        int mode, const float *gout, float *gtex, float *guv, hipStream_t st);
 int launch_sample3d(const float *tex, int D, int H, int W, int C, const float *uvw, long long n, int wrap, int mode,
                     float *out, hipStream_t st);
 int launch_sample3d_bwd(const float *tex, int D, int H, int W, int C, const float *uvw, long long n, int wrap,

@@ -189,11 +189,16 @@ int drp_rasterize_bwd(void *stream, const float *pos, int n_img, int V, int pos_
  * row).  wrap: 0 border, 1 reflection, 2 cyclic (2-D only), 3 latlong
  * (reflection, align_corners); mode: 0 bilinear, 1 nearest (no coordinate
  * gradient), 2 bicubic (2-D only; Keys A = -0.75, padding per tap).  out [n,C].  Backward: grad_tex accumulated (float atomics, may
- * be NULL), grad_uv / grad_uvw written (may be NULL). */
+ * be NULL), grad_uv / grad_uvw written (may be NULL).  The image form of the
+ * 2-D backward names the samples' row width (samples i and i + width are
+ * vertical neighbours; 0: unknown), so that neighbours' texture gradients are
+ * summed before the atomics. */
 int drp_sample2d_fwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n, int wrap,
                      int mode, float *out);
 int drp_sample2d_bwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n, int wrap,
                      int mode, const float *grad_out, float *grad_tex, float *grad_uv);
+int drp_sample2d_image_bwd(void *stream, const float *tex, int H, int W, int C, const float *uv, long long n,
+                           int width, int wrap, int mode, const float *grad_out, float *grad_tex, float *grad_uv);
 int drp_sample3d_fwd(void *stream, const float *tex, int D, int H, int W, int C, const float *uvw, long long n,
                      int wrap, int mode, float *out);
 int drp_sample3d_bwd(void *stream, const float *tex, int D, int H, int W, int C, const float *uvw, long long n,
