@@ -17,6 +17,7 @@
 // fixed order), and the backward counterparts.
 #include "drp_common.h"
 #include "drp_kernels.h"
+#include "drp_wave.h"
 
 namespace drp {
 
@@ -421,16 +422,10 @@ __global__ void __launch_bounds__(256, 8) k_aa_pairs(AALaunch L, float2 *__restr
     if (tid == 0) q_n = 0;
     __syncthreads();
     // wave-aggregated append
-    int x = nq;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    const int wtot = __shfl(x, 63, 64);
+    const int x = wave_incl_scan(nq);
     int base = 0;
-    if (lane == 63 && wtot > 0) base = atomicAdd(&q_n, wtot);
-    base = __shfl(base, 63, 64) + x - nq;
+    if (lane == 63 && x > 0) base = atomicAdd(&q_n, x);
+    base = __builtin_amdgcn_readlane(base, 63) + x - nq;
 #pragma unroll
     for (int j = 0; j < kAAPairPer; ++j) {
         if (cand[j] & 1) q[base++] = tid + 256 * j;
@@ -756,15 +751,10 @@ __global__ void __launch_bounds__(256) k_aa_pairs_bwd(AALaunch L, float2 *__rest
         if (!want_pos || !live_block) continue;  // uniform across the block
         // wave-aggregated append of the pixel's queued pairs
         const int lane = tid & 63;
-        int x = nq;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            int y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        int wtot = __shfl(x, 63, 64), base = 0;
-        if (lane == 63 && wtot > 0) base = atomicAdd(&q_n, wtot);
-        base = __shfl(base, 63, 64) + x - nq;
+        const int x = wave_incl_scan(nq);
+        int base = 0;
+        if (lane == 63 && x > 0) base = atomicAdd(&q_n, x);
+        base = __builtin_amdgcn_readlane(base, 63) + x - nq;
         if (nq > 0) {
             q_tri[base] = qa.tri;
             q_meta[base] = px | (da << 10) | ((qa.recv << 4 | qa.clamped << 3 | qa.from_a << 2 | qa.edge) << 11);

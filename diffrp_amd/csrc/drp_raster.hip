@@ -21,6 +21,7 @@
 #include "drp_common.h"
 #include "drp_grad.h"
 #include "drp_kernels.h"
+#include "drp_wave.h"
 
 namespace drp {
 
@@ -102,14 +103,9 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
     // full pair goes to the spill list.  (Every shuffle and ballot below runs
     // in wave-uniform control flow.)
     constexpr unsigned kNoTile = (1u << 26) - 1;  // tile field of a lane with nothing to insert
-    int incl = mine;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += y;
-    }
+    const int incl = wave_incl_scan(mine);
     const int excl = incl - mine;
-    const int total = __shfl(incl, 63, 64);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
     for (int r0 = 0; r0 < total; r0 += 64) {
         const int p = r0 + lane;
         const bool active = p < total;
@@ -127,7 +123,7 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
             const int ty = py0 + k / nc, tx = px0 + k % nc;
             key = ((unsigned)(ty * d.tiles_x + tx) << 6) | (unsigned)lane;
         }
-        const unsigned sk = wave_sort64<unsigned>(key);
+        const unsigned sk = wave_sort(key);
         const unsigned tl = sk >> 6;
         const int src = (int)(sk & 63);
         const bool valid = tl != kNoTile;
@@ -249,28 +245,6 @@ __device__ __forceinline__ void row_span32(const FineRec &R, int box, int y, int
         xl = nxl;
         xr = nxr;
     }
-}
-
-template <int NT>
-__device__ __forceinline__ int block_excl_scan(int v, int *wsum, int &total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wave] = x;
-    __syncthreads();
-    int pre = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) {
-        int s = wsum[w];
-        if (w < wave) pre += s;
-        tot += s;
-    }
-    total = tot;
-    return pre + x - v;
 }
 
 __device__ __forceinline__ float inv_ord_f32(uint32_t k) {
@@ -524,7 +498,7 @@ __device__ __forceinline__ void fine_entries(FineLds<TW, TH, PEEL> &S, const Fin
                 count = 0;
         }
         int nrows;
-        const int ex = block_excl_scan<NT>(count, S.wsum, nrows);  // this lane's record owns rows [ex, ex + count)
+        const int ex = block_scan<NT>(count, S.wsum, nrows);  // this lane's record owns rows [ex, ex + count)
         // Row items (record, tile row) in sub-rounds of NT: each lane finds the
         // exact covered span of its row; the covered pixels are queued (block
         // prefix sum, at most kQueue per pass) and evaluated by all lanes, so
@@ -552,7 +526,7 @@ __device__ __forceinline__ void fine_entries(FineLds<TW, TH, PEEL> &S, const Fin
                 len = max(xr - xl + 1, 0);
             }
             int npix;
-            const int off = block_excl_scan<NT>(len, S.wsum + (NT / 64) * (1 + par), npix);
+            const int off = block_scan<NT>(len, S.wsum + (NT / 64) * (1 + par), npix);
             for (int q0 = 0; q0 < npix; q0 += kQueue) {
                 const int lo = max(off, q0), hi = min(off + len, q0 + kQueue);
                 for (int i = lo; i < hi; ++i) S.queue[i - q0] = k | ((xl + i - off) << 8) | (y << 16);

@@ -25,6 +25,7 @@
 #include "drp_common.h"
 #include "drp_grad.h"
 #include "drp_kernels.h"
+#include "drp_wave.h"
 
 namespace drp {
 
@@ -50,27 +51,6 @@ __device__ __forceinline__ int count_below64(const K *a, K k) {
     for (int half = 32; half >= 1; half >>= 1)
         if (a[base + half - 1] < k) base += half;
     return base + (a[base] < k ? 1 : 0);
-}
-
-__device__ __forceinline__ int block_excl_scan256(int v, int *wsum, int &total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[wave] = x;
-    __syncthreads();
-    int pre = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        int s = wsum[w];
-        if (w < wave) pre += s;
-        tot += s;
-    }
-    total = tot;
-    return pre + x - v;
 }
 
 // Quads [q0, q0 + NQP) of every segment's record: one thread per (segment,
@@ -279,7 +259,7 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C>())) k_tile_reduce(
     // each wave sorts its 64 across lanes, then every key's place is its lane
     // plus the keys below it in the other three runs
     {
-        K k = wave_sort64<K>(((t >= 0 ? (K)t : kEmptyT) << 8) | (K)tid);
+        K k = wave_sort(((t >= 0 ? (K)t : kEmptyT) << 8) | (K)tid);
         const int wave = tid >> 6;
         U.run[tid] = k;
         __syncthreads();
@@ -308,7 +288,7 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C>())) k_tile_reduce(
     bool valid = (sk >> 8) != kEmptyT;
     bool head = valid && (tid == 0 || (key[tid - 1] >> 8) != (sk >> 8));
     int nseg;
-    int seg = block_excl_scan256(head ? 1 : 0, wsum, nseg);
+    int seg = block_scan<kBTP>(head ? 1 : 0, wsum, nseg);
     int nvalid = __syncthreads_count(valid);
     if (head) U.seg_start[seg] = tid;
     if (tid == 0) U.seg_start[nseg] = nvalid;
