@@ -384,7 +384,7 @@ class _URasterize(torch.autograd.Function):
         return _rasterize_bwd(ub.plan, pos, ub.tri, rast, False, grast, None, boxes, ub.inc), None
 
 
-_FUSED_C = (4, 8)  # channel counts of the fused attribute + position backward (tests switch it off)
+_FUSED_C = (1, 2, 3, 4, 8, 16)  # channel counts of the fused attribute + position backward (tests switch it off)
 
 
 class _UInterpolate(torch.autograd.Function):

@@ -509,6 +509,9 @@ int drp_batch_interpolate_fwd(void *stream, const void *plan, const float *attr,
     return 0;
 }
 
+// the tile backward takes at most kMaxPassChannels channels at a time
+static int pass_width(int C) { return C < kMaxPassChannels ? C : kMaxPassChannels; }
+
 static size_t batch_interp_partial_bytes(const BatchPlanHeader &h, int C) {
     return align256((size_t)h.n_tri * 3 * (size_t)C * 4);
 }
@@ -518,7 +521,7 @@ size_t drp_batch_interpolate_bwd_workspace_size(const void *plan, int C) {
     if (!plan || C <= 0) return 0;
     memcpy(&v.h, plan, sizeof(v.h));
     long long tiles = plan_map(plan, v.h.n_img, v.h.n_tiles).bt16[v.h.n_img];
-    return batch_interp_partial_bytes(v.h, C) + tile_records_bytes_tiles(tiles, 3 * C, v.h.n_tri);
+    return batch_interp_partial_bytes(v.h, C) + tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, false), v.h.n_tri);
 }
 
 int drp_batch_interpolate_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr, int C,
@@ -577,7 +580,7 @@ size_t drp_batch_interpolate_rasterize_bwd_workspace_size(const void *plan, int 
     if (h.n_tri <= 0) return 0;
     long long tiles = plan_map(plan, h.n_img, h.n_tiles).bt16[h.n_img];
     return align256((size_t)h.n_tri * 3 * (size_t)C * 4) + align256((size_t)h.n_tri * 3 * 16) +
-           tile_records_bytes_tiles(tiles, 3 * C + 12, h.n_tri) + align256((size_t)h.n_tri * 3 * 4);
+           tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, true), h.n_tri) + align256((size_t)h.n_tri * 3 * 4);
 }
 
 int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr,
@@ -587,12 +590,14 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
                                         void *workspace, size_t workspace_bytes) {
     PlanView v;
     if (int e = plan_view(plan, plan_dev, v)) return e;
-    if (!(C == 4 || C == 8)) return fail(-1, "the fused backward takes C in {4, 8} (got %d)", C);
+    if (C < 1 || C > kMaxPassChannels)
+        return fail(-1, "the fused backward takes 1 to %d channels (got %d)", kMaxPassChannels, C);
     if (v.h.n_pix == 0 || v.h.n_tri == 0 || v.h.n_vert == 0) return 0;
     if (!attr || !pos || !rast || !tri || !grad_out || !grad_attr || !grad_pos || !boxes || !inc_off || !inc)
         return fail(-1, "null pointer argument");
-    if (!aligned16(attr) || !aligned16(pos) || !aligned16(rast) || !aligned16(grad_out) || !aligned16(grad_pos))
-        return fail(-1, "attr, pos, rast, grad_out and grad_pos must be 16-byte aligned");
+    if (!aligned16(pos) || !aligned16(rast) || !aligned16(grad_pos) ||
+        (C % 4 == 0 && (!aligned16(attr) || !aligned16(grad_out))))
+        return fail(-1, "pos, rast and grad_pos (and attr, grad_out when C %% 4 == 0) must be 16-byte aligned");
     const size_t need = drp_batch_interpolate_rasterize_bwd_workspace_size(plan, C);
     if (!workspace || workspace_bytes < need)
         return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -603,7 +608,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     float *partial_pos = (float *)b;
     b += align256((size_t)F * 3 * 16);
     void *records = b;
-    b += tile_records_bytes_tiles(v.bt16, 3 * C + 12, F);
+    b += tile_records_bytes_tiles(v.bt16, tile_record_floats(C, true, true), F);
     int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
     if (int rc = launch_corner_slots(inc, inc_off, V, F, slot, st))
@@ -622,6 +627,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     T.attr = attr;
     T.V = V;
     T.attr_batched = 0;
+    T.ldc = C;
     T.grad_rast_out = nullptr;
     T.boxes = (const ItemBox *)boxes;
     T.partial = partial_attr;
@@ -638,7 +644,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     int rc = launch_tri_bwd_fused(T, C, st);
     Fork f{};  // the two vertex gathers are independent
     const bool par = !rc && fork_begin(st, f);
-    if (!rc) rc = launch_gather_attr(partial_attr, 1, F, V, C, inc_off, inc, grad_attr, par ? f.side : st);
+    if (!rc) rc = launch_gather_attr(partial_attr, 1, F, V, C, C, 0, 1, 0, inc_off, inc, grad_attr, par ? f.side : st);
     if (!rc) rc = launch_gather_pos(partial_pos, 1, F, V, 0, inc_off, grad_pos, st);
     if (par && fork_end(st, f)) rc = -2;
     if (rc) return fail(rc, "batch fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
@@ -875,14 +881,14 @@ int drp_interpolate_fwd(void *stream, const float *attr, int n_img, int V, int a
 static size_t interp_partial_bytes(int n_img, int F, int C, int attr_batched, int views_per_group) {
     int vpg = attr_batched ? 1 : views_per_block(views_per_group);
     size_t groups = ((size_t)n_img + vpg - 1) / vpg;
-    return align256(groups * (size_t)F * 3 * (size_t)C * 4);
+    return align256(groups * (size_t)F * 3 * (size_t)pass_width(C) * 4);
 }
 
 size_t drp_interpolate_bwd_workspace_size(int n_img, int H, int W, int F, int C, int attr_batched,
                                           int views_per_group) {
     if (n_img <= 0 || F <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
     return interp_partial_bytes(n_img, F, C, attr_batched, views_per_group) +
-           tile_records_bytes(n_img, H, W, 3 * C, (long long)n_img * F);
+           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, false), (long long)n_img * F);
 }
 
 int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int attr_batched, int C,
@@ -922,13 +928,21 @@ int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int a
     L.H = H;
     L.W = W;
     L.views_per_group = attr_batched ? 1 : views_per_block(views_per_group);
-    bool tri_path = F > 0 && boxes && inc_off && inc && n_diff == 0 && L.cv > 0;
+    // the tile passes, given pixel boxes; channel counts without a compiled
+    // forward and derivative gradients may also come without the workspace or
+    // the alignment they need (per-pixel atomics then)
+    bool tri_path = F > 0 && boxes && inc_off && inc && (n_diff == 0 || grad_da);
     if (tri_path) {
-        size_t need = drp_interpolate_bwd_workspace_size(n_img, H, W, F, C, attr_batched, L.views_per_group);
-        if (!workspace || workspace_bytes < need)
-            return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-        if (C % 4 == 0 && (!aligned16(grad_out) || (V > 0 && !aligned16(attr))))
-            return fail(-1, "grad_out and attr must be 16-byte aligned when C %% 4 == 0");
+        const size_t need = drp_interpolate_bwd_workspace_size(n_img, H, W, F, C, attr_batched, L.views_per_group);
+        const bool room = workspace && workspace_bytes >= need;
+        const bool quads = C % 4 != 0 || (aligned16(grad_out) && (V == 0 || aligned16(attr)));
+        if (n_diff == 0 && L.cv > 0) {
+            if (!room) return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
+            if (!quads) return fail(-1, "grad_out and attr must be 16-byte aligned when C %% 4 == 0");
+        }
+        tri_path = room && quads;
+    }
+    if (tri_path) {
         L.boxes = (const ItemBox *)boxes;
         L.partial = (float *)workspace;
         L.records = (char *)workspace + interp_partial_bytes(n_img, F, C, attr_batched, L.views_per_group);
@@ -947,7 +961,7 @@ size_t drp_interpolate_rasterize_bwd_workspace_size(int n_img, int H, int W, int
     const int vpg = views_per_block(views_per_group);
     const size_t groups = (size_t)((n_img + vpg - 1) / vpg);
     return align256(groups * (size_t)F * 3 * (size_t)C * 4) + align256((size_t)n_img * (size_t)F * 3 * 16) +
-           tile_records_bytes(n_img, H, W, 3 * C + 12, (long long)n_img * F) + align256((size_t)F * 3 * 4);
+           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F) + align256((size_t)F * 3 * 4);
 }
 
 int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
@@ -957,13 +971,14 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
                                   const int32_t *inc, void *workspace, size_t workspace_bytes) {
     if (int e = check_dims(n_img, H, W)) return e;
     if (n_img == 0) return 0;
-    if (!(C == 4 || C == 8)) return fail(-1, "the fused backward takes C in {4, 8} (got %d)", C);
+    if (C < 1 || C > kMaxPassChannels)
+        return fail(-1, "the fused backward takes 1 to %d channels (got %d)", kMaxPassChannels, C);
     if (F <= 0 || V <= 0) return fail(-1, "the fused backward needs triangles and vertices");
     if (!attr || !rast || !tri || !pos || !grad_out || !grad_attr || !grad_pos || !boxes || !inc_off || !inc)
         return fail(-1, "null pointer argument");
     if (!aligned16(rast) || (grad_rast && !aligned16(grad_rast)) || !aligned16(pos) || !aligned16(grad_pos) ||
-        !aligned16(grad_out) || !aligned16(attr))
-        return fail(-1, "rast, grad_rast, pos, grad_pos, grad_out and attr must be 16-byte aligned");
+        (C % 4 == 0 && (!aligned16(grad_out) || !aligned16(attr))))
+        return fail(-1, "rast, grad_rast, pos and grad_pos (and grad_out, attr when C %% 4 == 0) must be 16-byte aligned");
     const size_t need = drp_interpolate_rasterize_bwd_workspace_size(n_img, H, W, F, C, views_per_group);
     if (!workspace || workspace_bytes < need)
         return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -975,7 +990,7 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     float *partial_pos = (float *)b;
     b += align256((size_t)n_img * (size_t)F * 3 * 16);
     void *records = b;
-    b += tile_records_bytes(n_img, H, W, 3 * C + 12, (long long)n_img * F);
+    b += tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F);
     int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
     if (int rc = launch_corner_slots(inc, inc_off, V, F, slot, st))
@@ -994,6 +1009,7 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     T.attr = attr;
     T.V = V;
     T.attr_batched = 0;
+    T.ldc = C;
     T.grad_rast_out = grad_rast;
     T.boxes = (const ItemBox *)boxes;
     T.partial = partial_attr;
@@ -1008,7 +1024,7 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     int rc = launch_tri_bwd_fused(T, C, st);
     Fork f{};  // the two vertex gathers are independent
     const bool par = !rc && fork_begin(st, f);
-    if (!rc) rc = launch_gather_attr(partial_attr, groups, F, V, C, inc_off, inc, grad_attr, par ? f.side : st);
+    if (!rc) rc = launch_gather_attr(partial_attr, groups, F, V, C, C, 0, 1, 0, inc_off, inc, grad_attr, par ? f.side : st);
     if (!rc) rc = launch_gather_pos(partial_pos, n_img, F, V, pos_batched, inc_off, grad_pos, st);
     if (par && fork_end(st, f)) rc = -2;
     if (rc) return fail(rc, "fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));

@@ -168,73 +168,26 @@ int launch_interpolate(const InterpLaunch &L, hipStream_t st) {
 
 // ----------------------------------------------------------------------------
 // deterministic backward (no atomics)
-//   k_tile_reduce / k_tile_gather (drp_tribwd.hip): grad_rast per pixel and,
+//   k_tile_reduce / k_tile_gather (drp_tribwd.h): grad_rast per pixel and,
 //       per (view group, triangle), (u, v, 1-u-v) * g per corner
-//   k_gather_attr: per vertex, sum the corner partials (CSR, fixed order)
+//   k_gather_attr_*: per vertex, sum the corner partials (CSR, fixed order)
+// Any channel count and the derivatives' gradients: the per-pixel atomics of
+// k_interp_bwd above remain for rast that comes without pixel boxes (range
+// mode, a modified rast).
 // ----------------------------------------------------------------------------
-// grad_attr[out][v] += sum over groups g in the output's range and incident corners
-template <int NC>
-__global__ void __launch_bounds__(256) k_gather_attr(const float *__restrict__ partial, int n_groups, int F, int V,
-                                                     int per_output_groups, const int *__restrict__ inc_off,
-                                                     const int *__restrict__ inc, float *__restrict__ grad_attr) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    int out = blockIdx.y;
-    if (v >= V) return;
-    float s[NC];
-#pragma unroll
-    for (int ch = 0; ch < NC; ++ch) s[ch] = 0.f;
-    int i0 = inc_off[v], i1 = inc_off[v + 1];
-    int g0 = per_output_groups ? out : 0, g1 = per_output_groups ? out + 1 : n_groups;
-    for (int g = g0; g < g1; ++g) {
-        const float *P = partial + (long long)g * F * 3 * NC;
-        if (NC % 4 == 0 && NC <= 8) {
-            // four corners' loads in flight at once (corner partials are NC * 4 bytes from an
-            // aligned base), summed in corner order
-            for (int i = i0; i < i1; i += 4) {
-                float4 x[4][NC / 4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) {
-                        const float4 *q = reinterpret_cast<const float4 *>(P + (long long)inc[i + k] * NC);
-#pragma unroll
-                        for (int h = 0; h < NC / 4; ++h) x[k][h] = q[h];
-                    }
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) {
-#pragma unroll
-                        for (int h = 0; h < NC / 4; ++h) {
-                            s[4 * h] += x[k][h].x; s[4 * h + 1] += x[k][h].y;
-                            s[4 * h + 2] += x[k][h].z; s[4 * h + 3] += x[k][h].w;
-                        }
-                    }
-            }
-        } else {
-            for (int i = i0; i < i1; ++i) {
-                const float *q = P + (long long)inc[i] * NC;
-#pragma unroll
-                for (int ch = 0; ch < NC; ++ch) s[ch] += q[ch];
-            }
-        }
-    }
-    float *o = grad_attr + ((long long)out * V + v) * NC;
-#pragma unroll
-    for (int ch = 0; ch < NC; ++ch) o[ch] += s[ch];
-}
-
-// The same for 8 and 16 channels with `lanes` lanes per (vertex, four
-// channels) (1, 2 or 4: up to the groups each output sums): lane s takes
-// groups s, s + lanes, ... (two groups' corner rows in flight together, each
-// group's corners summed in order), and the lanes' sums are added in a fixed
-// tree.  (One lane per (vertex, quad) left the 64-view grid at barely one wave
-// per SIMD waiting on its loads.)
+// grad_attr[out][v][c0 ..) += sum over groups g in the output's range and
+// incident corners, channel counts that are whole quads, with `lanes` lanes per
+// (vertex, four channels) (1, 2 or 4: up to the groups each output sums): lane
+// s takes groups s, s + lanes, ... (two groups' corner rows in flight together,
+// each group's corners summed in order), and the lanes' sums are added in a
+// fixed tree.  (One lane per (vertex, quad) left the 64-view grid at barely one
+// wave per SIMD waiting on its loads.)
 constexpr int kAttrLanes = 4;
-template <int NC>
 __global__ void __launch_bounds__(256) k_gather_attr_q(const float *__restrict__ partial, int n_groups, int F,
-                                                       int V, int per_output_groups, const int *__restrict__ inc_off,
-                                                       const int *__restrict__ inc, float *__restrict__ grad_attr,
-                                                       int lanes) {
-    constexpr int NQ = NC / 4;
+                                                       int V, int NC, int ldc, int c0, int per_output_groups,
+                                                       const int *__restrict__ inc_off, const int *__restrict__ inc,
+                                                       float *__restrict__ grad_attr, int lanes) {
+    const int NQ = NC / 4;
     const long long tl = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int s = (int)(tl & (lanes - 1));
     const long long tq = tl / lanes;
@@ -290,30 +243,66 @@ __global__ void __launch_bounds__(256) k_gather_attr_q(const float *__restrict__
         acc.w += __shfl_xor(acc.w, o, 64);
     }
     if (s != 0) return;
-    float *o = grad_attr + ((long long)out * V + v) * NC + 4 * q;
+    float *o = grad_attr + ((long long)out * V + v) * ldc + c0 + 4 * q;
     o[0] += acc.x;
     o[1] += acc.y;
     o[2] += acc.z;
     o[3] += acc.w;
 }
 
-template <int NC>
-static void launch_gather_attr_t(const float *partial, int groups, int F, int V, int outs, int per_output_groups,
-                                 const int *inc_off, const int *inc, float *grad_attr, hipStream_t st) {
-    if constexpr (NC == 8 || NC == 16) {
-        const int per_out = per_output_groups ? 1 : groups;
-        const int lanes = per_out >= kAttrLanes ? kAttrLanes : (per_out >= 2 ? 2 : 1);
-        const long long n = (long long)V * (NC / 4) * lanes;
-        hipLaunchKernelGGL(k_gather_attr_q<NC>, dim3((unsigned)((n + 255) / 256), outs), dim3(256), 0, st, partial,
-                           groups, F, V, per_output_groups, inc_off, inc, grad_attr, lanes);
-    } else {
-        hipLaunchKernelGGL(k_gather_attr<NC>, dim3((V + 255) / 256, outs), dim3(256), 0, st, partial, groups, F, V,
-                           per_output_groups, inc_off, inc, grad_attr);
+// The same one lane per (vertex, channel), for channel counts that are not
+// whole quads: consecutive lanes read consecutive floats of a corner's row;
+// four corners' loads in flight, summed in corner order.
+__global__ void __launch_bounds__(256) k_gather_attr_c(const float *__restrict__ partial, int n_groups, int F,
+                                                       int V, int NC, int ldc, int c0, int per_output_groups,
+                                                       const int *__restrict__ inc_off, const int *__restrict__ inc,
+                                                       float *__restrict__ grad_attr) {
+    const long long tl = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = (int)(tl / NC), ch = (int)(tl - (long long)v * NC);
+    const int out = blockIdx.y;
+    if (v >= V) return;
+    const int i0 = inc_off[v], i1 = inc_off[v + 1];
+    const int g0 = per_output_groups ? out : 0, g1 = per_output_groups ? out + 1 : n_groups;
+    float s = 0.f;
+    for (int g = g0; g < g1; ++g) {
+        const float *P = partial + (long long)g * F * 3 * NC + ch;
+        for (int i = i0; i < i1; i += 4) {
+            float x[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = i + k < i1 ? P[(long long)inc[i + k] * NC] : 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (i + k < i1) s += x[k];
+        }
     }
+    grad_attr[((long long)out * V + v) * ldc + c0 + ch] += s;
 }
 
-template <int NC>
-static void launch_interp_bwd_tri_t(const InterpLaunch &L, hipStream_t st) {
+int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
+                       int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st) {
+    if (V == 0) return 0;
+    if (C % 4 == 0) {
+        const int per_out = per_output ? 1 : groups;
+        const int lanes = per_out >= kAttrLanes ? kAttrLanes : (per_out >= 2 ? 2 : 1);
+        const long long n = (long long)V * (C / 4) * lanes;
+        hipLaunchKernelGGL(k_gather_attr_q, dim3((unsigned)((n + 255) / 256), outs), dim3(256), 0, st, partial,
+                           groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr, lanes);
+    } else {
+        hipLaunchKernelGGL(k_gather_attr_c, dim3((unsigned)(((long long)V * C + 255) / 256), outs), dim3(256), 0, st,
+                           partial, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+// channels of the next pass over an attribute of C channels, `left` to go: at
+// most `most`, and where the rows are not whole quads no multiple of 4 (those
+// passes read 16 bytes at a time)
+static int pass_channels(int left, int C, int most) {
+    const int k = left < most ? left : most;
+    return C % 4 && k % 4 == 0 ? k - 1 : k;
+}
+
+static int launch_interp_bwd_tri(const InterpLaunch &L, hipStream_t st) {
     int n_img = L.um.n ? 1 : (int)(L.total_pix / L.pix_per_img);  // an uneven batch sums as one group
     int vpg = L.attr_batched ? 1 : L.views_per_group;
     int groups = (n_img + vpg - 1) / vpg;
@@ -324,7 +313,13 @@ static void launch_interp_bwd_tri_t(const InterpLaunch &L, hipStream_t st) {
     T.attr = L.attr;
     T.V = L.V;
     T.attr_batched = L.attr_batched;
+    T.ldc = L.C;
     T.grad_rast_out = L.grad_rast;
+    T.rast_db = L.rast_db;
+    T.diff_idx = L.diff_idx;
+    T.n_diff = L.n_diff;
+    T.grad_da = L.grad_da;
+    T.grad_db_out = L.grad_db;
     T.boxes = L.boxes;
     T.partial = L.partial;
     T.n_img = n_img;
@@ -339,36 +334,23 @@ static void launch_interp_bwd_tri_t(const InterpLaunch &L, hipStream_t st) {
     } else {
         tile_records_layout(T, L.records, n_img, L.H, L.W, (long long)n_img * L.F);
     }
-    launch_tri_bwd_attr(T, NC, st);
-    int outs = L.attr_batched ? n_img : 1;
-    launch_gather_attr_t<NC>(L.partial, groups, L.F, L.V, outs, L.attr_batched, L.inc_off, L.inc, L.grad_attr, st);
-}
-
-int launch_gather_attr(const float *partial, int groups, int F, int V, int C, const int *inc_off, const int *inc,
-                       float *grad_attr, hipStream_t st) {
-    if (V == 0) return 0;
-    switch (C) {
-        case 4: launch_gather_attr_t<4>(partial, groups, F, V, 1, 0, inc_off, inc, grad_attr, st); break;
-        case 8: launch_gather_attr_t<8>(partial, groups, F, V, 1, 0, inc_off, inc, grad_attr, st); break;
-        default: return -1;
+    const int outs = L.attr_batched ? n_img : 1;
+    for (int c0 = 0; c0 < L.C;) {
+        const int nc = pass_channels(L.C - c0, L.C, L.n_diff > 0 ? 4 : kMaxPassChannels);
+        T.c0 = c0;
+        T.accum = c0 > 0;
+        if (int rc = launch_tri_bwd_attr(T, nc, st)) return rc;
+        if (int rc = launch_gather_attr(L.partial, groups, L.F, L.V, nc, L.C, c0, outs, L.attr_batched, L.inc_off,
+                                        L.inc, L.grad_attr, st))
+            return rc;
+        c0 += nc;
     }
-    return hipGetLastError() == hipSuccess ? 0 : -2;
+    return 0;
 }
 
 int launch_interpolate_bwd(const InterpLaunch &L, hipStream_t st) {
     if (L.total_pix == 0) return 0;
-    if (L.boxes && L.partial && L.records && L.inc_off && L.inc && L.n_diff == 0 && L.cv > 0) {
-        switch (L.cv) {
-            case 1: launch_interp_bwd_tri_t<1>(L, st); break;
-            case 2: launch_interp_bwd_tri_t<2>(L, st); break;
-            case 3: launch_interp_bwd_tri_t<3>(L, st); break;
-            case 4: launch_interp_bwd_tri_t<4>(L, st); break;
-            case 8: launch_interp_bwd_tri_t<8>(L, st); break;
-            case 16: launch_interp_bwd_tri_t<16>(L, st); break;
-            default: return -1;
-        }
-        return hipGetLastError() == hipSuccess ? 0 : -2;
-    }
+    if (L.boxes && L.partial && L.records && L.inc_off && L.inc) return launch_interp_bwd_tri(L, st);
     dim3 grid((unsigned)((L.total_pix + 255) / 256)), block(256);
     DRP_INTERP_DISPATCH(k_interp_bwd, L.attr, L.V, L.C, L.attr_batched, (const float4 *)L.rast, L.tri, L.F,
                         L.total_pix, L.pix_per_img, L.grad_out, L.grad_attr, (float4 *)L.grad_rast,

@@ -115,8 +115,8 @@ struct InterpLaunch {
     // triangle-centric backward (all set) or per-pixel atomics (any null)
     int H, W;
     const ItemBox *boxes;
-    float *partial;          // [groups, F, 3, C]
-    void *records;           // tile records (tile_records_bytes(n_img, H, W, 3 C, n_img * F))
+    float *partial;          // [groups, F, 3, min(C, kMaxPassChannels)]
+    void *records;           // tile records of min(C, kMaxPassChannels) channels
     const int *inc_off, *inc;
     int views_per_group;
     UnevenMap um;            // uneven batch (um.n > 0): packed items, global ids and vertices, one group
@@ -154,6 +154,9 @@ struct AALaunch {
     int total_blk, total_t32;    // uneven batch: pair blocks and backward tiles of all items
 };
 
+// channels of one pass of the tile backward (wider attributes take several)
+constexpr int kMaxPassChannels = 16;
+
 // tiles of a triangle's pixel box whose record index the tile pass stores
 constexpr int kBoxSlots = 4;
 
@@ -164,7 +167,13 @@ struct TriBwdLaunch {
     const float *rast, *grad_rast, *grad_db, *grad_out;
     const float *attr;       // attribute mode: attributes (for grad_rast)
     int V, attr_batched;
+    int ldc, c0;             // attribute mode: row stride of attr and grad_out, first channel of this pass
+    int accum;               // attribute mode: a later chunk of channels, added to grad_rast_out (and grad_db_out)
     float *grad_rast_out;    // attribute mode: grad_rast written by the tile pass (fused mode: null skips it)
+    const float *rast_db, *grad_da;  // attribute mode, n_diff > 0: gradients [.., 2 n_diff] of the derivatives
+    const int *diff_idx;             //   of channels diff_idx[n_diff]
+    int n_diff;
+    float *grad_db_out;      // nullable
     const ItemBox *boxes;
     float *partial;
     float *partial_pos;      // fused mode: the position partial [n_img, 3F] float4 (partial: attributes)
@@ -189,14 +198,20 @@ struct Fork {
 bool fork_begin(hipStream_t main, Fork &f);
 int fork_end(hipStream_t main, const Fork &f);
 
+// C: channels of the pass, 1 .. 16 (with n_diff > 0: 1 .. 4); a multiple of 4
+// only where ldc is one too (16-byte rows)
 int launch_tri_bwd_pos(const TriBwdLaunch &L, hipStream_t st);
 int launch_tri_bwd_attr(const TriBwdLaunch &L, int C, hipStream_t st);
 int launch_tri_bwd_fused(const TriBwdLaunch &L, int C, hipStream_t st);
 int launch_corner_slots(const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st);
 int launch_gather_pos(const float *partial, int n_img, int F, int V, int pos_batched, const int *inc_off,
                       float *grad_pos, hipStream_t st);
-int launch_gather_attr(const float *partial, int groups, int F, int V, int C, const int *inc_off, const int *inc,
-                       float *grad_attr, hipStream_t st);
+// partial [groups, F, 3, C] added to channels [c0, c0 + C) of grad_attr rows of ldc floats; outs outputs, one
+// group each when per_output
+int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
+                       int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st);
+// floats of a tile record with the attribute and position sums
+int tile_record_floats(int C, bool attr, bool pos);
 // workspace of the tile records for nv floats per record and n_boxes pixel
 // boxes (n_img * F for a uniform batch, the triangles of an uneven one), and
 // its layout

@@ -461,9 +461,6 @@ def _attr_layout(attr, rast):
     raise ValueError(f'attr must have shape [V, C] or [n, V, C] (got {tuple(attr.shape)})')
 
 
-_TRI_BWD_C = (1, 2, 3, 4, 8, 16)
-
-
 def _views_per_group(n, F):
     """Views folded into one partial of the triangle-centric attribute backward
     (a power of two up to 8: fewer partials to gather, blocks still fill the GPU)."""
@@ -473,7 +470,7 @@ def _views_per_group(n, F):
     return p
 
 
-_FUSED_C = (4, 8)
+_FUSED_C = tuple(range(1, 17))  # channel counts of the fused attribute + position backward
 
 
 class _InterpolateFunc(torch.autograd.Function):
@@ -534,13 +531,11 @@ class _InterpolateFunc(torch.autograd.Function):
             dda = torch.zeros((n, H, W, 2 * nd), dtype=torch.float32, device=attr.device)
         off = inc = ws = None
         ws_bytes = vpg = 0
-        if boxes is not None and nd == 0 and C in _TRI_BWD_C:
+        if boxes is not None:
             off, inc = incidence(tri, V)
             vpg = _views_per_group(n, F)
             ws_bytes = L.drp_interpolate_bwd_workspace_size(n, H, W, F, C, batched, vpg)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=attr.device)
-        else:
-            boxes = None
         rc = L.drp_interpolate_bwd(stream_of(attr), ptr(attr), n, V, batched, C, ptr(rast), H, W, ptr(tri), F,
                                    ptr(rast_db), ptr(diff_idx), nd, ptr(dy), ptr(dda), ptr(gattr), ptr(grast),
                                    ptr(gdb), ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws_bytes)

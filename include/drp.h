@@ -150,7 +150,7 @@ int drp_batch_rasterize_bwd(void *stream, const void *plan, const void *plan_dev
  * its pixels: drp_batch_interpolate_bwd and drp_batch_rasterize_bwd (global
  * ids, no grad_db) of the grad_rast the first would write, without writing
  * it (the batched form of drp_interpolate_rasterize_bwd); grad_attr and
- * grad_pos accumulated (caller zero-fills).  C in {4, 8}; pos [n_vert, 4] as
+ * grad_pos accumulated (caller zero-fills).  C in 1 .. 16; pos [n_vert, 4] as
  * rasterized, tri the batch triangles (global vertex indices). */
 size_t drp_batch_interpolate_rasterize_bwd_workspace_size(const void *plan, int C);
 int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr,
@@ -244,10 +244,11 @@ int drp_interpolate_fwd(void *stream, const float *attr, int n_img, int V, int a
 
 /* Backward: grad_attr accumulated (caller zero-fills), grad_rast (and grad_db
  * when not null) written; channels 2, 3 of grad_rast are zero.  With boxes
- * (from the rasterize call that produced rast), the incidence table, no
- * diff_attrs, C in {1,2,3,4,8,16} and a workspace of
- * drp_interpolate_bwd_workspace_size bytes, grad_attr is gathered per triangle
- * (views_per_group views per partial) and per vertex without atomics. */
+ * (from the rasterize call that produced rast), the incidence table and a
+ * workspace of drp_interpolate_bwd_workspace_size bytes, grad_attr is gathered
+ * per triangle (views_per_group views per partial) and per vertex without
+ * atomics, in passes of up to 16 channels (with diff_attrs: 4); grad_out and
+ * attr are 16-byte aligned then where C % 4 == 0. */
 size_t drp_interpolate_bwd_workspace_size(int n_img, int H, int W, int F, int C, int attr_batched,
                                           int views_per_group);
 int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int attr_batched, int C,
@@ -269,7 +270,7 @@ int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int a
  * drp_rasterize_bwd on the grad_rast it wrote.  The rasterize backward is
  * linear in grad_rast, so gradients that rast receives from other consumers
  * can go through drp_rasterize_bwd on their own.  attr [V,C] (not batched),
- * C in {4, 8}; pos [V,4] or [n,V,4] (pos_batched); tri and boxes those of the
+ * C in 1 .. 16; pos [V,4] or [n,V,4] (pos_batched); tri and boxes those of the
  * rasterize call. */
 size_t drp_interpolate_rasterize_bwd_workspace_size(int n_img, int H, int W, int F, int C, int views_per_group);
 int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
