@@ -47,9 +47,9 @@ def bin_load(pos, tri, resolution, tile, probe_cap=4096) -> Tuple[int, int]:
     boxes = torch.empty((n, F, 3), dtype=torch.int32, device=pos.device)
     _run(pos, tri, H, W, tile, probe_cap, ws, boxes, rast)
     n_tiles = n * ((W + tile[0] - 1) // tile[0]) * ((H + tile[1] - 1) // tile[1])
-    # workspace layout: int32 bin counts [n_tiles], then spill-list counts [n]
+    # workspace layout: int32 bin counts [n_tiles], then spill-list counts [n] (top bit: a mark)
     counts = ws[:4 * (n_tiles + n)].view(torch.int32)
-    return int(counts[:n_tiles].max().item()), int(counts[n_tiles:].sum().item())
+    return int(counts[:n_tiles].max().item()), int((counts[n_tiles:] & 0x7fffffff).sum().item())
 
 
 def tune_rasterize(ctx: 'nvdr.RasterizeCudaContext', pos: torch.Tensor, tri: torch.Tensor, resolution,
