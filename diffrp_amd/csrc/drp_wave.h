@@ -23,14 +23,37 @@ __device__ __forceinline__ unsigned dpp_mov(unsigned x) {
     return (unsigned)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
 }
 
-// x of lane ^ XOR, XOR in {1, 2, 4, 8}
+// x of lane ^ XOR, XOR a power of two
 template <int XOR>
 __device__ __forceinline__ unsigned lane_xor(unsigned x) {
-    static_assert(XOR == 1 || XOR == 2 || XOR == 4 || XOR == 8, "within a row of 16");
+    static_assert(XOR == 1 || XOR == 2 || XOR == 4 || XOR == 8 || XOR == 16 || XOR == 32, "a power of two");
     if constexpr (XOR == 1) return dpp_mov<kDppXor1>(x);
     else if constexpr (XOR == 2) return dpp_mov<kDppXor2>(x);
     else if constexpr (XOR == 4) return dpp_mov<kDppXor3>(dpp_mov<kDppXor7>(x));
-    else return dpp_mov<kDppXor8>(x);
+    else if constexpr (XOR == 8) return dpp_mov<kDppXor8>(x);
+    else if constexpr (XOR == 16) {  // the odd rows' partners arrive in the first word, the even rows' in the second
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        return __builtin_amdgcn_inverse_ballot_w64(0xffff0000ffff0000ull) ? r[0] : r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        return __builtin_amdgcn_inverse_ballot_w64(0xffffffff00000000ull) ? r[0] : r[1];
+    }
+}
+template <int XOR>
+__device__ __forceinline__ float lane_xor(float x) {
+    return __uint_as_float(lane_xor<XOR>(__float_as_uint(x)));
+}
+
+// largest x over aligned groups of N lanes, in every lane of the group
+template <int N>
+__device__ __forceinline__ float group_max(float x) {
+    if constexpr (N >= 2) x = fmaxf(x, lane_xor<1>(x));
+    if constexpr (N >= 4) x = fmaxf(x, lane_xor<2>(x));
+    if constexpr (N >= 8) x = fmaxf(x, lane_xor<4>(x));
+    if constexpr (N >= 16) x = fmaxf(x, lane_xor<8>(x));
+    if constexpr (N >= 32) x = fmaxf(x, lane_xor<16>(x));
+    if constexpr (N >= 64) x = fmaxf(x, lane_xor<32>(x));
+    return x;
 }
 
 // lanes that keep the minimum in the bitonic step (size, stride)
