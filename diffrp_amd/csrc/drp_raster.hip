@@ -1,7 +1,7 @@
 // Rasterizer kernels for gfx950.
 //
 // Forward: (1) k_setup_bin, one thread per (image, triangle): setup (stored as
-// a 32-byte setup record: snapped vertices, class, top-left flags), per-(image,
+// a 32-byte setup record: snapped vertices, class, top-left flags, depth bounds), per-(image,
 // triangle) pixel box, and wave-aggregated insertion into fixed-capacity
 // screen-tile bins (full bins and large triangles spill to a per-image list);
 // (2) k_fine, one workgroup per tile: triangle records staged
@@ -41,19 +41,97 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
     return (1ull << (threadIdx.x & 63)) - 1ull;
 }
 
+// Bounds of a direct-class triangle's depth: no pixel centre of the box
+// [px0, px1] x [py0, py1] can receive from it a computed z/w below zlo or above
+// zhi (-INFINITY and INFINITY for slivers, which have no useful bound).
+//
+// With X_k = x_k - w_k px, Y_k = y_k - w_k py and e_k = X_i Y_j - X_j Y_i
+// ((i, j) = (k+1, k+2) mod 3), wn* = sum e_k w_k is the determinant of the
+// rows (x_k, y_k, w_k), the same at every pixel, and zn* = sum e_k z_k is
+// affine in (px, py), so the exact depth zn* / wn* is affine over the box:
+// its extremes are at corners.  eval_pixel's float zn and wn (X, Y one
+// rounding each; e_k two products and an fma: 4.02 u T_k; the nested fmas:
+// 3.01 u sum |e_k z_k|) are within Ez = 7.04 u sum T_k |z_k| and
+// Ew = 7.04 u sum T_k w_k of the exact ones at any pixel centre of the box,
+// with u = 2^-24 and T_k = |X_i Y_j| + |X_j Y_i| bounded through the box's
+// end columns and rows (X_k is affine in px, Y_k in py); 8 u in place of
+// 7.04 u covers the roundings of the bound itself.  The corners are evaluated
+// with eval_pixel too, and their depths taken as zn * rcp(wn) (within 4 u of
+// zn / wn).  With W0 = |wn(corner 0)| - Ew <= |wn*| > 3 Ew (slivers have no
+// bound), every |wn| >= W0 - Ew > 0; the exact depth over the box is at most
+// ZB = 2 (QA (1 + 5 u) + Ez / (W0 - Ew)) in magnitude (QA: the corners'
+// largest |depth|), a pixel's computed depth is within E + u (ZB + E) of the
+// exact one, E = (Ez + ZB Ew) / (W0 - Ew), and the exact extremes are within
+// E + 4 u QA (1 + 5 u) of the corners' smallest and largest depths: the margin
+// below (2 E + 8 u QA + 2 u (ZB + E)) exceeds the sum.
+__device__ __forceinline__ void depth_bounds(const TriVerts &v, float px0, float px1, float py0, float py1,
+                                             float &zlo, float &zhi) {
+    constexpr float u = 0x1p-24f;
+    float ez = 0.f, ew = 0.f;
+    {
+        float MX[3], MY[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            MX[k] = fmaxf(fabsf(fmaf(-v.w[k], px0, v.x[k])), fabsf(fmaf(-v.w[k], px1, v.x[k])));
+            MY[k] = fmaxf(fabsf(fmaf(-v.w[k], py0, v.y[k])), fabsf(fmaf(-v.w[k], py1, v.y[k])));
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int i = k == 2 ? 0 : k + 1, j = k == 0 ? 2 : k - 1;
+            const float T = fmaf(MX[i], MY[j], MX[j] * MY[i]);
+            ez = fmaf(T, fabsf(v.z[k]), ez);
+            ew = fmaf(T, v.w[k], ew);
+        }
+        ez *= 8.f * u;
+        ew *= 8.f * u;
+    }
+    float qmin = INFINITY, qmax = -INFINITY, w0 = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        PixEval p;
+        eval_pixel(v, (c & 1) ? px1 : px0, (c & 2) ? py1 : py0, p);
+        if (c == 0) w0 = fabsf(p.wn) - ew;
+        const float q = p.zn * __builtin_amdgcn_rcpf(p.wn);
+        qmin = fminf(qmin, q);
+        qmax = fmaxf(qmax, q);
+    }
+    zlo = -INFINITY;
+    zhi = INFINITY;
+    const float qa = fmaxf(fabsf(qmin), fabsf(qmax));
+    if (!(w0 > 3.f * ew) || !(qa < INFINITY)) return;
+    const float zb = 2.f * (qa * (1.f + 5.f * u) + ez / (w0 - ew));
+    const float E = (ez + zb * ew) / (w0 - ew);
+    const float m = 2.f * E + 8.f * u * qa + 2.f * u * (zb + E);
+    if (!(m < INFINITY)) return;
+    zlo = qmin - m;
+    zhi = qmax + m;
+}
+
+// the upper bound in a setup record: the float's upper 27 bits, rounded up
+__device__ __forceinline__ int pack_zhi(float zhi) {
+    uint32_t b = __float_as_uint(zhi);
+    if (!(b & 0x80000000u)) b += 31u;  // (a negative float's magnitude shrinks by dropping bits)
+    return (int)(b & ~31u);
+}
+__device__ __forceinline__ float unpack_zhi(int meta) { return __uint_as_float((uint32_t)meta & ~31u); }
+
 // ----------------------------------------------------------------------------
 // setup records: two int4 per (image, triangle), at the image's list offset
-//   direct: {X0, X1, X2, meta}, {Y0, Y1, Y2, 0}  (snapped, counter-clockwise)
-//   homogeneous: {c0 | c1 << 16, r0 | r1 << 16, 0, meta}, {0, 0, 0, 0}
-//   meta = class | top-left flags << 2 (class kCull: nothing to draw)
+//   direct: {X0, X1, X2, meta}, {Y0, Y1, Y2, zlo}  (snapped, counter-clockwise)
+//   homogeneous: {c0 | c1 << 16, r0 | r1 << 16, 0, meta}, {0, 0, 0, zlo}
+//   meta = class | top-left flags << 2 | zhi (27 bits, pack_zhi)  (class kCull: nothing to draw)
+// zlo, zhi: depth bounds over the triangle's pixel box (-INFINITY, INFINITY:
+// none), for the launches that ask for them
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ void store_setup(int4 *__restrict__ setup, long long i, const TriSetup &s) {
-    int4 a = make_int4(0, 0, 0, s.cls), b = make_int4(0, 0, 0, 0);
+__device__ __forceinline__ void store_setup(int4 *__restrict__ setup, long long i, const TriSetup &s, float zlo,
+                                            float zhi) {
+    const int hi = pack_zhi(zhi), lo = __float_as_int(zlo);
+    int4 a = make_int4(0, 0, 0, s.cls | hi), b = make_int4(0, 0, 0, lo);
     if (s.cls == kDirect) {
-        a = make_int4(s.X[0], s.X[1], s.X[2], s.cls | (s.tl[0] << 2) | (s.tl[1] << 3) | (s.tl[2] << 4));
-        b = make_int4(s.Y[0], s.Y[1], s.Y[2], 0);
+        a = make_int4(s.X[0], s.X[1], s.X[2], s.cls | (s.tl[0] << 2) | (s.tl[1] << 3) | (s.tl[2] << 4) | hi);
+        b = make_int4(s.Y[0], s.Y[1], s.Y[2], lo);
     } else if (s.cls == kHomog) {
-        a = make_int4(s.c0 | (s.c1 << 16), s.r0 | (s.r1 << 16), 0, s.cls);
+        a = make_int4(s.c0 | (s.c1 << 16), s.r0 | (s.r1 << 16), 0, s.cls | hi);
     }
     setup[2 * i] = a;
     setup[2 * i + 1] = b;
@@ -62,6 +140,7 @@ __device__ __forceinline__ void store_setup(int4 *__restrict__ setup, long long 
 // ----------------------------------------------------------------------------
 // setup + binning
 // ----------------------------------------------------------------------------
+template <bool BOUNDS>
 __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restrict__ pos,
                                                    const int *__restrict__ tri, int tile_w, int tile_h,
                                                    int *__restrict__ bin_count,
@@ -77,7 +156,10 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
     if (valid) {
         TriVerts v;
         if (load_tri(pos, tri, t, d, v)) setup_tri(v, d.H, d.W, s);
-        store_setup(setup, (long long)d.list_off + (t - d.f0), s);
+        float zlo = -INFINITY, zhi = INFINITY;
+        if (BOUNDS && s.cls == kDirect)
+            depth_bounds(v, pix_ndc(s.c0, d.W), pix_ndc(s.c1, d.W), pix_ndc(s.r0, d.H), pix_ndc(s.r1, d.H), zlo, zhi);
+        store_setup(setup, (long long)d.list_off + (t - d.f0), s, zlo, zhi);
         if (boxes) {
             int2 pb = s.cls == kCull ? empty_box() : pack_box(s.c0, s.c1, s.r0, s.r1);
             boxes[(long long)d.list_off + (t - d.f0)] = ItemBox{pb.x, pb.y, 0};  // hit: set by k_fine
@@ -263,71 +345,20 @@ __device__ __forceinline__ float inv_ord_f32(uint32_t k) {
     return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
 }
 
-// Depth cull of a direct-class triangle against tile rows whose every pixel
-// already holds a fragment: true when no pixel centre of the box
-// [px0, px1] x [py0, py1] can receive from this triangle a depth z/w at or
-// below zcut, the farthest current nearest depth over the box's rows, so that
-// the triangle cannot change any depth key (the test is a strict >, whatever
-// the triangle index).
-//
-// With X_k = x_k - w_k px, Y_k = y_k - w_k py and e_k = X_i Y_j - X_j Y_i
-// ((i, j) = (k+1, k+2) mod 3), wn* = sum e_k w_k is the determinant of the
-// rows (x_k, y_k, w_k), the same at every pixel, and zn* = sum e_k z_k is
-// affine in (px, py), so the exact depth zn* / wn* is affine over the box:
-// its minimum is at a corner.  eval_pixel's float zn and wn (X, Y one
-// rounding each; e_k two products and an fma: 4.02 u T_k; the nested fmas:
-// 3.01 u sum |e_k z_k|) are within Ez = 7.04 u sum T_k |z_k| and
-// Ew = 7.04 u sum T_k w_k of the exact ones at any pixel centre of the box,
-// with u = 2^-24 and T_k = |X_i Y_j| + |X_j Y_i| bounded through the box's
-// end columns and rows (X_k is affine in px, Y_k in py); 8 u in place of
-// 7.04 u covers the roundings of the bound itself.  The corners are evaluated
-// with eval_pixel too, and their depths taken as zn * rcp(wn) (within 4 u of
-// zn / wn).  With W0 = |wn(corner 0)| - Ew <= |wn*| > 3 Ew (slivers are never
-// culled), every |wn| >= W0 - Ew > 0; the exact depth over the box is at most
-// ZB = 2 (QA (1 + 5 u) + Ez / (W0 - Ew)) in magnitude (QA: the corners'
-// largest |depth|), a pixel's computed depth is within E + u (ZB + E) of the
-// exact one, E = (Ez + ZB Ew) / (W0 - Ew), and the exact minimum is within
-// E + 4 u QA (1 + 5 u) of the corners' smallest depth: the margin below
-// (2 E + 8 u QA + 2 u (ZB + E)) exceeds the sum.
-__device__ __forceinline__ bool depth_culled(const TriVerts &v, float px0, float px1, float py0, float py1,
-                                             float zcut) {
-    constexpr float u = 0x1p-24f;
-    float ez = 0.f, ew = 0.f;
-    {
-        float MX[3], MY[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            MX[k] = fmaxf(fabsf(fmaf(-v.w[k], px0, v.x[k])), fabsf(fmaf(-v.w[k], px1, v.x[k])));
-            MY[k] = fmaxf(fabsf(fmaf(-v.w[k], py0, v.y[k])), fabsf(fmaf(-v.w[k], py1, v.y[k])));
-        }
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int i = k == 2 ? 0 : k + 1, j = k == 0 ? 2 : k - 1;
-            const float T = fmaf(MX[i], MY[j], MX[j] * MY[i]);
-            ez = fmaf(T, fabsf(v.z[k]), ez);
-            ew = fmaf(T, v.w[k], ew);
-        }
-        ez *= 8.f * u;
-        ew *= 8.f * u;
-    }
-    float qmin = INFINITY, qa = 0.f, w0 = 0.f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        PixEval p;
-        eval_pixel(v, (c & 1) ? px1 : px0, (c & 2) ? py1 : py0, p);
-        if (c == 0) w0 = fabsf(p.wn) - ew;
-        const float q = p.zn * __builtin_amdgcn_rcpf(p.wn);
-        qmin = fminf(qmin, q);
-        qa = fmaxf(qa, fabsf(q));
-    }
-    if (!(w0 > 3.f * ew) || !(qa < INFINITY)) return false;
-    const float zb = 2.f * (qa * (1.f + 5.f * u) + ez / (w0 - ew));
-    const float E = (ez + zb * ew) / (w0 - ew);
-    return qmin - (2.f * E + 8.f * u * qa + 2.f * u * (zb + E)) > zcut;
-}
+// Depth-ordered entries: a tile's entries are taken in batches of up to
+// kOrderRounds rounds, each batch in the order of its triangles' lower depth
+// bounds (kOrderBuckets equal steps between the batch's extremes).  Only the
+// launches whose tiles hold many rounds (depth_cull): 5.2M triangles at 2048^2,
+// four peeled layers forward and recomputed, take 6.59 -> 4.96 ms in the peeled
+// layers' fine raster and 1.99 -> 1.50 ms in the first ones'; tiles of two to
+// nine rounds of small triangles gain little (turntable 443 -> 424 us, 18 us of
+// it spent again on the bounds).  Two halves around the mean bound in one-round
+// tiles cost small launches more in barriers than they save.
+constexpr int kOrderRounds = 8;
+constexpr int kOrderBuckets = 64;
 
 // LDS of one fine-raster block
-template <int TW, int TH, bool PEEL>
+template <int TW, int TH, bool PEEL, bool ORDER>
 struct FineLds {
     static constexpr int NT = TW * TH;
     static constexpr int kQueue = NT * kQueuePerLane;
@@ -338,7 +369,11 @@ struct FineLds {
     unsigned long long pkey[PEEL ? NT : 1];
     float pxs[TW], pys[TH];             // NDC centres of the tile's columns and rows (one division each per tile)
     int wsum[3 * (NT / 64)];            // scan partials: records; row spans (two, alternating)
-    float zrow[TH];                     // per tile row: the farthest current nearest depth (depth cull)
+    float zrow[ORDER ? TH : 1];         // per tile row: the farthest current nearest depth
+    float prow[ORDER && PEEL ? TH : 1]; // per tile row: the nearest depth of the previous layer
+    unsigned short order[ORDER ? kOrderRounds * NT : 1];  // a batch's entries in depth order
+    int hist[ORDER ? kOrderBuckets : 1];
+    float zred[ORDER ? 2 * (NT / 64) : 1];
     int bcast;                          // block-wide broadcast slot
 };
 
@@ -377,8 +412,8 @@ __device__ __forceinline__ ImageDesc uniform_desc(const ImageDesc &s) {
     return d;
 }
 
-template <int TW, int TH, bool PEEL>
-__device__ __forceinline__ FineTile fine_begin(FineLds<TW, TH, PEEL> &S, const Batch &b, int tile,
+template <int TW, int TH, bool PEEL, bool ORDER>
+__device__ __forceinline__ FineTile fine_begin(FineLds<TW, TH, PEEL, ORDER> &S, const Batch &b, int tile,
                                                const int *__restrict__ bin_count,
                                                const int *__restrict__ list_count, const float4 *__restrict__ prev) {
     FineTile T;
@@ -396,12 +431,20 @@ __device__ __forceinline__ FineTile fine_begin(FineLds<TW, TH, PEEL> &S, const B
     if (tid < TH) S.pys[tid] = pix_ndc(T.tr0 + tid, d.H);
     if (PEEL) {
         unsigned long long pk = ~0ull;  // empty previous layer: nothing can follow
+        float pz = INFINITY;
         const int c = T.tc0 + (tid % TW), r = T.tr0 + (tid / TW);
         if (c < d.W && r < d.H) {
             float4 pv = prev[d.pix_off + (long long)r * d.W + c];
-            if (pv.w > 0.f) pk = frag_key(pv.z, float_to_triidx(pv.w) - 1 + (b.local_ids ? d.f0 : 0));
+            if (pv.w > 0.f) {
+                pk = frag_key(pv.z, float_to_triidx(pv.w) - 1 + (b.local_ids ? d.f0 : 0));
+                pz = pv.z;
+            }
         }
         S.pkey[tid] = pk;
+        if (ORDER) {
+            pz = -group_max<TW>(-pz);
+            if (tid % TW == 0) S.prow[tid / TW] = pz;
+        }
     }
     T.tw_img = min(TW, d.W - T.tc0);  // tile clipped to the image
     T.th_img = min(TH, d.H - T.tr0);
@@ -415,161 +458,289 @@ __device__ __forceinline__ FineTile fine_begin(FineLds<TW, TH, PEEL> &S, const B
     return T;
 }
 
-// depth test of the tile's entries [e0, e1) into S.zbuf; with CULL, after the
-// first round (from the first when S.zbuf was seeded with real keys),
-// direct-class triangles are culled against the tile's depths
+// triangle of entry idx of the tile's list; -1 for none that concerns it
+__device__ __forceinline__ int fine_entry(const FineTile &T, int idx, const int *__restrict__ bins,
+                                          const int *__restrict__ lists) {
+    const ImageDesc &d = T.d;
+    int t;
+    if (idx < T.nbin) t = bins[d.bin_off + (long long)(T.tile - d.tile_off) * d.bin_cap + idx];
+    else if (T.full_scan) t = d.f0 + (idx - T.nbin);
+    else {
+        t = lists[(long long)d.list_off + idx - T.nbin];
+        if (t < 0) t = T.over ? ~t : -1;  // a bin spill: in this tile's bin unless that is full
+    }
+    return t >= d.f0 && t < d.f1 ? t : -1;  // every entry names a triangle of this image
+}
+
+// a setup record's pixel box, clipped to the tile (tile-local); false when empty
+__device__ __forceinline__ bool fine_box(const FineTile &T, int cls, const int4 &sa, const int4 &sb, int &x0, int &x1,
+                                         int &y0, int &y1) {
+    int c0, c1, r0, r1;
+    if (cls == kDirect) {
+        const int X[3] = {sa.x, sa.y, sa.z}, Y[3] = {sb.x, sb.y, sb.z};
+        direct_box(X, Y, T.d.H, T.d.W, c0, c1, r0, r1);  // not empty: the setup pass kept it
+    } else {
+        c0 = sa.x & 0xffff; c1 = (unsigned)sa.x >> 16;
+        r0 = sa.y & 0xffff; r1 = (unsigned)sa.y >> 16;
+    }
+    x0 = max(c0 - T.tc0, 0); x1 = min(c1 - T.tc0, T.tw_img - 1);
+    y0 = max(r0 - T.tr0, 0); y1 = min(r1 - T.tr0, T.th_img - 1);
+    return x0 <= x1 && y0 <= y1;
+}
+
+// Per tile row, the farthest of its current nearest depths (INFINITY while a
+// pixel that can still receive a fragment has none): nothing at or behind it
+// can change the row.  One barrier.
+template <int TW, int TH, bool PEEL, bool ORDER>
+__device__ __forceinline__ void fine_zrow(FineLds<TW, TH, PEEL, ORDER> &S, const FineTile &T) {
+    const int tid = threadIdx.x;
+    float zt = -INFINITY;
+    if ((tid % TW) < T.tw_img && (tid / TW) < T.th_img && !(PEEL && S.pkey[tid] == ~0ull)) {
+        const unsigned long long key = S.zbuf[tid];
+        zt = key == ~0ull ? INFINITY : inv_ord_f32((uint32_t)(key >> 32));
+    }
+    zt = group_max<TW>(zt);
+    if (tid % TW == 0) S.zrow[tid / TW] = zt;
+    __syncthreads();
+}
+
+// one round: the depth test of the lanes' entries (triangle t, -1 for none)
+// into S.zbuf.  CULL: entries whose depth bounds show that they cannot change
+// a key of their rows are dropped before their vertices are read -- against
+// S.zrow where `behind`, and against the previous layer's rows when peeling.
 template <int TW, int TH, bool PEEL, bool CULL>
-__device__ __forceinline__ void fine_entries(FineLds<TW, TH, PEEL> &S, const FineTile &T, int e0, int e1,
-                                             const float *__restrict__ pos, const int *__restrict__ tri,
-                                             const int *__restrict__ bins, const int *__restrict__ lists,
-                                             const int4 *__restrict__ setup, bool seeded) {
+__device__ __forceinline__ void fine_round(FineLds<TW, TH, PEEL, CULL> &S, const FineTile &T, int t, bool behind,
+                                           int &par, const float *__restrict__ pos, const int *__restrict__ tri,
+                                           const int4 *__restrict__ setup) {
     constexpr int NT = TW * TH;
     constexpr int kQueue = NT * kQueuePerLane;
     const ImageDesc &d = T.d;
     const int tid = threadIdx.x;
-    const int tc0 = T.tc0, tr0 = T.tr0;
-    int par = 0;  // scan partials of the row spans in use; alternates every sub-round
-    for (int base = e0; base < e1; base += NT) {
-        // After the first round: per tile row, the farthest of its current
-        // nearest depths (infinite while a pixel of the row has no fragment
-        // yet), against which direct-class triangles are culled over the rows
-        // of their box (depth_culled).
-        const bool cull_round = CULL && (base > e0 || seeded);
-        if (cull_round) {
-            float zt = -INFINITY;
-            if ((tid % TW) < T.tw_img && (tid / TW) < T.th_img) {
-                const unsigned long long key = S.zbuf[tid];
-                zt = key == ~0ull ? INFINITY : inv_ord_f32((uint32_t)(key >> 32));
+    int count = 0;
+    if (t >= 0) {
+        // both setup words and the corner indices depend on t alone: one round of loads,
+        // then the corners' positions
+        const long long si = 2 * ((long long)d.list_off + (t - d.f0));
+        const int4 sa = setup[si], sb = setup[si + 1];
+        const int cls = sa.w & 3;
+        int x0, x1, y0, y1;
+        bool live = cls != kCull && fine_box(T, cls, sa, sb, x0, x1, y0, y1);
+        if (CULL && live && (behind || PEEL)) {
+            float zcut = behind ? -INFINITY : INFINITY, pcut = INFINITY;
+            for (int y = y0; y <= y1; ++y) {
+                if (behind) zcut = fmaxf(zcut, S.zrow[y]);
+                if (PEEL) pcut = fminf(pcut, S.prow[y]);
             }
-#pragma unroll
-            for (int o = TW / 2; o >= 1; o >>= 1) zt = fmaxf(zt, __shfl_xor(zt, o, 64));  // a row: TW lanes
-            if (tid % TW == 0) S.zrow[tid / TW] = zt;
-            __syncthreads();
+            if (__int_as_float(sb.w) > zcut || (PEEL && unpack_zhi(sa.w) < pcut)) live = false;
         }
-        int idx = base + tid;
-        int count = 0;
-        if (idx < e1) {
-            int t;
-            if (idx < T.nbin) t = bins[d.bin_off + (long long)(T.tile - d.tile_off) * d.bin_cap + idx];
-            else if (T.full_scan) t = d.f0 + (idx - T.nbin);
-            else {
-                t = lists[(long long)d.list_off + idx - T.nbin];
-                if (t < 0) t = T.over ? ~t : -1;  // a bin spill: in this tile's bin unless that is full
+        if (!CULL || live) {
+            const int *t3 = tri + 3 * (long long)t;
+            const int i0 = t3[0], i1 = t3[1], i2 = t3[2];
+            const bool in_range = (unsigned)i0 < (unsigned)d.V && (unsigned)i1 < (unsigned)d.V &&
+                                  (unsigned)i2 < (unsigned)d.V;
+            TriVerts v;
+            if (in_range) {
+                const float4 *P = reinterpret_cast<const float4 *>(pos + d.pos_off);
+                const float4 a = P[i0], b = P[i1], c = P[i2];
+                v.x[0] = a.x; v.y[0] = a.y; v.z[0] = a.z; v.w[0] = a.w;
+                v.x[1] = b.x; v.y[1] = b.y; v.z[1] = b.z; v.w[1] = b.w;
+                v.x[2] = c.x; v.y[2] = c.y; v.z[2] = c.z; v.w[2] = c.w;
             }
-            if (t >= d.f0 && t < d.f1) {  // every entry names a triangle of this image
-                // both setup words and the corner indices depend on t alone: one round of loads,
-                // then the corners' positions
-                const long long si = 2 * ((long long)d.list_off + (t - d.f0));
-                const int4 sa = setup[si], sb = setup[si + 1];
-                const int *t3 = tri + 3 * (long long)t;
-                const int i0 = t3[0], i1 = t3[1], i2 = t3[2];
-                const bool in_range = (unsigned)i0 < (unsigned)d.V && (unsigned)i1 < (unsigned)d.V &&
-                                      (unsigned)i2 < (unsigned)d.V;
-                TriVerts v;
-                if (in_range) {
-                    const float4 *P = reinterpret_cast<const float4 *>(pos + d.pos_off);
-                    const float4 a = P[i0], b = P[i1], c = P[i2];
-                    v.x[0] = a.x; v.y[0] = a.y; v.z[0] = a.z; v.w[0] = a.w;
-                    v.x[1] = b.x; v.y[1] = b.y; v.z[1] = b.z; v.w[1] = b.w;
-                    v.x[2] = c.x; v.y[2] = c.y; v.z[2] = c.z; v.w[2] = c.w;
+            if (live && in_range) {
+                FineRec &R = S.rec[tid];
+                R.t = t;
+                R.v = v;
+                count = y1 - y0 + 1;  // row items
+                int box = x0 | (y0 << 6) | (x1 << 12) | (cls << 18);
+                if (cls == kDirect) {
+                    const int Px = kSubpix * T.tc0 + kHalfSub, Py = kSubpix * T.tr0 + kHalfSub;
+                    R.X[0] = sa.x - Px; R.X[1] = sa.y - Px; R.X[2] = sa.z - Px;
+                    R.Y[0] = sb.x - Py; R.Y[1] = sb.y - Py; R.Y[2] = sb.z - Py;
+                    box |= ((sa.w >> 2) & 7) << 20;  // top-left flags
+                    const int m = max(max(max(abs(R.X[0]), abs(R.X[1])), abs(R.X[2])),
+                                      max(max(abs(R.Y[0]), abs(R.Y[1])), abs(R.Y[2])));
+                    if (m < kSmallRec) box |= 1 << 23;  // 32-bit row spans
                 }
-                const int cls = sa.w & 3;
-                if (cls != kCull) {
-                    int c0, c1, r0, r1;
-                    if (cls == kDirect) {
-                        const int X[3] = {sa.x, sa.y, sa.z}, Y[3] = {sb.x, sb.y, sb.z};
-                        direct_box(X, Y, d.H, d.W, c0, c1, r0, r1);  // not empty: the setup pass kept it
-                    } else {
-                        c0 = sa.x & 0xffff; c1 = (unsigned)sa.x >> 16;
-                        r0 = sa.y & 0xffff; r1 = (unsigned)sa.y >> 16;
-                    }
-                    const int x0 = max(c0 - tc0, 0), x1 = min(c1 - tc0, T.tw_img - 1);
-                    const int y0 = max(r0 - tr0, 0), y1 = min(r1 - tr0, T.th_img - 1);
-                    if (x0 <= x1 && y0 <= y1 && in_range) {
-                        FineRec &R = S.rec[tid];
-                        R.t = t;
-                        R.v = v;
-                        count = y1 - y0 + 1;  // row items
-                        int box = x0 | (y0 << 6) | (x1 << 12) | (cls << 18);
-                        if (cls == kDirect) {
-                            const int Px = kSubpix * tc0 + kHalfSub, Py = kSubpix * tr0 + kHalfSub;
-                            R.X[0] = sa.x - Px; R.X[1] = sa.y - Px; R.X[2] = sa.z - Px;
-                            R.Y[0] = sb.x - Py; R.Y[1] = sb.y - Py; R.Y[2] = sb.z - Py;
-                            box |= ((sa.w >> 2) & 7) << 20;  // top-left flags
-                            const int m = max(max(max(abs(R.X[0]), abs(R.X[1])), abs(R.X[2])),
-                                              max(max(abs(R.Y[0]), abs(R.Y[1])), abs(R.Y[2])));
-                            if (m < kSmallRec) box |= 1 << 23;  // 32-bit row spans
-                        }
-                        R.box = box;
-                    }
-                }
+                R.box = box;
             }
         }
-        if (cull_round && count > 0) {  // the lane's own record, read back from LDS
-            const FineRec &R = S.rec[tid];
-            const int box = R.box, x0 = rec_x0(box), y0 = rec_y0(box);
-            float zcut = -INFINITY;
-            for (int y = y0; y < y0 + count; ++y) zcut = fmaxf(zcut, S.zrow[y]);
-            if (rec_cls(box) == kDirect && zcut < INFINITY &&
-                depth_culled(R.v, S.pxs[x0], S.pxs[rec_x1(box)], S.pys[y0], S.pys[y0 + count - 1], zcut))
-                count = 0;
-        }
-        int nrows;
-        const int ex = block_scan<NT>(count, S.wsum, nrows);  // this lane's record owns rows [ex, ex + count)
-        // Row items (record, tile row) in sub-rounds of NT: each lane finds the
-        // exact covered span of its row; the covered pixels are queued (block
-        // prefix sum, at most kQueue per pass) and evaluated by all lanes, so
-        // the barycentric and depth work runs without divergence.  The depth
-        // test is a minimum, so the queue order does not matter.
-        for (int sb = 0; sb < nrows; sb += NT, par ^= 1) {
-            // each record marks its rows of this sub-round's window (at most 32 rows per record)
-            for (int rr = max(ex, sb), re = min(ex + count, sb + NT); rr < re; ++rr)
-                S.rowmap[rr - sb] = (unsigned short)((tid << 5) | (rr - ex));
-            __syncthreads();
-            const int ri = sb + tid;
-            int len = 0, k = 0, y = 0, xl = 0;
-            if (ri < nrows) {
-                const int m = S.rowmap[tid];
-                k = m >> 5;
-                const FineRec &R = S.rec[k];
-                const int box = R.box;
-                y = rec_y0(box) + (m & 31);
-                xl = rec_x0(box);
-                int xr = rec_x1(box);
-                if (rec_cls(box) == kDirect) {
-                    if ((box >> 23) & 1) row_span32(R, box, y, xl, xr);
-                    else row_span(R, box, y, xl, xr);
-                }
-                len = max(xr - xl + 1, 0);
-            }
-            int npix;
-            const int off = block_scan<NT>(len, S.wsum + (NT / 64) * (1 + par), npix);
-            for (int q0 = 0; q0 < npix; q0 += kQueue) {
-                const int lo = max(off, q0), hi = min(off + len, q0 + kQueue);
-                for (int i = lo; i < hi; ++i) S.queue[i - q0] = k | ((xl + i - off) << 8) | (y << 16);
-                __syncthreads();
-                const int nq = min(kQueue, npix - q0);
-                for (int qi = tid; qi < nq; qi += NT) {
-                    int en = S.queue[qi];
-                    const FineRec &R = S.rec[en & 255];
-                    int lx = (en >> 8) & 255, ly = en >> 16;
-                    TriVerts v = R.v;
-                    float px = S.pxs[lx], py = S.pys[ly];
-                    PixEval p;
-                    eval_pixel(v, px, py, p);
-                    if ((rec_cls(R.box) != kHomog || homog_inside(p)) && p.s != 0.f) {
-                        float zw = p.zn / p.wn;
-                        if (zw >= -1.f && zw <= 1.f) {
-                            unsigned long long key = frag_key(zw, R.t);
-                            int q = ly * TW + lx;
-                            if (!PEEL || key > S.pkey[q]) atomicMin(&S.zbuf[q], key);
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
+    }
+    int nrows;
+    const int ex = block_scan<NT>(count, S.wsum, nrows);  // this lane's record owns rows [ex, ex + count)
+    // Row items (record, tile row) in sub-rounds of NT: each lane finds the
+    // exact covered span of its row; the covered pixels are queued (block
+    // prefix sum, at most kQueue per pass) and evaluated by all lanes, so
+    // the barycentric and depth work runs without divergence.  The depth
+    // test is a minimum, so the queue order does not matter.
+    for (int sb = 0; sb < nrows; sb += NT, par ^= 1) {
+        // each record marks its rows of this sub-round's window (at most 32 rows per record)
+        for (int rr = max(ex, sb), re = min(ex + count, sb + NT); rr < re; ++rr)
+            S.rowmap[rr - sb] = (unsigned short)((tid << 5) | (rr - ex));
         __syncthreads();
+        const int ri = sb + tid;
+        int len = 0, k = 0, y = 0, xl = 0;
+        if (ri < nrows) {
+            const int m = S.rowmap[tid];
+            k = m >> 5;
+            const FineRec &R = S.rec[k];
+            const int box = R.box;
+            y = rec_y0(box) + (m & 31);
+            xl = rec_x0(box);
+            int xr = rec_x1(box);
+            if (rec_cls(box) == kDirect) {
+                if ((box >> 23) & 1) row_span32(R, box, y, xl, xr);
+                else row_span(R, box, y, xl, xr);
+            }
+            len = max(xr - xl + 1, 0);
+        }
+        int npix;
+        const int off = block_scan<NT>(len, S.wsum + (NT / 64) * (1 + par), npix);
+        for (int q0 = 0; q0 < npix; q0 += kQueue) {
+            const int lo = max(off, q0), hi = min(off + len, q0 + kQueue);
+            for (int i = lo; i < hi; ++i) S.queue[i - q0] = k | ((xl + i - off) << 8) | (y << 16);
+            __syncthreads();
+            const int nq = min(kQueue, npix - q0);
+            for (int qi = tid; qi < nq; qi += NT) {
+                int en = S.queue[qi];
+                const FineRec &R = S.rec[en & 255];
+                int lx = (en >> 8) & 255, ly = en >> 16;
+                TriVerts v = R.v;
+                float px = S.pxs[lx], py = S.pys[ly];
+                PixEval p;
+                eval_pixel(v, px, py, p);
+                if ((rec_cls(R.box) != kHomog || homog_inside(p)) && p.s != 0.f) {
+                    float zw = p.zn / p.wn;
+                    if (zw >= -1.f && zw <= 1.f) {
+                        unsigned long long key = frag_key(zw, R.t);
+                        int q = ly * TW + lx;
+                        if (!PEEL || key > S.pkey[q]) atomicMin(&S.zbuf[q], key);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    __syncthreads();
+}
+
+// Depth order of the batch of entries [b0, b0 + n), n <= kOrderRounds NT, into
+// S.order; returns how many are kept.  Dropped here: entries that no pixel of
+// the tile can take (behind every current depth where `behind`; in front of
+// the whole previous layer when peeling; listed triangles whose box misses the
+// tile).  Order and bounds only decide what is skipped: the keys' minimum does
+// not depend on either.
+template <int TW, int TH, bool PEEL>
+__device__ __forceinline__ int fine_order(FineLds<TW, TH, PEEL, true> &S, const FineTile &T, int b0, int n, bool behind,
+                                          const int *__restrict__ bins, const int *__restrict__ lists,
+                                          const int4 *__restrict__ setup) {
+    constexpr int NT = TW * TH;
+    const ImageDesc &d = T.d;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    float zcut = INFINITY, pcut = -INFINITY;
+    if (behind || PEEL) {
+        float zm = -INFINITY, pm = INFINITY;
+#pragma unroll
+        for (int y = 0; y < TH; ++y) {
+            if (behind && y < T.th_img) zm = fmaxf(zm, S.zrow[y]);
+            if (PEEL) pm = fminf(pm, S.prow[y]);
+        }
+        if (behind) zcut = zm;
+        if (PEEL) pcut = pm;
+    }
+    float z[kOrderRounds];
+    float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kOrderRounds; ++j) {
+        z[j] = INFINITY;  // INFINITY: not taken; -INFINITY: no bound
+        const int e = j * NT + tid;
+        if (j * NT >= n) continue;  // uniform
+        const int t = e < n ? fine_entry(T, b0 + e, bins, lists) : -1;
+        if (t < 0) continue;
+        const long long si = 2 * ((long long)d.list_off + (t - d.f0));
+        const int4 sa = setup[si], sb = setup[si + 1];
+        const int cls = sa.w & 3;
+        const float zl = __int_as_float(sb.w);
+        bool keep = cls != kCull && !(zl > zcut) && !(PEEL && unpack_zhi(sa.w) < pcut);
+        if (keep && b0 + e >= T.nbin) {
+            int x0, x1, y0, y1;
+            keep = fine_box(T, cls, sa, sb, x0, x1, y0, y1);
+        }
+        if (!keep) continue;
+        z[j] = zl;
+        if (zl > -INFINITY) {
+            lo = fminf(lo, zl);
+            hi = fmaxf(hi, zl);
+        }
+    }
+    lo = -group_max<64>(-lo);
+    hi = group_max<64>(hi);
+    if ((tid & 63) == 0) {
+        S.zred[2 * wave] = lo;
+        S.zred[2 * wave + 1] = hi;
+    }
+    if (tid < kOrderBuckets) S.hist[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        lo = fminf(lo, S.zred[2 * w]);
+        hi = fmaxf(hi, S.zred[2 * w + 1]);
+    }
+    const float scale = hi > lo ? (float)(kOrderBuckets - 1) / (hi - lo) : 0.f;
+    int place[kOrderRounds];  // bucket << 16 | rank within it; -1: not taken
+#pragma unroll
+    for (int j = 0; j < kOrderRounds; ++j) {
+        place[j] = -1;
+        if (z[j] < INFINITY) {
+            const int b = z[j] > -INFINITY ? min((int)((z[j] - lo) * scale), kOrderBuckets - 1) : 0;
+            place[j] = (b << 16) | atomicAdd(&S.hist[b], 1);
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int c = S.hist[tid], x = wave_incl_scan(c);
+        S.hist[tid] = x - c;
+        if (tid == 63) S.bcast = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kOrderRounds; ++j)
+        if (place[j] >= 0) S.order[S.hist[place[j] >> 16] + (place[j] & 0xffff)] = (unsigned short)(j * NT + tid);
+    const int kept = rfl(S.bcast);
+    __syncthreads();
+    return kept;
+}
+
+// depth test of the tile's entries [e0, e1) into S.zbuf: round by round as they
+// come, or (CULL) in depth order, so that the first round's depths hide most
+// of what follows.  seeded: S.zbuf already holds real keys.
+template <int TW, int TH, bool PEEL, bool CULL>
+__device__ __forceinline__ void fine_entries(FineLds<TW, TH, PEEL, CULL> &S, const FineTile &T, int e0, int e1,
+                                             const float *__restrict__ pos, const int *__restrict__ tri,
+                                             const int *__restrict__ bins, const int *__restrict__ lists,
+                                             const int4 *__restrict__ setup, bool seeded) {
+    constexpr int NT = TW * TH;
+    const int tid = threadIdx.x;
+    int par = 0;  // scan partials of the row spans in use; alternates every sub-round
+    if constexpr (CULL) {
+        __syncthreads();  // the tile's keys and rows are in place
+        for (int b0 = e0; b0 < e1; b0 += kOrderRounds * NT) {
+            const int n = min(kOrderRounds * NT, e1 - b0);
+            bool behind = b0 > e0 || seeded;
+            if (behind) fine_zrow(S, T);
+            const int kept = fine_order<TW, TH, PEEL>(S, T, b0, n, behind, bins, lists, setup);
+            for (int k = 0; k < kept; k += NT) {
+                if (k > 0) {
+                    fine_zrow(S, T);
+                    behind = true;
+                }
+                const int t = k + tid < kept ? fine_entry(T, b0 + S.order[k + tid], bins, lists) : -1;
+                fine_round<TW, TH, PEEL, true>(S, T, t, behind, par, pos, tri, setup);
+            }
+        }
+    } else {
+        for (int base = e0; base < e1; base += NT)
+            fine_round<TW, TH, PEEL, false>(S, T, base + tid < e1 ? fine_entry(T, base + tid, bins, lists) : -1, false, par,
+                                            pos, tri, setup);
     }
 }
 
@@ -643,10 +814,10 @@ __global__ void __launch_bounds__(TW *TH, kFineWavesPerEU) k_fine(Batch b, const
                                                  ItemBox *__restrict__ boxes) {
     constexpr int NT = TW * TH;
     static_assert(NT % 64 == 0, "tile must be a whole number of waves");
-    __shared__ FineLds<TW, TH, PEEL> S;
+    __shared__ FineLds<TW, TH, PEEL, CULL> S;
     int tile = xcd_deal(blockIdx.x, xcd_group);
     if (tile >= n_tiles) return;
-    const FineTile T = fine_begin<TW, TH, PEEL>(S, b, tile, bin_count, list_count, prev);
+    const FineTile T = fine_begin<TW, TH, PEEL, CULL>(S, b, tile, bin_count, list_count, prev);
     int e1 = T.total;
     int slot = -1;
     if (split_slots > 0 && T.total > kSplitRounds * NT) {
@@ -689,7 +860,7 @@ __global__ void __launch_bounds__(TW *TH, kFineWavesPerEU) k_fine_split(Batch b,
                                                  int split_slots, const float4 *__restrict__ prev,
                                                  float4 *__restrict__ rast, float4 *__restrict__ rast_db,
                                                  ItemBox *__restrict__ boxes) {
-    __shared__ FineLds<TW, TH, PEEL> S;
+    __shared__ FineLds<TW, TH, PEEL, CULL> S;
     const SplitWs sp = split_ws(list_count, b.n_img, split_base, split_slots);
     const int nq = sp.ctl[1];  // final: written by the previous kernel
     if (nq == 0) return;
@@ -705,7 +876,7 @@ __global__ void __launch_bounds__(TW *TH, kFineWavesPerEU) k_fine_split(Batch b,
         const int4 inf = sp.info[slot];
         const int itile = __builtin_amdgcn_readfirstlane(inf.x), per = __builtin_amdgcn_readfirstlane(inf.y),
                   nch = __builtin_amdgcn_readfirstlane(inf.z);
-        const FineTile T = fine_begin<TW, TH, PEEL>(S, b, itile, bin_count, list_count, prev);
+        const FineTile T = fine_begin<TW, TH, PEEL, CULL>(S, b, itile, bin_count, list_count, prev);
         const int e0 = chunk * per, e1 = min(e0 + per, T.total);
         unsigned long long *g = sp.gkey + (long long)slot * kMaxFineNT + tid;
         // With the cull, the chunk starts from the tile's keys merged so far
@@ -890,9 +1061,9 @@ static void launch_fine_c(const RasterLaunch &L, hipStream_t st) {
     }
 }
 
-// The culling kernels only where tiles hold many rounds of entries: in
-// one-round tiles the cull never runs, yet its registers and code slow the
-// fine raster slightly.
+// The ordering kernels only where tiles hold many rounds of entries: in
+// one-round tiles there is nothing to order, and the order's LDS, registers and
+// depth bounds would slow the fine raster.
 template <int TW, int TH, bool PEEL, bool DB>
 static void launch_fine_v(const RasterLaunch &L, hipStream_t st) {
     if (L.n_tiles <= 0) return;
@@ -917,8 +1088,12 @@ int launch_rasterize(const RasterLaunch &L, hipStream_t st) {
     hipLaunchKernelGGL(k_zero_i32, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, st, L.bin_count, nz);
     if (L.max_tris > 0) {
         dim3 grid((L.max_tris + 255) / 256, L.b.n_img);
-        hipLaunchKernelGGL(k_setup_bin, grid, dim3(256), 0, st, L.b, L.pos, L.tri, L.tile_w, L.tile_h,
-                           L.bin_count, L.bins, L.list_count, L.lists, L.setup, L.boxes);
+        if (L.depth_cull)
+            hipLaunchKernelGGL(k_setup_bin<true>, grid, dim3(256), 0, st, L.b, L.pos, L.tri, L.tile_w, L.tile_h,
+                               L.bin_count, L.bins, L.list_count, L.lists, L.setup, L.boxes);
+        else
+            hipLaunchKernelGGL(k_setup_bin<false>, grid, dim3(256), 0, st, L.b, L.pos, L.tri, L.tile_w, L.tile_h,
+                               L.bin_count, L.bins, L.list_count, L.lists, L.setup, L.boxes);
     }
     const bool tile_known = (L.tile_w == 8 && L.tile_h == 8) || (L.tile_w == 16 && L.tile_h == 16) ||
                             (L.tile_w == 32 && L.tile_h == 8) || (L.tile_w == 16 && L.tile_h == 8);
