@@ -72,6 +72,9 @@ _SIGS = {
     'drp_stencil_partition_workspace_size': (c_size, [c_int, c_int, c_int]),
     'drp_stencil_partition': (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_size]),
+    'drp_compose_layer_fwd': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_ll, c_void_p, c_void_p]),
+    'drp_compose_layer_bwd': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_ll, c_void_p, c_void_p, c_void_p,
+                                      c_void_p]),
     'drp_count_covered': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     'drp_incidence_workspace_size': (c_size, [c_int, c_int]),
     'drp_incidence_build': (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_size]),

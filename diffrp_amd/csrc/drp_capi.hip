@@ -1043,6 +1043,30 @@ int drp_edge_grad_bwd(void *stream, const float *grad_out, const float *rgb, int
     return 0;
 }
 
+int drp_compose_layer_fwd(void *stream, const float *rgba, const float *rast,
+                          const float *out_prev, const float *trans_prev, long long n_pix, float *out, float *trans) {
+    if (n_pix < 0 || n_pix >= (1ll << 39)) return fail(-1, "pixel count out of range");
+    if (n_pix == 0) return 0;
+    if (!rgba || !rast || !out || !trans || !out_prev != !trans_prev) return fail(-1, "null pointer argument");
+    if (!aligned16(rgba)) return fail(-1, "rgba must be 16-byte aligned");
+    int rc = launch_compose_fwd(rgba, rast, out_prev, trans_prev, n_pix, out, trans, (hipStream_t)stream);
+    if (rc) return fail(rc, "compose launch failed: %s", hipGetErrorString(hipGetLastError()));
+    return 0;
+}
+
+int drp_compose_layer_bwd(void *stream, const float *rgba, const float *rast,
+                          const float *trans_prev, long long n_pix, const float *grad_out, const float *grad_trans,
+                          float *grad_rgba, float *grad_trans_prev) {
+    if (n_pix < 0 || n_pix >= (1ll << 39)) return fail(-1, "pixel count out of range");
+    if (n_pix == 0) return 0;
+    if (!rgba || !rast || !grad_rgba || (grad_trans_prev && !trans_prev)) return fail(-1, "null pointer argument");
+    if (!aligned16(rgba) || !aligned16(grad_rgba)) return fail(-1, "rgba and grad_rgba must be 16-byte aligned");
+    int rc = launch_compose_bwd(rgba, rast, trans_prev, n_pix, grad_out, grad_trans, grad_rgba,
+                                grad_trans_prev, (hipStream_t)stream);
+    if (rc) return fail(rc, "compose backward launch failed: %s", hipGetErrorString(hipGetLastError()));
+    return 0;
+}
+
 int drp_count_covered(void *stream, const float *rast, int n_img, int H, int W, int32_t *counts) {
     if (int e = check_dims(n_img, H, W)) return e;
     if (n_img > 65535) return fail(-1, "at most 65535 images per call (got %d)", n_img);

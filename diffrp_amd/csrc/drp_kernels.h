@@ -259,4 +259,11 @@ int launch_l2_loss_bwd(const float *a, const float *b, long long n, const float 
 int launch_clip_fwd(const float *xyz, int V, const float *VP, int n, float *pos, hipStream_t st);
 int launch_clip_bwd(const float *grad_pos, int V, const float *VP, int n, float *grad_xyz, hipStream_t st);
 
+// one front-to-back compositing step of n pixels (drp_compose.hip)
+int launch_compose_fwd(const float *rgba, const float *rast, const float *out_prev, const float *trans_prev,
+                       long long n, float *out, float *trans, hipStream_t st);
+int launch_compose_bwd(const float *rgba, const float *rast, const float *trans_prev, long long n,
+                       const float *grad_out, const float *grad_trans, float *grad_rgba, float *grad_trans_prev,
+                       hipStream_t st);
+
 }  // namespace drp

@@ -70,12 +70,68 @@ def peel_layers(glctx: 'nvdr.RasterizeCudaContext', pos: torch.Tensor, tri: torc
     return layers
 
 
+def _blend(rgba, rast, out, trans):
+    """One compositing step with torch operators: (out, transmittance) behind the layer."""
+    rgba = rgba * (rast[..., 3:4] > 0).to(rgba.dtype)
+    rgb, a = rgba[..., :3], rgba[..., 3:4]
+    if out is None:
+        return rgb * a, 1.0 - a
+    return out + trans * a * rgb, trans * (1.0 - a)
+
+
+class _Compose(torch.autograd.Function):
+    """``_blend`` as one kernel forward and one backward (``drp_compose.hip``), the same values bit for bit."""
+
+    @staticmethod
+    def forward(fctx, rgba, rast, out, trans):
+        o = torch.empty(rast.shape[:3] + (3,), dtype=torch.float32, device=rgba.device)
+        t = torch.empty(rast.shape[:3] + (1,), dtype=torch.float32, device=rgba.device)
+        check(_lib.lib().drp_compose_layer_fwd(stream_of(rgba), ptr(rgba), ptr(rast), ptr(out), ptr(trans), t.numel(),
+                                               ptr(o), ptr(t)), 'compose')
+        fctx.save_for_backward(rgba, rast, out, trans)
+        fctx.set_materialize_grads(False)
+        return o, t
+
+    @staticmethod
+    def backward(fctx, go, gt):
+        rgba, rast, out, trans = fctx.saved_tensors
+        if go is None and gt is None:
+            return None, None, None, None
+        if torch.is_grad_enabled():  # a differentiable backward: through the operators
+            given = [x for x in (rgba, out, trans) if x is not None and x.requires_grad]
+            res = [(y, g) for y, g in zip(_blend(rgba, rast, out, trans), (go, gt)) if g is not None]
+            got = iter(torch.autograd.grad([y for y, _ in res], given, [g for _, g in res], create_graph=True,
+                                           allow_unused=True))
+            ga, gb, gc = (next(got) if x is not None and x.requires_grad else None for x in (rgba, out, trans))
+            return ga, None, gb, gc
+        go = None if go is None else go.contiguous()
+        gt = None if gt is None else gt.contiguous()
+        grgba = torch.empty(rast.shape, dtype=torch.float32, device=rgba.device)
+        gtrans = torch.empty_like(trans) if trans is not None else None
+        check(_lib.lib().drp_compose_layer_bwd(stream_of(rgba), ptr(rgba), ptr(rast), ptr(trans), rast.numel() // 4,
+                                               ptr(go), ptr(gt), ptr(grgba), ptr(gtrans)), 'compose backward')
+        return grgba, None, go if out is not None else None, gtrans
+
+
+def _compose(rgba, rast, out, trans):
+    # the kernel takes plain float32 buffers; what shade returns otherwise (another type or shape, a
+    # subclass, a forward-mode dual) goes through the operators
+    if (type(rgba) is torch.Tensor and rgba.dtype == torch.float32 and rgba.shape == rast.shape
+            and rgba.device == rast.device and rast.is_contiguous()
+            and (out is None or (out.dtype == torch.float32 and out.is_contiguous() and trans.is_contiguous()))
+            and torch.autograd.forward_ad._current_level < 0):
+        # a slice of a wider buffer is copied out: what is kept for the backward must not hold the buffer
+        if (not rgba.is_contiguous() or rgba.data_ptr() % 16
+                or rgba.untyped_storage().nbytes() > 2 * rgba.numel() * rgba.element_size()):
+            rgba = rgba.clone(memory_format=torch.contiguous_format)
+        return _Compose.apply(rgba, rast, out, trans)
+    return _blend(rgba, rast, out, trans)
+
+
 def _layer(ctx, pos, tri, attr, resolution, prev, shade):
     rast, _ = nvdr._rasterize_impl(ctx, pos, tri, resolution, None, False, prev)
     g, _ = nvdr.interpolate(attr, rast, tri)
-    rgba = shade(g, rast)
-    covered = (rast[..., 3:4] > 0).to(rgba.dtype)
-    return rast, rgba * covered
+    return rast, shade(g, rast)
 
 
 def render_layers(ctx: 'nvdr.RasterizeCudaContext', pos: torch.Tensor, tri: torch.Tensor, attr: torch.Tensor,
@@ -98,13 +154,10 @@ def render_layers(ctx: 'nvdr.RasterizeCudaContext', pos: torch.Tensor, tri: torc
             rast, rgba = ckpt.checkpoint(_layer, ctx, pos, tri, attr, resolution, prev, shade, use_reentrant=False)
         else:
             rast, rgba = _layer(ctx, pos, tri, attr, resolution, prev, shade)
-        rgb, a = rgba[..., :3], rgba[..., 3:4]
-        if out is None:
-            out, trans, first = rgb * a, 1.0 - a, rast
-        else:
-            out = out + trans * a * rgb
-            trans = trans * (1.0 - a)
+        if first is None:
+            first = rast
         prev = rast.detach()
+        out, trans = _compose(rgba, prev, out, trans)
     if antialias:
         out = nvdr.antialias(out.contiguous(), first, pos, tri)
     return out

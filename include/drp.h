@@ -217,6 +217,20 @@ size_t drp_stencil_partition_workspace_size(int H, int W, int n_owner);
 int drp_stencil_partition(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
                           int32_t *order, int32_t *starts, int32_t *ends, void *workspace, size_t workspace_bytes);
 
+/* One step of front-to-back compositing (diffrp blends its peeled layers with
+ * torch operators, diffrp/rendering/surface_deferred.py:348-395): with rgba
+ * masked by the layer's coverage (rast [n_pix,4], id > 0) and T = trans_prev,
+ * out = out_prev + (T a) rgb and trans = T (1 - a); out_prev and trans_prev are
+ * both NULL at the first layer (0 and 1).  rgba [n_pix,4], 16-byte aligned;
+ * out [n_pix,3], trans [n_pix].  Backward:
+ * grad_rgba [n_pix,4] and grad_trans_prev [n_pix] (nullable) written; the
+ * gradient of out_prev is grad_out.  grad_out, grad_trans nullable (zero). */
+int drp_compose_layer_fwd(void *stream, const float *rgba, const float *rast,
+                          const float *out_prev, const float *trans_prev, long long n_pix, float *out, float *trans);
+int drp_compose_layer_bwd(void *stream, const float *rgba, const float *rast,
+                          const float *trans_prev, long long n_pix, const float *grad_out, const float *grad_trans,
+                          float *grad_rgba, float *grad_trans_prev);
+
 /* Covered pixels (id channel > 0) of each of n_img rast images into counts[n]
  * (int32, device; no host synchronisation).  Replaces the host-side emptiness
  * test of the depth-peeling loop, (rast.a <= 0).all() at diffrp/rendering/
