@@ -32,7 +32,26 @@ int fail(int code, const char *fmt, ...) {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-constexpr int kMaxDecisionTris = (1 << 27) - 1;
+// the antialias workspace: per-vertex pixel positions, per-triangle orientation
+// and silhouette flags, the blending pairs (8 bytes for each of the two pairs
+// of a pixel, should all of them blend) and a record per pixel block
+size_t aa_bytes(size_t verts, size_t tris, size_t pixels, size_t blocks) {
+    return align256(verts * 16) + 2 * align256(tris) + 2 * align256(pixels * 8) + align256(blocks * sizeof(AAHalo));
+}
+void aa_pointers(AALaunch &L, void *workspace, size_t verts, size_t tris, size_t pixels) {
+    char *b = (char *)workspace;
+    L.proj = (double2 *)b;
+    b += align256(verts * 16);
+    L.orient = (signed char *)b;
+    b += align256(tris);
+    L.silh = (unsigned char *)b;
+    b += align256(tris);
+    L.ent_w = (float *)b;
+    b += align256(pixels * 8);
+    L.ent_word = (unsigned *)b;
+    b += align256(pixels * 8);
+    L.halo = (AAHalo *)b;
+}
 
 bool tile_ok(int tw, int th) {
     return (tw == 8 && th == 8) || (tw == 16 && th == 16) || (tw == 32 && th == 8) || (tw == 16 && th == 8);
@@ -273,7 +292,8 @@ static size_t plan_desc_off() { return (sizeof(BatchPlanHeader) + 15) & ~(size_t
 static size_t plan_t2i_off(int n_img) { return plan_desc_off() + (size_t)n_img * sizeof(ImageDesc); }
 // item map (UnevenMap) after the tile -> image table: pixel prefix (int64), the
 // vertex, triangle, 16 x 16 tile, 64 x 8 block and 32 x 32 tile prefixes
-// (int32, n + 1 each), then (H, W) per item
+// (int32, n + 1 each; no kernel reads the last, it holds the format), then
+// (H, W) per item
 static size_t plan_map_off(int n_img, long long n_tiles) {
     return (plan_t2i_off(n_img) + sizeof(int32_t) * (size_t)n_tiles + 15) & ~(size_t)15;
 }
@@ -287,7 +307,6 @@ static UnevenMap plan_map(const void *plan, int n_img, long long n_tiles) {
     m.tri = q + (n_img + 1);
     m.bt16 = q + 2 * (n_img + 1);
     m.blk = q + 3 * (n_img + 1);
-    m.t32 = q + 4 * (n_img + 1);
     m.hw = q + 5 * (n_img + 1);
     m.n = n_img;
     return m;
@@ -335,7 +354,7 @@ int drp_batch_plan(const int32_t *items, int n_img, int tile_w, int tile_h, void
         UnevenMap m = plan_map(plan, n_img, tb);
         long long *pix = (long long *)m.pix;
         int32_t *vert = (int32_t *)m.vert, *tri = (int32_t *)m.tri, *bt16 = (int32_t *)m.bt16;
-        int32_t *blk = (int32_t *)m.blk, *t32 = (int32_t *)m.t32, *hw = (int32_t *)m.hw;
+        int32_t *blk = (int32_t *)m.blk, *t32 = blk + (n_img + 1), *hw = (int32_t *)m.hw;
         long long p = 0, v = 0, f = 0, a = 0, k = 0, c = 0;
         for (int i = 0; i <= n_img; ++i) {
             pix[i] = p;
@@ -352,7 +371,7 @@ int drp_batch_plan(const int32_t *items, int n_img, int tile_w, int tile_h, void
             v += V;
             f += F;
             a += (long long)((W + 15) / 16) * ((H + 15) / 16);
-            k += (long long)((W + 63) / 64) * ((H + 7) / 8);
+            k += (long long)((W + kAAW - 1) / kAAW) * ((H + kAAH - 1) / kAAH);
             c += (long long)((W + 31) / 32) * ((H + 31) / 32);
         }
         if (a > 0x7fffffffll || k > 0x7fffffffll || c > 0x7fffffffll) return fail(-1, "batch too large");
@@ -466,7 +485,7 @@ namespace {
 struct PlanView {
     BatchPlanHeader h;
     UnevenMap um;
-    long long bt16, blk, t32;  // totals of the item map's tilings
+    long long bt16, blk;  // totals of the item map's tilings
 };
 
 int plan_view(const void *plan, const void *plan_dev, PlanView &v) {
@@ -477,7 +496,6 @@ int plan_view(const void *plan, const void *plan_dev, PlanView &v) {
     const UnevenMap host = plan_map(plan, v.h.n_img, v.h.n_tiles);
     v.bt16 = host.bt16[v.h.n_img];
     v.blk = host.blk[v.h.n_img];
-    v.t32 = host.t32[v.h.n_img];
     v.um = plan_map(plan_dev, v.h.n_img, v.h.n_tiles);
     return 0;
 }
@@ -711,7 +729,8 @@ size_t drp_batch_antialias_workspace_size(const void *plan) {
     if (!plan) return 0;
     BatchPlanHeader h;
     memcpy(&h, plan, sizeof(h));
-    return align256((size_t)h.n_vert * 16) + 2 * align256((size_t)h.n_tri) + 2 * align256((size_t)h.n_pix * 8);
+    const long long blocks = plan_map(plan, h.n_img, h.n_tiles).blk[h.n_img];
+    return aa_bytes((size_t)h.n_vert, (size_t)h.n_tri, (size_t)h.n_pix, (size_t)blocks);
 }
 
 static int batch_aa_common(AALaunch &L, const PlanView &v, const float *color, int C, const float *rast,
@@ -725,7 +744,6 @@ static int batch_aa_common(AALaunch &L, const PlanView &v, const float *color, i
     size_t need = drp_batch_antialias_workspace_size(plan);
     if (!workspace || workspace_bytes < need)
         return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-    char *b = (char *)workspace;
     L.color = color;
     L.rast = rast;
     L.pos = pos;
@@ -739,18 +757,9 @@ static int batch_aa_common(AALaunch &L, const PlanView &v, const float *color, i
     L.F = (int)v.h.n_tri;
     L.pos_batched = 0;
     L.cv = (C == 1 || C == 3 || C == 4 || C == 8 || C == 16) ? C : 0;
-    size_t o_orient = align256((size_t)v.h.n_vert * 16);
-    size_t o_silh = o_orient + align256((size_t)v.h.n_tri), o_w = o_silh + align256((size_t)v.h.n_tri);
-    size_t o_dec = o_w + align256((size_t)v.h.n_pix * 8);
-    L.proj = (double2 *)b;
-    L.orient = (signed char *)(b + o_orient);
-    L.silh = (unsigned char *)(b + o_silh);
-    L.weights = (float2 *)(b + o_w);
-    L.decisions = v.h.n_tri < kMaxDecisionTris ? (int2 *)(b + o_dec) : nullptr;
+    aa_pointers(L, workspace, (size_t)v.h.n_vert, (size_t)v.h.n_tri, (size_t)v.h.n_pix);
     L.um = v.um;
-    L.total_pix = v.h.n_pix;
     L.total_blk = (int)v.blk;
-    L.total_t32 = (int)v.t32;
     return 0;
 }
 
@@ -786,7 +795,7 @@ int drp_batch_antialias_bwd(void *stream, const void *plan, const void *plan_dev
     L.grad_color = grad_color;
     L.grad_pos = grad_pos;
     L.boost = pos_gradient_boost;
-    L.reuse = reuse_forward && L.decisions != nullptr;
+    L.reuse = reuse_forward;
     int rc = launch_antialias_bwd(L, (hipStream_t)stream);
     if (rc) return fail(rc, "batch antialias backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
@@ -1214,26 +1223,14 @@ int drp_topology_build(void *stream, const int32_t *tri, int F, int32_t *opp, vo
 
 size_t drp_antialias_workspace_size(int n_img, int H, int W, int V, int F, int pos_batched) {
     if (n_img <= 0) return 0;
-    size_t n_proj = pos_batched ? (size_t)n_img : 1;
-    size_t npx = (size_t)n_img * H * W;
-    return align256(n_proj * (size_t)V * 16) + 2 * align256(n_proj * (size_t)F) + 2 * align256(npx * 8);
+    const size_t n_proj = pos_batched ? (size_t)n_img : 1;
+    const size_t blocks = (size_t)((W + kAAW - 1) / kAAW) * ((H + kAAH - 1) / kAAH) * n_img;
+    return aa_bytes(n_proj * V, n_proj * F, (size_t)n_img * H * W, blocks);
 }
 
-// the antialias workspace: per-vertex pixel positions, per-triangle
-// orientation and silhouette flags, per-pixel pair weights and decisions
 static void aa_layout(AALaunch &L, void *workspace, int n_img, int H, int W, int V, int F, int pos_batched) {
     const size_t n_proj = pos_batched ? (size_t)n_img : 1;
-    const size_t npx = (size_t)n_img * H * W;
-    const size_t o_orient = align256(n_proj * (size_t)V * 16);
-    const size_t o_silh = o_orient + align256(n_proj * (size_t)F), o_w = o_silh + align256(n_proj * (size_t)F);
-    const size_t o_dec = o_w + align256(npx * 8);
-    char *b = (char *)workspace;
-    L.proj = (double2 *)b;
-    L.orient = (signed char *)(b + o_orient);
-    L.silh = (unsigned char *)(b + o_silh);
-    L.weights = (float2 *)(b + o_w);
-    // pair decisions pack the triangle into 27 bits; larger meshes recompute them in the backward
-    L.decisions = F < kMaxDecisionTris ? (int2 *)(b + o_dec) : nullptr;
+    aa_pointers(L, workspace, n_proj * V, n_proj * F, (size_t)n_img * H * W);
 }
 
 static int aa_common(AALaunch &L, void *stream, const float *color, int n_img, int H, int W, int C,
@@ -1341,7 +1338,7 @@ int drp_antialias_bwd(void *stream, const float *color, int n_img, int H, int W,
     L.grad_color = grad_color;
     L.grad_pos = grad_pos;
     L.boost = pos_gradient_boost;
-    L.reuse = reuse_forward && L.decisions != nullptr;
+    L.reuse = reuse_forward;
     int rc = launch_antialias_bwd(L, (hipStream_t)stream);
     if (rc) return fail(rc, "antialias_bwd launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;

@@ -15,8 +15,7 @@ struct UnevenMap {
     const int *vert;        // [n + 1] vertex offsets
     const int *tri;         // [n + 1] triangle offsets
     const int *bt16;        // [n + 1] 16 x 16 tiles (deterministic backward)
-    const int *blk;         // [n + 1] 64 x 8 blocks (antialias pairs)
-    const int *t32;         // [n + 1] 32 x 32 tiles (antialias backward)
+    const int *blk;         // [n + 1] 64 x 8 blocks (antialias)
     const int *hw;          // [2 n] (H, W) per item
     int n;
 };
@@ -133,6 +132,15 @@ struct TopoLaunch {
     int *opp;
 };
 
+// pixels of an antialias block, and what the forward leaves of it beside its
+// list of blending pairs: which pairs are listed (right, up per row) and the
+// weights of the pairs that reach in from below and from the left
+constexpr int kAAW = 64, kAAH = 8;
+struct AAHalo {
+    unsigned long long mask[2 * kAAH];
+    float below[kAAW], left[kAAH];
+};
+
 struct AALaunch {
     const float *color, *rast, *pos;
     const int *tri, *opp;
@@ -141,17 +149,17 @@ struct AALaunch {
     double2 *proj;               // [n_proj, V] pixel coordinates (NaN: w <= 0)
     signed char *orient;
     unsigned char *silh;
-    float2 *weights;
-    int2 *decisions;             // [n, H, W] pair decisions for the backward (nullptr: not kept)
+    float *ent_w;                // [2 x pixels] weights of the blending pairs, a run per block
+    unsigned *ent_word;          // [2 x pixels] their edges
+    AAHalo *halo;                // [blocks]
     int reuse;                   // backward: workspace holds the forward's state
     int prepared;                // forward: drp_antialias_prepare filled the per-vertex / per-triangle state
-    float *out;
+    float *out;                  // forward (nullptr: the pair lists alone)
     const float *grad_out;
     float *grad_color, *grad_pos;
     float boost;
     UnevenMap um;                // uneven batch (um.n > 0): n_img items, packed; pos / tri global
-    long long total_pix;         // uneven batch: pixels of all items
-    int total_blk, total_t32;    // uneven batch: pair blocks and backward tiles of all items
+    int total_blk;               // uneven batch: blocks of all items
 };
 
 // channels of one pass of the tile backward (wider attributes take several)
