@@ -629,7 +629,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     b += tile_records_bytes_tiles(v.bt16, tile_record_floats(C, true, true), F);
     int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = launch_corner_slots(inc, inc_off, V, F, slot, st))
+    if (int rc = launch_corner_slots(tri, inc, inc_off, V, F, slot, st))
         return fail(rc, "corner slots launch failed: %s", hipGetErrorString(hipGetLastError()));
     TriBwdLaunch T{};
     T.b.n_img = 1;  // one image of packed items: the item map names each tile's item
@@ -660,11 +660,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     T.local_ids = 0;
     tile_records_layout_tiles(T, records, v.bt16, F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    Fork f{};  // the two vertex gathers are independent
-    const bool par = !rc && fork_begin(st, f);
-    if (!rc) rc = launch_gather_attr(partial_attr, 1, F, V, C, C, 0, 1, 0, inc_off, inc, grad_attr, par ? f.side : st);
-    if (!rc) rc = launch_gather_pos(partial_pos, 1, F, V, 0, inc_off, grad_pos, st);
-    if (par && fork_end(st, f)) rc = -2;
+    if (!rc) rc = launch_gather_both(partial_attr, 1, C, partial_pos, 1, 0, F, V, inc_off, inc, grad_attr, grad_pos, st);
     if (rc) return fail(rc, "batch fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
 }
@@ -1002,7 +998,7 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     b += tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F);
     int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = launch_corner_slots(inc, inc_off, V, F, slot, st))
+    if (int rc = launch_corner_slots(tri, inc, inc_off, V, F, slot, st))
         return fail(rc, "corner slots launch failed: %s", hipGetErrorString(hipGetLastError()));
     TriBwdLaunch T{};
     T.b.n_img = n_img;
@@ -1031,11 +1027,9 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     T.views_per_block = vpg;
     tile_records_layout(T, records, n_img, H, W, (long long)n_img * F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    Fork f{};  // the two vertex gathers are independent
-    const bool par = !rc && fork_begin(st, f);
-    if (!rc) rc = launch_gather_attr(partial_attr, groups, F, V, C, C, 0, 1, 0, inc_off, inc, grad_attr, par ? f.side : st);
-    if (!rc) rc = launch_gather_pos(partial_pos, n_img, F, V, pos_batched, inc_off, grad_pos, st);
-    if (par && fork_end(st, f)) rc = -2;
+    if (!rc)
+        rc = launch_gather_both(partial_attr, groups, C, partial_pos, n_img, pos_batched, F, V, inc_off, inc, grad_attr,
+                                grad_pos, st);
     if (rc) return fail(rc, "fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
 }

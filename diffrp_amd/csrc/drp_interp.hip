@@ -175,125 +175,6 @@ int launch_interpolate(const InterpLaunch &L, hipStream_t st) {
 // k_interp_bwd above remain for rast that comes without pixel boxes (range
 // mode, a modified rast).
 // ----------------------------------------------------------------------------
-// grad_attr[out][v][c0 ..) += sum over groups g in the output's range and
-// incident corners, channel counts that are whole quads, with `lanes` lanes per
-// (vertex, four channels) (1, 2 or 4: up to the groups each output sums): lane
-// s takes groups s, s + lanes, ... (two groups' corner rows in flight together,
-// each group's corners summed in order), and the lanes' sums are added in a
-// fixed tree.  (One lane per (vertex, quad) left the 64-view grid at barely one
-// wave per SIMD waiting on its loads.)
-constexpr int kAttrLanes = 4;
-__global__ void __launch_bounds__(256) k_gather_attr_q(const float *__restrict__ partial, int n_groups, int F,
-                                                       int V, int NC, int ldc, int c0, int per_output_groups,
-                                                       const int *__restrict__ inc_off, const int *__restrict__ inc,
-                                                       float *__restrict__ grad_attr, int lanes) {
-    const int NQ = NC / 4;
-    const long long tl = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = (int)(tl & (lanes - 1));
-    const long long tq = tl / lanes;
-    const int v = (int)(tq / NQ), q = (int)(tq % NQ);
-    const int out = blockIdx.y;
-    if (v >= V) return;  // all lanes of (v, q) together
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int i0 = inc_off[v], i1 = inc_off[v + 1], deg = i1 - i0;
-    const int g0 = per_output_groups ? out : 0, g1 = per_output_groups ? out + 1 : n_groups;
-    const long long gstride = (long long)F * 3 * NC;
-    if (deg <= 8) {
-        int c[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) c[k] = k < deg ? inc[i0 + k] : 0;
-        for (int g = g0 + s; g < g1; g += 2 * lanes) {
-            float4 x[2][8];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int gh = g + h * lanes;
-                const float *P = partial + (long long)gh * gstride + 4 * q;
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (gh < g1 && k < deg) x[h][k] = *reinterpret_cast<const float4 *>(P + (long long)c[k] * NC);
-            }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (g + h * lanes < g1 && k < deg) {
-                        acc.x += x[h][k].x; acc.y += x[h][k].y; acc.z += x[h][k].z; acc.w += x[h][k].w;
-                    }
-        }
-    } else {
-        for (int g = g0 + s; g < g1; g += lanes) {
-            const float *P = partial + (long long)g * gstride + 4 * q;
-            for (int i = i0; i < i1; i += 4) {  // four corners' loads in flight, summed in corner order
-                float4 x[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) x[k] = *reinterpret_cast<const float4 *>(P + (long long)inc[i + k] * NC);
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) {
-                        acc.x += x[k].x; acc.y += x[k].y; acc.z += x[k].z; acc.w += x[k].w;
-                    }
-            }
-        }
-    }
-    for (int o = 1; o < lanes; o <<= 1) {  // (a + b on one lane, b + a on the other: the same sum)
-        acc.x += __shfl_xor(acc.x, o, 64);
-        acc.y += __shfl_xor(acc.y, o, 64);
-        acc.z += __shfl_xor(acc.z, o, 64);
-        acc.w += __shfl_xor(acc.w, o, 64);
-    }
-    if (s != 0) return;
-    float *o = grad_attr + ((long long)out * V + v) * ldc + c0 + 4 * q;
-    o[0] += acc.x;
-    o[1] += acc.y;
-    o[2] += acc.z;
-    o[3] += acc.w;
-}
-
-// The same one lane per (vertex, channel), for channel counts that are not
-// whole quads: consecutive lanes read consecutive floats of a corner's row;
-// four corners' loads in flight, summed in corner order.
-__global__ void __launch_bounds__(256) k_gather_attr_c(const float *__restrict__ partial, int n_groups, int F,
-                                                       int V, int NC, int ldc, int c0, int per_output_groups,
-                                                       const int *__restrict__ inc_off, const int *__restrict__ inc,
-                                                       float *__restrict__ grad_attr) {
-    const long long tl = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int v = (int)(tl / NC), ch = (int)(tl - (long long)v * NC);
-    const int out = blockIdx.y;
-    if (v >= V) return;
-    const int i0 = inc_off[v], i1 = inc_off[v + 1];
-    const int g0 = per_output_groups ? out : 0, g1 = per_output_groups ? out + 1 : n_groups;
-    float s = 0.f;
-    for (int g = g0; g < g1; ++g) {
-        const float *P = partial + (long long)g * F * 3 * NC + ch;
-        for (int i = i0; i < i1; i += 4) {
-            float x[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) x[k] = i + k < i1 ? P[(long long)inc[i + k] * NC] : 0.f;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (i + k < i1) s += x[k];
-        }
-    }
-    grad_attr[((long long)out * V + v) * ldc + c0 + ch] += s;
-}
-
-int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
-                       int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st) {
-    if (V == 0) return 0;
-    if (C % 4 == 0) {
-        const int per_out = per_output ? 1 : groups;
-        const int lanes = per_out >= kAttrLanes ? kAttrLanes : (per_out >= 2 ? 2 : 1);
-        const long long n = (long long)V * (C / 4) * lanes;
-        hipLaunchKernelGGL(k_gather_attr_q, dim3((unsigned)((n + 255) / 256), outs), dim3(256), 0, st, partial,
-                           groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr, lanes);
-    } else {
-        hipLaunchKernelGGL(k_gather_attr_c, dim3((unsigned)(((long long)V * C + 255) / 256), outs), dim3(256), 0, st,
-                           partial, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr);
-    }
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
 // channels of the next pass over an attribute of C channels, `left` to go: at
 // most `most`, and where the rows are not whole quads no multiple of 4 (those
 // passes read 16 bytes at a time)

@@ -211,11 +211,14 @@ int fork_end(hipStream_t main, const Fork &f);
 int launch_tri_bwd_pos(const TriBwdLaunch &L, hipStream_t st);
 int launch_tri_bwd_attr(const TriBwdLaunch &L, int C, hipStream_t st);
 int launch_tri_bwd_fused(const TriBwdLaunch &L, int C, hipStream_t st);
-int launch_corner_slots(const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st);
+int launch_corner_slots(const int *tri, const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st);
 int launch_gather_pos(const float *partial, int n_img, int F, int V, int pos_batched, const int *inc_off,
                       float *grad_pos, hipStream_t st);
 // partial [groups, F, 3, C] added to channels [c0, c0 + C) of grad_attr rows of ldc floats; outs outputs, one
 // group each when per_output
+int launch_gather_both(const float *partial_attr, int groups, int C, const float *partial_pos, int n_img,
+                       int pos_batched, int F, int V, const int *inc_off, const int *inc, float *grad_attr,
+                       float *grad_pos, hipStream_t st);
 int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
                        int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st);
 // floats of a tile record with the attribute and position sums

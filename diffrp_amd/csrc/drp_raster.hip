@@ -948,65 +948,6 @@ __global__ void __launch_bounds__(256) k_raster_bwd(Batch b, const float *__rest
     }
 }
 
-// vertex gather: grad_pos[img][v] += sum over incident corners of partial[pimg][t][corner]
-// (pos_batched: one output per image; else all images sum into one buffer).
-// The corners of a block's 256 vertices are one contiguous range of each
-// image's partials (CSR order): it is staged in LDS with coalesced loads
-// when it fits, and each vertex then sums its slice from there, in corner
-// order as the direct loads do.
-constexpr int kGatherPosLds = 2048;  // float4 per block (32 KiB)
-__global__ void __launch_bounds__(256) k_gather_pos(const float4 *__restrict__ partial, int n_img, int F, int V,
-                                                    int pos_batched, const int *__restrict__ inc_off,
-                                                    float4 *__restrict__ grad_pos) {
-    __shared__ float4 buf[kGatherPosLds];
-    const int vb = blockIdx.x * blockDim.x, v = vb + threadIdx.x;
-    const int oimg = blockIdx.y;
-    const int b0 = inc_off[vb], b1 = inc_off[min(vb + (int)blockDim.x, V)];  // (vb < V: the grid covers V)
-    const bool staged = b1 - b0 <= kGatherPosLds;  // uniform per block
-    const int i0 = v < V ? inc_off[v] : b0, i1 = v < V ? inc_off[v + 1] : b0;
-    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int ia = pos_batched ? oimg : 0, ib = pos_batched ? oimg + 1 : n_img;
-    for (int img = ia; img < ib; ++img) {
-        const float4 *P = partial + (long long)img * F * 3;  // this vertex's corners are P[i0 .. i1)
-        if (staged) {
-            if (img > ia) __syncthreads();  // the previous image's sums have read the buffer
-            for (int i = b0 + (int)threadIdx.x; i < b1; i += blockDim.x) buf[i - b0] = P[i];
-            __syncthreads();
-            for (int i = i0; i < i1; ++i) {
-                const float4 q = buf[i - b0];
-                s.x += q.x; s.y += q.y; s.z += q.z; s.w += q.w;
-            }
-            continue;
-        }
-        // eight corners' loads in flight at once, summed in corner order
-        for (int i = i0; i < i1; i += 8) {
-            float4 q[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (i + k < i1) q[k] = P[i + k];
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (i + k < i1) { s.x += q[k].x; s.y += q[k].y; s.z += q[k].z; s.w += q[k].w; }
-        }
-    }
-    if (v >= V) return;
-    float4 *o = grad_pos + (long long)oimg * V + v;
-    float4 cur = *o;
-    *o = make_float4(cur.x + s.x, cur.y + s.y, cur.z + s.z, cur.w + s.w);
-}
-
-// slot[c] = position of corner c in the incidence list (inverse permutation);
-// -1 for corners whose vertex index is outside [0, V) (not in the list)
-__global__ void k_corner_slots_clear(long long n, int *__restrict__ slot) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) slot[i] = -1;
-}
-__global__ void k_corner_slots(const int *__restrict__ inc, const int *__restrict__ inc_off, int V,
-                               int *__restrict__ slot) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < inc_off[V]) slot[inc[i]] = (int)i;
-}
-
 // ----------------------------------------------------------------------------
 // host launchers
 // ----------------------------------------------------------------------------
@@ -1111,23 +1052,6 @@ int launch_rasterize(const RasterLaunch &L, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_corner_slots(const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st) {
-    long long nc = 3ll * F;
-    if (nc == 0) return 0;
-    hipLaunchKernelGGL(k_corner_slots_clear, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, nc, slot);
-    hipLaunchKernelGGL(k_corner_slots, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, inc, inc_off, V, slot);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-int launch_gather_pos(const float *partial, int n_img, int F, int V, int pos_batched, const int *inc_off,
-                      float *grad_pos, hipStream_t st) {
-    if (V == 0) return 0;
-    int n_out = pos_batched ? n_img : 1;
-    hipLaunchKernelGGL(k_gather_pos, dim3((V + 255) / 256, n_out), dim3(256), 0, st, (const float4 *)partial, n_img, F,
-                       V, pos_batched, inc_off, (float4 *)grad_pos);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
 int launch_rasterize_bwd(const RasterBwdLaunch &L, hipStream_t st) {
     if (L.total_pix == 0) return 0;
     if (L.boxes && L.partial && L.records && L.inc_off && L.inc) {
@@ -1153,18 +1077,10 @@ int launch_rasterize_bwd(const RasterBwdLaunch &L, hipStream_t st) {
         } else {
             tile_records_layout(T, L.records, L.b.n_img, L.b.H, L.b.W, (long long)L.b.n_img * L.b.F);
         }
-        long long nc = 3ll * L.b.F;
-        hipLaunchKernelGGL(k_corner_slots_clear, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, nc,
-                           L.corner_slot);
-        hipLaunchKernelGGL(k_corner_slots, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, L.inc, L.inc_off,
-                           L.b.V, L.corner_slot);
+        if (int rc = launch_corner_slots(L.tri, L.inc, L.inc_off, L.b.V, L.b.F, L.corner_slot, st)) return rc;
         T.corner_slot = L.corner_slot;
         if (int rc = launch_tri_bwd_pos(T, st)) return rc;
-        int n_out = L.b.pos_batched ? L.b.n_img : 1;
-        dim3 gg((L.b.V + 255) / 256, n_out);
-        hipLaunchKernelGGL(k_gather_pos, gg, dim3(256), 0, st, (const float4 *)L.partial, T.n_img, L.b.F, L.b.V,
-                           L.b.pos_batched, L.inc_off, (float4 *)L.grad_pos);
-        return hipGetLastError() == hipSuccess ? 0 : -2;
+        return launch_gather_pos(L.partial, T.n_img, L.b.F, L.b.V, L.b.pos_batched, L.inc_off, L.grad_pos, st);
     }
     dim3 grid((unsigned)((L.total_pix + 255) / 256));
     if (L.grad_db)

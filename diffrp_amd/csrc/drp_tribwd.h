@@ -590,6 +590,7 @@ __device__ __forceinline__ void gather_records(const TriBwdLaunch &L, int t, int
 template <int NA>
 __device__ __forceinline__ void gather_records_fused(const TriBwdLaunch &L, int t, int v0, int v1, float *acc) {
     const int *slot = L.corner_slot + 3 * (long long)t;
+    const unsigned n_c = 3u * (unsigned)L.F;
     float pos[12];
 #pragma unroll
     for (int j = 0; j < 12; ++j) pos[j] = 0.f;
@@ -601,9 +602,9 @@ __device__ __forceinline__ void gather_records_fused(const TriBwdLaunch &L, int 
         },
         [&](int img) {
             float4 *P = reinterpret_cast<float4 *>(L.partial_pos) + (long long)img * 3 * L.F;
-            if (slot[0] >= 0) P[slot[0]] = make_float4(pos[0], pos[1], pos[2], pos[3]);  // -1: vertex out of range
-            if (slot[1] >= 0) P[slot[1]] = make_float4(pos[4], pos[5], pos[6], pos[7]);
-            if (slot[2] >= 0) P[slot[2]] = make_float4(pos[8], pos[9], pos[10], pos[11]);
+            if ((unsigned)slot[0] < n_c) P[slot[0]] = make_float4(pos[0], pos[1], pos[2], pos[3]);  // -1: vertex out of range
+            if ((unsigned)slot[1] < n_c) P[slot[1]] = make_float4(pos[4], pos[5], pos[6], pos[7]);
+            if ((unsigned)slot[2] < n_c) P[slot[2]] = make_float4(pos[8], pos[9], pos[10], pos[11]);
 #pragma unroll
             for (int j = 0; j < 12; ++j) pos[j] = 0.f;
         });
@@ -635,9 +636,10 @@ __global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(
         // corners go to their vertex's slots (CSR order), so the vertex gather reads contiguously
         float4 *P = reinterpret_cast<float4 *>(L.partial) + (long long)grp * 3 * L.F;
         const int *slot = L.corner_slot + 3 * (long long)t;
-        if (slot[0] >= 0) P[slot[0]] = make_float4(acc[0], acc[1], acc[2], acc[3]);  // -1: vertex out of range
-        if (slot[1] >= 0) P[slot[1]] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-        if (slot[2] >= 0) P[slot[2]] = make_float4(acc[8], acc[9], acc[10], acc[11]);
+        const unsigned n_c = 3u * (unsigned)L.F;
+        if ((unsigned)slot[0] < n_c) P[slot[0]] = make_float4(acc[0], acc[1], acc[2], acc[3]);  // -1: vertex out of range
+        if ((unsigned)slot[1] < n_c) P[slot[1]] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+        if ((unsigned)slot[2] < n_c) P[slot[2]] = make_float4(acc[8], acc[9], acc[10], acc[11]);
     } else {
         constexpr int NA = 3 * C;  // the record's attribute part, without its padding
         float *P = L.partial + ((long long)grp * L.F + t) * NA;
