@@ -539,7 +539,9 @@ size_t drp_batch_interpolate_bwd_workspace_size(const void *plan, int C) {
     if (!plan || C <= 0) return 0;
     memcpy(&v.h, plan, sizeof(v.h));
     long long tiles = plan_map(plan, v.h.n_img, v.h.n_tiles).bt16[v.h.n_img];
-    return batch_interp_partial_bytes(v.h, C) + tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, false), v.h.n_tri);
+    return batch_interp_partial_bytes(v.h, C) +
+           tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, false), v.h.n_tri) +
+           align256((size_t)v.h.n_tri);
 }
 
 int drp_batch_interpolate_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr, int C,
@@ -576,6 +578,8 @@ int drp_batch_interpolate_bwd(void *stream, const void *plan, const void *plan_d
     L.boxes = (const ItemBox *)boxes;
     L.partial = (float *)workspace;
     L.records = (char *)workspace + batch_interp_partial_bytes(v.h, C);
+    L.live = (unsigned char *)L.records +
+             tile_records_bytes_tiles(v.bt16, tile_record_floats(pass_width(C), true, false), v.h.n_tri);
     L.inc_off = inc_off;
     L.inc = inc;
     L.um = v.um;
@@ -598,7 +602,7 @@ size_t drp_batch_interpolate_rasterize_bwd_workspace_size(const void *plan, int 
     if (h.n_tri <= 0) return 0;
     long long tiles = plan_map(plan, h.n_img, h.n_tiles).bt16[h.n_img];
     return align256((size_t)h.n_tri * 3 * (size_t)C * 4) + align256((size_t)h.n_tri * 3 * 16) +
-           tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, true), h.n_tri) + align256((size_t)h.n_tri * 3 * 4);
+           tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, true), h.n_tri) + 2 * align256((size_t)h.n_tri);
 }
 
 int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr,
@@ -627,11 +631,10 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     b += align256((size_t)F * 3 * 16);
     void *records = b;
     b += tile_records_bytes_tiles(v.bt16, tile_record_floats(C, true, true), F);
-    int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = launch_corner_slots(tri, inc, inc_off, V, F, slot, st))
-        return fail(rc, "corner slots launch failed: %s", hipGetErrorString(hipGetLastError()));
     TriBwdLaunch T{};
+    T.live = (unsigned char *)b;
+    T.live_pos = T.live + align256((size_t)F);
     T.b.n_img = 1;  // one image of packed items: the item map names each tile's item
     T.b.V = V;
     T.b.F = F;
@@ -650,7 +653,6 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     T.boxes = (const ItemBox *)boxes;
     T.partial = partial_attr;
     T.partial_pos = partial_pos;
-    T.corner_slot = slot;
     T.n_img = 1;
     T.F = F;
     T.H = 1;
@@ -660,7 +662,7 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     T.local_ids = 0;
     tile_records_layout_tiles(T, records, v.bt16, F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    if (!rc) rc = launch_gather_both(partial_attr, 1, C, partial_pos, 1, 0, F, V, inc_off, inc, grad_attr, grad_pos, st);
+    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, st);
     if (rc) return fail(rc, "batch fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
 }
@@ -672,7 +674,7 @@ size_t drp_batch_rasterize_bwd_workspace_size(const void *plan) {
     if (h.n_tri <= 0) return 0;
     long long tiles = plan_map(plan, h.n_img, h.n_tiles).bt16[h.n_img];
     return align256((size_t)h.n_tri * 3 * 16) + tile_records_bytes_tiles(tiles, 12, h.n_tri) +
-           align256((size_t)h.n_tri * 3 * 4);
+           align256((size_t)h.n_tri);
 }
 
 int drp_batch_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *pos, const int32_t *tri,
@@ -710,7 +712,7 @@ int drp_batch_rasterize_bwd(void *stream, const void *plan, const void *plan_dev
     L.boxes = (const ItemBox *)boxes;
     L.partial = (float *)workspace;
     L.records = (char *)workspace + align256((size_t)v.h.n_tri * 3 * 16);
-    L.corner_slot = (int *)((char *)L.records + tile_records_bytes_tiles(v.bt16, 12, v.h.n_tri));
+    L.live = (unsigned char *)L.records + tile_records_bytes_tiles(v.bt16, 12, v.h.n_tri);
     L.inc_off = inc_off;
     L.inc = inc;
     L.um = v.um;
@@ -801,7 +803,7 @@ size_t drp_rasterize_bwd_workspace_size(int n_img, int H, int W, int F) {
     if (n_img <= 0 || F <= 0 || H <= 0 || W <= 0) return 0;
     return align256((size_t)n_img * (size_t)F * 3 * 16) +
            tile_records_bytes(n_img, H, W, 12, (long long)n_img * F) +
-           align256((size_t)F * 3 * 4);
+           align256((size_t)n_img * (size_t)F);
 }
 
 int drp_rasterize_bwd(void *stream, const float *pos, int n_img, int V, int pos_batched, const int32_t *tri, int F,
@@ -826,7 +828,7 @@ int drp_rasterize_bwd(void *stream, const float *pos, int n_img, int V, int pos_
         L.boxes = (const ItemBox *)boxes;
         L.partial = (float *)workspace;
         L.records = (char *)workspace + align256((size_t)n_img * (size_t)F * 3 * 16);
-        L.corner_slot = (int *)((char *)L.records + tile_records_bytes(n_img, H, W, 12, (long long)n_img * F));
+        L.live = (unsigned char *)L.records + tile_records_bytes(n_img, H, W, 12, (long long)n_img * F);
         L.inc_off = inc_off;
         L.inc = inc;
     }
@@ -883,9 +885,12 @@ int drp_interpolate_fwd(void *stream, const float *attr, int n_img, int V, int a
     return 0;
 }
 
+static size_t interp_groups(int n_img, int attr_batched, int views_per_group) {
+    const int vpg = attr_batched ? 1 : views_per_block(views_per_group);
+    return ((size_t)n_img + vpg - 1) / vpg;
+}
 static size_t interp_partial_bytes(int n_img, int F, int C, int attr_batched, int views_per_group) {
-    int vpg = attr_batched ? 1 : views_per_block(views_per_group);
-    size_t groups = ((size_t)n_img + vpg - 1) / vpg;
+    const size_t groups = interp_groups(n_img, attr_batched, views_per_group);
     return align256(groups * (size_t)F * 3 * (size_t)pass_width(C) * 4);
 }
 
@@ -893,7 +898,8 @@ size_t drp_interpolate_bwd_workspace_size(int n_img, int H, int W, int F, int C,
                                           int views_per_group) {
     if (n_img <= 0 || F <= 0 || C <= 0 || H <= 0 || W <= 0) return 0;
     return interp_partial_bytes(n_img, F, C, attr_batched, views_per_group) +
-           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, false), (long long)n_img * F);
+           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, false), (long long)n_img * F) +
+           align256(interp_groups(n_img, attr_batched, views_per_group) * (size_t)F);
 }
 
 int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int attr_batched, int C,
@@ -951,6 +957,8 @@ int drp_interpolate_bwd(void *stream, const float *attr, int n_img, int V, int a
         L.boxes = (const ItemBox *)boxes;
         L.partial = (float *)workspace;
         L.records = (char *)workspace + interp_partial_bytes(n_img, F, C, attr_batched, L.views_per_group);
+        L.live = (unsigned char *)L.records +
+                 tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, false), (long long)n_img * F);
         L.inc_off = inc_off;
         L.inc = inc;
     }
@@ -966,7 +974,8 @@ size_t drp_interpolate_rasterize_bwd_workspace_size(int n_img, int H, int W, int
     const int vpg = views_per_block(views_per_group);
     const size_t groups = (size_t)((n_img + vpg - 1) / vpg);
     return align256(groups * (size_t)F * 3 * (size_t)C * 4) + align256((size_t)n_img * (size_t)F * 3 * 16) +
-           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F) + align256((size_t)F * 3 * 4);
+           tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F) +
+           align256(groups * (size_t)F) + align256((size_t)n_img * (size_t)F);
 }
 
 int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
@@ -996,11 +1005,10 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     b += align256((size_t)n_img * (size_t)F * 3 * 16);
     void *records = b;
     b += tile_records_bytes(n_img, H, W, tile_record_floats(pass_width(C), true, true), (long long)n_img * F);
-    int *slot = (int *)b;
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = launch_corner_slots(tri, inc, inc_off, V, F, slot, st))
-        return fail(rc, "corner slots launch failed: %s", hipGetErrorString(hipGetLastError()));
     TriBwdLaunch T{};
+    T.live = (unsigned char *)b;
+    T.live_pos = T.live + align256((size_t)groups * (size_t)F);
     T.b.n_img = n_img;
     T.b.V = V;
     T.b.F = F;
@@ -1019,7 +1027,6 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     T.boxes = (const ItemBox *)boxes;
     T.partial = partial_attr;
     T.partial_pos = partial_pos;
-    T.corner_slot = slot;
     T.n_img = n_img;
     T.F = F;
     T.H = H;
@@ -1027,9 +1034,7 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     T.views_per_block = vpg;
     tile_records_layout(T, records, n_img, H, W, (long long)n_img * F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    if (!rc)
-        rc = launch_gather_both(partial_attr, groups, C, partial_pos, n_img, pos_batched, F, V, inc_off, inc, grad_attr,
-                                grad_pos, st);
+    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, st);
     if (rc) return fail(rc, "fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
 }

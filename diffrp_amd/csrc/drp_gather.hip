@@ -1,5 +1,6 @@
 // Per-vertex sums of the tile backward's per-corner partials: attributes,
-// positions, and both in one launch, with the tables they read.
+// positions, and both in one launch.  A corner's row is read only if its
+// triangle is live (won a pixel): the tile gather writes no other.
 #include "drp_common.h"
 #include "drp_kernels.h"
 
@@ -7,6 +8,7 @@ namespace drp {
 
 struct AttrGather {
     const float *partial;  // [groups, F, 3, nc]
+    const unsigned char *live;  // [groups, F]: triangles whose rows are written
     int groups, F, V, nc;
     int ldc, c0;           // channels of grad_attr's rows, first channel of this pass
     int per_output;        // one group per output (else every group sums into output 0)
@@ -15,9 +17,10 @@ struct AttrGather {
     float *grad_attr;
 };
 struct PosGather {
-    const float4 *partial;  // [n_img, 3 F], a vertex's corners adjacent
+    const float4 *partial;  // [n_img, 3 F]
+    const unsigned char *live;  // [n_img, F]
     int n_img, F, V, pos_batched;
-    const int *inc_off;
+    const int *inc_off, *inc;
     float4 *grad_pos;
 };
 
@@ -48,35 +51,40 @@ __device__ __forceinline__ void gather_attr_q(const AttrGather &A, int blk, int 
         int c[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) c[k] = k < deg ? inc[i0 + k] : 0;
-        for (int g = g0 + s; g < g1; g += 2 * lanes) {
-            float4 x[2][8];
+        for (int g = g0 + s; g < g1; g += lanes) {
+            const float *P = partial + (long long)g * gstride + 4 * q;
+            const unsigned char *live = A.live + (long long)g * F;
+            float4 x[8];
+            bool on[8];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int gh = g + h * lanes;
-                const float *P = partial + (long long)gh * gstride + 4 * q;
+            for (int k = 0; k < 8; ++k) on[k] = k < deg && live[(unsigned)c[k] / 3u];
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (gh < g1 && k < deg) x[h][k] = *reinterpret_cast<const float4 *>(P + (long long)c[k] * NC);
-            }
+            for (int k = 0; k < 8; ++k)
+                if (on[k]) x[k] = *reinterpret_cast<const float4 *>(P + (long long)c[k] * NC);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (g + h * lanes < g1 && k < deg) {
-                        acc.x += x[h][k].x; acc.y += x[h][k].y; acc.z += x[h][k].z; acc.w += x[h][k].w;
-                    }
+            for (int k = 0; k < 8; ++k)
+                if (on[k]) {
+                    acc.x += x[k].x; acc.y += x[k].y; acc.z += x[k].z; acc.w += x[k].w;
+                }
         }
     } else {
         for (int g = g0 + s; g < g1; g += lanes) {
             const float *P = partial + (long long)g * gstride + 4 * q;
+            const unsigned char *live = A.live + (long long)g * F;
             for (int i = i0; i < i1; i += 4) {  // four corners' loads in flight, summed in corner order
                 float4 x[4];
+                int c[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) c[k] = i + k < i1 ? inc[i + k] : -1;
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) x[k] = *reinterpret_cast<const float4 *>(P + (long long)inc[i + k] * NC);
+                    if (c[k] >= 0 && !live[(unsigned)c[k] / 3u]) c[k] = -1;
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (i + k < i1) {
+                    if (c[k] >= 0) x[k] = *reinterpret_cast<const float4 *>(P + (long long)c[k] * NC);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (c[k] >= 0) {
                         acc.x += x[k].x; acc.y += x[k].y; acc.z += x[k].z; acc.w += x[k].w;
                     }
             }
@@ -111,69 +119,68 @@ __device__ __forceinline__ void gather_attr_c(const AttrGather &A, int blk, int 
     float s = 0.f;
     for (int g = g0; g < g1; ++g) {
         const float *P = partial + (long long)g * F * 3 * NC + ch;
+        const unsigned char *live = A.live + (long long)g * F;
         for (int i = i0; i < i1; i += 4) {
             float x[4];
+            int c[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) x[k] = i + k < i1 ? P[(long long)inc[i + k] * NC] : 0.f;
+            for (int k = 0; k < 4; ++k) c[k] = i + k < i1 ? inc[i + k] : -1;
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                if (i + k < i1) s += x[k];
+                if (c[k] >= 0 && !live[(unsigned)c[k] / 3u]) c[k] = -1;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = c[k] >= 0 ? P[(long long)c[k] * NC] : 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s += x[k];
         }
     }
     A.grad_attr[((long long)out * V + v) * A.ldc + A.c0 + ch] += s;
 }
 
-// vertex gather: grad_pos[img][v] += sum over incident corners of partial[pimg][t][corner]
-// (pos_batched: one output per image; else all images sum into one buffer).
-// The corners of a block's 256 vertices are one contiguous range of each
-// image's partials (CSR order): it is staged in LDS with coalesced loads
-// when it fits, and each vertex then sums its slice from there, in corner
-// order as the direct loads do.
-constexpr int kGatherPosLds = 2048;  // float4 per block (32 KiB)
-__device__ __forceinline__ void gather_pos(const PosGather &G, int blk, int oimg, float4 *buf) {
-    const float4 *__restrict__ partial = G.partial;
-    const int *__restrict__ inc_off = G.inc_off;
-    const int n_img = G.n_img, F = G.F, V = G.V, pos_batched = G.pos_batched;
-    const int vb = blk * blockDim.x, v = vb + threadIdx.x;
-    const int b0 = inc_off[vb], b1 = inc_off[min(vb + (int)blockDim.x, V)];  // (vb < V: the grid covers V)
-    const bool staged = b1 - b0 <= kGatherPosLds;  // uniform per block
-    const int i0 = v < V ? inc_off[v] : b0, i1 = v < V ? inc_off[v + 1] : b0;
+// grad_pos[img][v] += sum over incident corners of partial[pimg][corner]
+// (pos_batched: one output per image; else all images sum into one buffer): a
+// thread per vertex, eight corners' bytes, then their rows, in flight together,
+// summed in corner order
+__device__ __forceinline__ void gather_pos(const PosGather &G, int blk, int oimg) {
+    const int v = blk * blockDim.x + threadIdx.x;
+    if (v >= G.V) return;
+    const int i0 = G.inc_off[v], i1 = G.inc_off[v + 1];
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    const int ia = pos_batched ? oimg : 0, ib = pos_batched ? oimg + 1 : n_img;
+    const int ia = G.pos_batched ? oimg : 0, ib = G.pos_batched ? oimg + 1 : G.n_img;
     for (int img = ia; img < ib; ++img) {
-        const float4 *P = partial + (long long)img * F * 3;  // this vertex's corners are P[i0 .. i1)
-        if (staged) {
-            if (img > ia) __syncthreads();  // the previous image's sums have read the buffer
-            for (int i = b0 + (int)threadIdx.x; i < b1; i += blockDim.x) buf[i - b0] = P[i];
-            __syncthreads();
-            for (int i = i0; i < i1; ++i) {
-                const float4 q = buf[i - b0];
-                s.x += q.x; s.y += q.y; s.z += q.z; s.w += q.w;
-            }
-            continue;
-        }
-        // eight corners' loads in flight at once, summed in corner order
+        const float4 *P = G.partial + (long long)img * G.F * 3;
+        const unsigned char *live = G.live + (long long)img * G.F;
         for (int i = i0; i < i1; i += 8) {
             float4 q[8];
+            int c[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) c[k] = i + k < i1 ? G.inc[i + k] : -1;
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-                if (i + k < i1) q[k] = P[i + k];
+                if (c[k] >= 0 && !live[(unsigned)c[k] / 3u]) c[k] = -1;
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-                if (i + k < i1) { s.x += q[k].x; s.y += q[k].y; s.z += q[k].z; s.w += q[k].w; }
+                if (c[k] >= 0) q[k] = P[c[k]];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (c[k] >= 0) { s.x += q[k].x; s.y += q[k].y; s.z += q[k].z; s.w += q[k].w; }
         }
     }
-    if (v >= V) return;
-    float4 *o = G.grad_pos + (long long)oimg * V + v;
+    float4 *o = G.grad_pos + (long long)oimg * G.V + v;
     float4 cur = *o;
     *o = make_float4(cur.x + s.x, cur.y + s.y, cur.z + s.z, cur.w + s.w);
 }
 
-__global__ void __launch_bounds__(256) k_gather_attr_q(AttrGather A) { gather_attr_q(A, blockIdx.x, blockIdx.y); }
-__global__ void __launch_bounds__(256) k_gather_attr_c(AttrGather A) { gather_attr_c(A, blockIdx.x, blockIdx.y); }
+// Grids are padded to a multiple of 8 blocks (x): XCD k takes the k-th eighth of
+// the vertices, whose corners' rows share cache lines.
+__global__ void __launch_bounds__(256) k_gather_attr_q(AttrGather A) {
+    gather_attr_q(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
+}
+__global__ void __launch_bounds__(256) k_gather_attr_c(AttrGather A) {
+    gather_attr_c(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
+}
 __global__ void __launch_bounds__(256) k_gather_pos(PosGather G) {
-    __shared__ float4 buf[kGatherPosLds];
-    gather_pos(G, blockIdx.x, blockIdx.y, buf);
+    gather_pos(G, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
 }
 
 // Both gathers of the fused backward (one attribute output), the first
@@ -182,78 +189,64 @@ __global__ void __launch_bounds__(256) k_gather_pos(PosGather G) {
 // stream and four event calls (some 15 us of host time) to overlap.
 template <bool QUADS>
 __global__ void __launch_bounds__(256) k_gather_both(AttrGather A, PosGather G, int attr_blocks, int pos_blocks) {
-    __shared__ float4 buf[kGatherPosLds];
     const int blk = blockIdx.x;
     if (blk < attr_blocks) {
-        if (QUADS) gather_attr_q(A, blk, 0);
-        else gather_attr_c(A, blk, 0);
+        if (QUADS) gather_attr_q(A, xcd_remap(blk, attr_blocks), 0);
+        else gather_attr_c(A, xcd_remap(blk, attr_blocks), 0);
         return;
     }
-    const int p = blk - attr_blocks;
-    gather_pos(G, p % pos_blocks, p / pos_blocks, buf);
+    const int p = blk - attr_blocks, img = p / pos_blocks;
+    gather_pos(G, xcd_remap(p - img * pos_blocks, pos_blocks), img);
 }
 
-// slot[c] = position of corner c in the incidence list (the list's inverse),
-// -1 for corners whose vertex index is outside [0, V): those are not listed
-__global__ void k_corner_slots(const int *__restrict__ tri, const int *__restrict__ inc,
-                               const int *__restrict__ inc_off, int V, long long n, int *__restrict__ slot) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if ((unsigned)tri[i] >= (unsigned)V) slot[i] = -1;
-    if (i < inc_off[V]) slot[inc[i]] = (int)i;
-}
-
-int launch_corner_slots(const int *tri, const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st) {
-    const long long nc = 3ll * F;
-    if (nc == 0) return 0;
-    hipLaunchKernelGGL(k_corner_slots, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, st, tri, inc, inc_off, V, nc,
-                       slot);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-static AttrGather attr_gather(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int per_output,
-                              const int *inc_off, const int *inc, float *grad_attr) {
+static AttrGather attr_gather(const float *partial, const unsigned char *live, int groups, int F, int V, int C,
+                              int ldc, int c0, int per_output, const int *inc_off, const int *inc, float *grad_attr) {
     const int per_out = per_output ? 1 : groups;
     const int lanes = per_out >= kAttrLanes ? kAttrLanes : (per_out >= 2 ? 2 : 1);
-    return {partial, groups, F, V, C, ldc, c0, per_output, lanes, inc_off, inc, grad_attr};
+    return {partial, live, groups, F, V, C, ldc, c0, per_output, lanes, inc_off, inc, grad_attr};
 }
+static unsigned blocks8(long long n) { return (unsigned)(((n + 255) / 256 + 7) & ~7ll); }
 static unsigned attr_blocks(const AttrGather &A) {
-    const long long n = A.nc % 4 == 0 ? (long long)A.V * (A.nc / 4) * A.lanes : (long long)A.V * A.nc;
-    return (unsigned)((n + 255) / 256);
+    return blocks8(A.nc % 4 == 0 ? (long long)A.V * (A.nc / 4) * A.lanes : (long long)A.V * A.nc);
 }
 
-int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
-                       int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st) {
+int launch_gather_attr(const float *partial, const unsigned char *live, int groups, int F, int V, int C, int ldc,
+                       int c0, int outs, int per_output, const int *inc_off, const int *inc, float *grad_attr,
+                       hipStream_t st) {
     if (V == 0) return 0;
-    const AttrGather A = attr_gather(partial, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr);
+    const AttrGather A = attr_gather(partial, live, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr);
     const dim3 grid(attr_blocks(A), outs);
     if (C % 4 == 0) hipLaunchKernelGGL(k_gather_attr_q, grid, dim3(256), 0, st, A);
     else hipLaunchKernelGGL(k_gather_attr_c, grid, dim3(256), 0, st, A);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_gather_pos(const float *partial, int n_img, int F, int V, int pos_batched, const int *inc_off,
-                      float *grad_pos, hipStream_t st) {
+int launch_gather_pos(const float *partial, const unsigned char *live, int n_img, int F, int V, int pos_batched,
+                      const int *inc_off, const int *inc, float *grad_pos, hipStream_t st) {
     if (V == 0) return 0;
-    const PosGather G{(const float4 *)partial, n_img, F, V, pos_batched, inc_off, (float4 *)grad_pos};
-    hipLaunchKernelGGL(k_gather_pos, dim3((V + 255) / 256, pos_batched ? n_img : 1), dim3(256), 0, st, G);
+    const PosGather G{(const float4 *)partial, live, n_img, F, V, pos_batched, inc_off, inc, (float4 *)grad_pos};
+    hipLaunchKernelGGL(k_gather_pos, dim3(blocks8(V), pos_batched ? n_img : 1), dim3(256), 0, st, G);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_gather_both(const float *partial_attr, int groups, int C, const float *partial_pos, int n_img,
-                       int pos_batched, int F, int V, const int *inc_off, const int *inc, float *grad_attr,
+int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const int *inc, float *grad_attr,
                        float *grad_pos, hipStream_t st) {
-    if (V == 0) return 0;
-    const AttrGather A = attr_gather(partial_attr, groups, F, V, C, C, 0, 0, inc_off, inc, grad_attr);
-    const PosGather G{(const float4 *)partial_pos, n_img, F, V, pos_batched, inc_off, (float4 *)grad_pos};
-    const unsigned na = attr_blocks(A), np = (unsigned)((V + 255) / 256);
-    const unsigned long long blocks = na + (unsigned long long)np * (pos_batched ? n_img : 1);
+    if (T.V == 0) return 0;
+    const int groups = (T.n_img + T.views_per_block - 1) / T.views_per_block;
+    const AttrGather A =
+        attr_gather(T.partial, T.live, groups, T.F, T.V, C, C, 0, 0, inc_off, inc, grad_attr);
+    const PosGather G{(const float4 *)T.partial_pos, T.live_pos, T.n_img, T.F, T.V, T.b.pos_batched, inc_off, inc,
+                      (float4 *)grad_pos};
+    const unsigned na = attr_blocks(A), np = blocks8(T.V);
+    const unsigned long long blocks = na + (unsigned long long)np * (T.b.pos_batched ? T.n_img : 1);
     if (blocks >= (1ull << 31)) {  // past one launch's blocks
-        if (int rc = launch_gather_attr(partial_attr, groups, F, V, C, C, 0, 1, 0, inc_off, inc, grad_attr, st)) return rc;
-        return launch_gather_pos(partial_pos, n_img, F, V, pos_batched, inc_off, grad_pos, st);
+        if (int rc = launch_gather_attr(T.partial, T.live, groups, T.F, T.V, C, C, 0, 1, 0, inc_off, inc, grad_attr, st))
+            return rc;
+        return launch_gather_pos(T.partial_pos, T.live_pos, T.n_img, T.F, T.V, T.b.pos_batched, inc_off, inc, grad_pos, st);
     }
-    if (C % 4 == 0) hipLaunchKernelGGL((k_gather_both<true>), dim3((unsigned)blocks), dim3(256), 0, st, A, G, (int)na, (int)np);
-    else hipLaunchKernelGGL((k_gather_both<false>), dim3((unsigned)blocks), dim3(256), 0, st, A, G, (int)na, (int)np);
+    const dim3 grid((unsigned)blocks);
+    if (C % 4 == 0) hipLaunchKernelGGL((k_gather_both<true>), grid, dim3(256), 0, st, A, G, (int)na, (int)np);
+    else hipLaunchKernelGGL((k_gather_both<false>), grid, dim3(256), 0, st, A, G, (int)na, (int)np);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

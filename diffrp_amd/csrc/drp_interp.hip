@@ -203,6 +203,7 @@ static int launch_interp_bwd_tri(const InterpLaunch &L, hipStream_t st) {
     T.grad_db_out = L.grad_db;
     T.boxes = L.boxes;
     T.partial = L.partial;
+    T.live = L.live;
     T.n_img = n_img;
     T.F = L.F;
     T.H = L.H;
@@ -221,8 +222,8 @@ static int launch_interp_bwd_tri(const InterpLaunch &L, hipStream_t st) {
         T.c0 = c0;
         T.accum = c0 > 0;
         if (int rc = launch_tri_bwd_attr(T, nc, st)) return rc;
-        if (int rc = launch_gather_attr(L.partial, groups, L.F, L.V, nc, L.C, c0, outs, L.attr_batched, L.inc_off,
-                                        L.inc, L.grad_attr, st))
+        if (int rc = launch_gather_attr(L.partial, L.live, groups, L.F, L.V, nc, L.C, c0, outs, L.attr_batched,
+                                        L.inc_off, L.inc, L.grad_attr, st))
             return rc;
         c0 += nc;
     }

@@ -88,9 +88,9 @@ struct RasterBwdLaunch {
     int pix_per_img;
     // triangle-centric path (all set) or per-pixel atomics (any null)
     const ItemBox *boxes;
-    float *partial;          // [n_img, 3F] float4, corners in vertex (CSR) order
+    float *partial;          // [n_img, 3F] float4
     void *records;           // tile records (tile_records_bytes(n_img, H, W, 12, n_img * F))
-    int *corner_slot;        // [3F]: position of corner 3t+k in the incidence list
+    unsigned char *live;     // [n_img, F]: the partial's written triangles
     const int *inc_off, *inc;
     UnevenMap um;            // uneven batch (um.n > 0): packed items, global vertices
     long long um_tiles;      // uneven batch: 16 x 16 tiles of all items
@@ -115,6 +115,7 @@ struct InterpLaunch {
     int H, W;
     const ItemBox *boxes;
     float *partial;          // [groups, F, 3, min(C, kMaxPassChannels)]
+    unsigned char *live;     // [groups, F]
     void *records;           // tile records of min(C, kMaxPassChannels) channels
     const int *inc_off, *inc;
     int views_per_group;
@@ -185,7 +186,7 @@ struct TriBwdLaunch {
     const ItemBox *boxes;
     float *partial;
     float *partial_pos;      // fused mode: the position partial [n_img, 3F] float4 (partial: attributes)
-    const int *corner_slot;  // positions mode: partial index of corner 3t+k (vertex order)
+    unsigned char *live, *live_pos;  // [groups, F], fused mode [n_img, F]: triangles whose partials are written
     int n_img, F, H, W;
     int views_per_block;     // images summed per partial (attribute mode); 1 for positions
     // per-tile records (16 x 16 tiles): count, triangle, sums
@@ -211,16 +212,16 @@ int fork_end(hipStream_t main, const Fork &f);
 int launch_tri_bwd_pos(const TriBwdLaunch &L, hipStream_t st);
 int launch_tri_bwd_attr(const TriBwdLaunch &L, int C, hipStream_t st);
 int launch_tri_bwd_fused(const TriBwdLaunch &L, int C, hipStream_t st);
-int launch_corner_slots(const int *tri, const int *inc, const int *inc_off, int V, int F, int *slot, hipStream_t st);
-int launch_gather_pos(const float *partial, int n_img, int F, int V, int pos_batched, const int *inc_off,
-                      float *grad_pos, hipStream_t st);
-// partial [groups, F, 3, C] added to channels [c0, c0 + C) of grad_attr rows of ldc floats; outs outputs, one
-// group each when per_output
-int launch_gather_both(const float *partial_attr, int groups, int C, const float *partial_pos, int n_img,
-                       int pos_batched, int F, int V, const int *inc_off, const int *inc, float *grad_attr,
+// partial (and its live triangles) [groups, F, 3, C] added to channels [c0, c0 + C) of grad_attr rows of ldc
+// floats; outs outputs, one group each when per_output
+int launch_gather_attr(const float *partial, const unsigned char *live, int groups, int F, int V, int C, int ldc,
+                       int c0, int outs, int per_output, const int *inc_off, const int *inc, float *grad_attr,
+                       hipStream_t st);
+int launch_gather_pos(const float *partial, const unsigned char *live, int n_img, int F, int V, int pos_batched,
+                      const int *inc_off, const int *inc, float *grad_pos, hipStream_t st);
+// both, after launch_tri_bwd_fused(T, C, ..)
+int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const int *inc, float *grad_attr,
                        float *grad_pos, hipStream_t st);
-int launch_gather_attr(const float *partial, int groups, int F, int V, int C, int ldc, int c0, int outs,
-                       int per_output, const int *inc_off, const int *inc, float *grad_attr, hipStream_t st);
 // floats of a tile record with the attribute and position sums
 int tile_record_floats(int C, bool attr, bool pos);
 // workspace of the tile records for nv floats per record and n_boxes pixel

@@ -1077,10 +1077,9 @@ int launch_rasterize_bwd(const RasterBwdLaunch &L, hipStream_t st) {
         } else {
             tile_records_layout(T, L.records, L.b.n_img, L.b.H, L.b.W, (long long)L.b.n_img * L.b.F);
         }
-        if (int rc = launch_corner_slots(L.tri, L.inc, L.inc_off, L.b.V, L.b.F, L.corner_slot, st)) return rc;
-        T.corner_slot = L.corner_slot;
+        T.live = L.live;
         if (int rc = launch_tri_bwd_pos(T, st)) return rc;
-        return launch_gather_pos(L.partial, T.n_img, L.b.F, L.b.V, L.b.pos_batched, L.inc_off, L.grad_pos, st);
+        return launch_gather_pos(L.partial, L.live, T.n_img, L.b.F, L.b.V, L.b.pos_batched, L.inc_off, L.inc, L.grad_pos, st);
     }
     dim3 grid((unsigned)((L.total_pix + 255) / 256));
     if (L.grad_db)

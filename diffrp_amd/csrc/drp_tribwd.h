@@ -22,14 +22,13 @@
 // for bit.
 //
 //   POS  (12 floats): d rast (u, v, z/w [, db]) -> d clip (x, y, z, w) of the 3
-//        corners (double-precision chain, drp_grad.h); partial [n, 3F] float4
-//        with the corners of each vertex adjacent (incidence order), summed per
-//        vertex by k_gather_pos.
+//        corners (double-precision chain, drp_grad.h); partial [n, 3F] float4,
+//        summed per vertex by the position gather.
 //   ATTR (3 C floats): (u, v, 1-u-v) * g per corner, plus the terms of the
 //        screen-space derivatives' gradients where those are wanted; the same
 //        pass writes grad_rast = (<g, a0-a2>, <g, a1-a2>, 0, 0) (and grad_db);
 //        k_tile_gather sums the views of a group, partial [groups, F, 3, C],
-//        reduced by k_gather_attr.
+//        summed per vertex by the attribute gather.
 //   BOTH (3 C + 12): the attribute sums, then the position sums of the
 //        grad_rast just computed, from one sort and one record search.
 // C is a compile-time count of 1 .. 16 channels; wider attributes go through
@@ -465,12 +464,16 @@ __device__ __forceinline__ BoxLoad load_box(const TriBwdLaunch &L, long long bi)
     return x;
 }
 
+__device__ __forceinline__ bool box_hit(const ItemBox &b) {  // won a pixel, inside its box
+    return b.hit && (b.cc & 0xffff) <= (int)((unsigned)b.cc >> 16) && (b.rr & 0xffff) <= (int)((unsigned)b.rr >> 16);
+}
+
+// (box_hit holds)
 template <int NV, typename Add>
 __device__ __forceinline__ void image_records(const TriBwdLaunch &L, int t, const BoxLoad &x, int tile_base,
                                               int tiles_x, Add &&add) {
     const ItemBox &b = x.b;
     const int c0 = b.cc & 0xffff, c1 = (unsigned)b.cc >> 16, r0 = b.rr & 0xffff, r1 = (unsigned)b.rr >> 16;
-    if (!b.hit || c0 > c1 || r0 > r1) return;
     const int tx0 = c0 / kBT, tx1 = c1 / kBT, ty0 = r0 / kBT, bw = tx1 - tx0 + 1;
     const int nb = bw * (r1 / kBT - ty0 + 1);
     int k0 = 0;
@@ -540,8 +543,8 @@ __device__ __forceinline__ void image_records(const TriBwdLaunch &L, int t, cons
     }
 }
 
-// Records of triangle t over images [v0, v1) in (image, tile) order; done(img)
-// after each image.  Uniform batch: box of (image, t) at image * F + t, tile
+// Records of triangle t over images [v0, v1) in (image, tile) order; done(img,
+// won a pixel) after each image.  Uniform batch: box of (image, t) at image * F + t, tile
 // image * tiles_per_img + ty * tiles_x + tx.  Uneven batch: t's item only, box
 // at t, tiles from the item's first.  The next image's box and slots are
 // loaded before this image's records are read.
@@ -564,8 +567,9 @@ __device__ __forceinline__ void triangle_records(const TriBwdLaunch &L, int t, i
     for (int img = v0; img < v1; ++img) {
         BoxLoad nxt;
         if (img + 1 < v1) nxt = load_box(L, (img + 1) * box_stride + t);
-        image_records<NV>(L, t, cur, tile_base + img * tile_stride, tiles_x, add);
-        done(img);
+        const bool hit = box_hit(cur.b);
+        if (hit) image_records<NV>(L, t, cur, tile_base + img * tile_stride, tiles_x, add);
+        done(img, hit);
         if (img + 1 < v1) cur = nxt;
     }
 }
@@ -581,33 +585,45 @@ __device__ __forceinline__ void add_record(float *acc, const float *q) {
 }
 
 template <int NV>
-__device__ __forceinline__ void gather_records(const TriBwdLaunch &L, int t, int v0, int v1, float *acc) {
-    triangle_records<NV>(L, t, v0, v1, [&](const float *q) { add_record<NV>(acc, q); }, [](int) {});
+__device__ __forceinline__ bool gather_records(const TriBwdLaunch &L, int t, int v0, int v1, float *acc) {
+    bool any = false;
+    triangle_records<NV>(
+        L, t, v0, v1, [&](const float *q) { add_record<NV>(acc, q); }, [&](int, bool hit) { any = any || hit; });
+    return any;
+}
+
+// corners of (image, triangle) i: 48 consecutive bytes
+__device__ __forceinline__ void store_pos(float *partial, long long i, const float *pos) {
+    float4 *P = reinterpret_cast<float4 *>(partial) + 3 * i;
+    P[0] = make_float4(pos[0], pos[1], pos[2], pos[3]);
+    P[1] = make_float4(pos[4], pos[5], pos[6], pos[7]);
+    P[2] = make_float4(pos[8], pos[9], pos[10], pos[11]);
 }
 
 // MODE 2: the attribute sums over the group's images (as MODE 1), and per
-// image the position sums, written to that image's corner slots (as MODE 0)
+// image the position sums, written to that image's partial (as MODE 0)
 template <int NA>
-__device__ __forceinline__ void gather_records_fused(const TriBwdLaunch &L, int t, int v0, int v1, float *acc) {
-    const int *slot = L.corner_slot + 3 * (long long)t;
-    const unsigned n_c = 3u * (unsigned)L.F;
+__device__ __forceinline__ bool gather_records_fused(const TriBwdLaunch &L, int t, int v0, int v1, float *acc) {
     float pos[12];
 #pragma unroll
     for (int j = 0; j < 12; ++j) pos[j] = 0.f;
+    bool any = false;
     triangle_records<NA + 12>(
         L, t, v0, v1,
         [&](const float *q) {
             add_record<NA>(acc, q);
             add_record<12>(pos, q + NA);
         },
-        [&](int img) {
-            float4 *P = reinterpret_cast<float4 *>(L.partial_pos) + (long long)img * 3 * L.F;
-            if ((unsigned)slot[0] < n_c) P[slot[0]] = make_float4(pos[0], pos[1], pos[2], pos[3]);  // -1: vertex out of range
-            if ((unsigned)slot[1] < n_c) P[slot[1]] = make_float4(pos[4], pos[5], pos[6], pos[7]);
-            if ((unsigned)slot[2] < n_c) P[slot[2]] = make_float4(pos[8], pos[9], pos[10], pos[11]);
+        [&](int img, bool hit) {
+            const long long i = (long long)img * L.F + t;
+            L.live_pos[i] = hit;
+            if (!hit) return;
+            any = true;
+            store_pos(L.partial_pos, i, pos);
 #pragma unroll
             for (int j = 0; j < 12; ++j) pos[j] = 0.f;
         });
+    return any;
 }
 
 // Waves per SIMD the register budget is cut for: 6 keeps the latency-bound
@@ -630,19 +646,19 @@ __global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(
     for (int j = 0; j < NV; ++j) acc[j] = 0.f;
     const int VB = L.views_per_block;
     const int v0 = grp * VB, v1 = min(v0 + VB, L.n_img);
-    if (MODE == 2) gather_records_fused<rec_attr<MODE, C>()>(L, t, v0, v1, acc);
-    else gather_records<NV>(L, t, v0, v1, acc);
+    // Only triangles that won a pixel have sums: the others' partials are neither
+    // written here nor read by the vertex gathers, which look at one byte each
+    // (half of a mesh faces away, and a dense one hides most of the rest).
+    const bool hit = MODE == 2 ? gather_records_fused<rec_attr<MODE, C>()>(L, t, v0, v1, acc)
+                               : gather_records<NV>(L, t, v0, v1, acc);
+    const long long gt = (long long)grp * L.F + t;
+    L.live[gt] = hit;
+    if (!hit) return;
     if (MODE == 0) {
-        // corners go to their vertex's slots (CSR order), so the vertex gather reads contiguously
-        float4 *P = reinterpret_cast<float4 *>(L.partial) + (long long)grp * 3 * L.F;
-        const int *slot = L.corner_slot + 3 * (long long)t;
-        const unsigned n_c = 3u * (unsigned)L.F;
-        if ((unsigned)slot[0] < n_c) P[slot[0]] = make_float4(acc[0], acc[1], acc[2], acc[3]);  // -1: vertex out of range
-        if ((unsigned)slot[1] < n_c) P[slot[1]] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-        if ((unsigned)slot[2] < n_c) P[slot[2]] = make_float4(acc[8], acc[9], acc[10], acc[11]);
+        store_pos(L.partial, gt, acc);
     } else {
         constexpr int NA = 3 * C;  // the record's attribute part, without its padding
-        float *P = L.partial + ((long long)grp * L.F + t) * NA;
+        float *P = L.partial + gt * NA;
         if (NA % 4 == 0) {
 #pragma unroll
             for (int j = 0; j < NA; j += 4)
