@@ -70,6 +70,8 @@ _SIGS = {
     'drp_sample3d_bwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_ll, c_int, c_int,
                                  c_void_p, c_void_p, c_void_p]),
     'drp_stencil_partition_workspace_size': (c_size, [c_int, c_int, c_int]),
+    'drp_stencil_fragments': (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p,
+                                      c_ll, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size]),
     'drp_stencil_partition': (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_size]),
     'drp_compose_layer_fwd': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_ll, c_void_p, c_void_p]),

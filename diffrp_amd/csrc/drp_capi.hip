@@ -1151,19 +1151,38 @@ size_t drp_stencil_partition_workspace_size(int H, int W, int n_owner) {
     return stencil_partition_ws_bytes((long long)H * W, n_owner);
 }
 
-int drp_stencil_partition(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
-                          int32_t *order, int32_t *starts, int32_t *ends, void *workspace, size_t workspace_bytes) {
+static int stencil_partition(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F,
+                             int n_owner, int32_t *order, float *frag, long long n_frag, int64_t *rows, int64_t *cols,
+                             int32_t *starts, int32_t *ends, void *workspace, size_t workspace_bytes) {
     if (int e = check_dims(1, H, W)) return e;
     if (F < 0 || n_owner < 0 || n_owner >= (1 << 30)) return fail(-1, "bad F or owner count");
     if (!rast || !stencils || !order || !starts || !ends) return fail(-1, "null pointer argument");
     if (!aligned16(rast)) return fail(-1, "rast must be 16-byte aligned");
-    const size_t need = stencil_partition_ws_bytes((long long)H * W, n_owner);
+    const long long npx = (long long)H * W;
+    const size_t need = stencil_partition_ws_bytes(npx, n_owner);
     if (!workspace || workspace_bytes < need)
         return fail(-1, "workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
-    int rc = launch_stencil_partition(rast, (long long)H * W, stencils, F, n_owner, order, starts, ends, workspace,
-                                      (hipStream_t)stream);
+    const PartitionLaunch L{rast, npx, W, stencils, F, n_owner, order, starts, ends, frag, n_frag, (long long *)rows,
+                            (long long *)cols};
+    int rc = launch_stencil_partition(L, workspace, (hipStream_t)stream);
     if (rc) return fail(rc, "stencil partition launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
+}
+
+int drp_stencil_partition(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
+                          int32_t *order, int32_t *starts, int32_t *ends, void *workspace, size_t workspace_bytes) {
+    return stencil_partition(stream, rast, H, W, stencils, F, n_owner, order, nullptr, 0, nullptr, nullptr, starts, ends,
+                             workspace, workspace_bytes);
+}
+
+int drp_stencil_fragments(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
+                          int32_t *order, float *frag, long long n_frag, int64_t *rows, int64_t *cols, int32_t *starts,
+                          int32_t *ends, void *workspace, size_t workspace_bytes) {
+    if (!frag || !rows || !cols) return fail(-1, "null pointer argument");
+    if (!aligned16(frag)) return fail(-1, "frag must be 16-byte aligned");
+    if (n_frag < (long long)H * W || n_frag > (1ll << 31)) return fail(-1, "frag must hold at least H * W fragments");
+    return stencil_partition(stream, rast, H, W, stencils, F, n_owner, order, frag, n_frag, rows, cols, starts, ends,
+                             workspace, workspace_bytes);
 }
 
 size_t drp_incidence_workspace_size(int V, int F) { return V > 0 && F >= 0 ? incidence_ws_bytes(V, F) : 0; }

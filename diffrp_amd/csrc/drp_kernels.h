@@ -163,6 +163,18 @@ struct AALaunch {
     int total_blk;               // uneven batch: blocks of all items
 };
 
+struct PartitionLaunch {
+    const float *rast;  // one layer of npx pixels, W wide
+    long long npx;
+    int W;
+    const int *stencils;  // [F + 1]
+    int F, n_owner;
+    int *order, *starts, *ends;
+    float *frag;            // [n_frag, 4] or nullptr (then rows and cols are not written either)
+    long long n_frag;       // at least npx; the rest is zeroed
+    long long *rows, *cols;
+};
+
 // channels of one pass of the tile backward (wider attributes take several)
 constexpr int kMaxPassChannels = 16;
 
@@ -258,8 +270,7 @@ int launch_sample3d(const float *tex, int D, int H, int W, int C, const float *u
                     float *out, hipStream_t st);
 int launch_sample3d_bwd(const float *tex, int D, int H, int W, int C, const float *uvw, long long n, int wrap,
                         int mode, const float *gout, float *gtex, float *guvw, hipStream_t st);
-int launch_stencil_partition(const float *rast, long long npx, const int *stencils, int F, int n_owner, int *order,
-                             int *starts, int *ends, void *ws, hipStream_t st);
+int launch_stencil_partition(const PartitionLaunch &L, void *ws, hipStream_t st);
 int launch_count_covered(const float *rast, int n_img, long long npx, int *counts, hipStream_t st);
 int launch_incidence(const int *tri, int F, int V, int *inc_off, int *inc, void *ws, hipStream_t st);
 size_t l2_loss_ws_bytes();

@@ -125,9 +125,13 @@ class MaskedSparseInterpolator:
     materialising the [P, 3, C] corner rows)."""
 
     def __init__(self, rast: torch.Tensor, tris: torch.Tensor, mask: Optional[torch.Tensor] = None,
-                 pixels: Optional[torch.Tensor] = None):
+                 pixels: Optional[torch.Tensor] = None, run: Optional['_Run'] = None):
         self.tris = tris
-        if pixels is None:
+        self.run = run
+        if run is not None:  # an owner's run of a partitioned layer
+            self.indices = run.indices()
+            self.vi_data = run.layer.frag[run.start:run.end]
+        elif pixels is None:
             self.indices = mask.nonzero(as_tuple=True)
             self.vi_data = rast[self.indices]
         else:  # flat row-major pixel ids of a [1, H, W, 4] layer (from stencil_partition)
@@ -147,8 +151,15 @@ class MaskedSparseInterpolator:
         P, C = self.vi_data.shape[0], values.shape[-1]
         if P == 0:
             return values.new_zeros(0, C)
-        frag = self.vi_data.contiguous()
         rows = -(-P // _FRAG_ROW)
+        if self.run is not None and not (torch.is_grad_enabled() and values.requires_grad):
+            # whole rows of the layer's fragments: what follows the run (other owners' fragments, then
+            # zeros) is interpolated and cut off
+            s = self.run.start
+            frag = self.run.layer.frag[s:s + (rows * _FRAG_ROW if rows > 1 else P)]
+            out, _ = nvdr.interpolate(values.float().contiguous(), frag.view(1, rows, -1, 4), self.tris)
+            return out.view(-1, C)[:P]
+        frag = self.vi_data.contiguous()
         if rows > 1:  # an image row holds at most _FRAG_ROW fragments; the padding is empty (id 0)
             frag = torch.cat([frag, frag.new_zeros(rows * _FRAG_ROW - P, 4)])
         frag = frag.view(1, rows, -1, 4)
@@ -156,24 +167,65 @@ class MaskedSparseInterpolator:
         return out.view(-1, C)[:P]
 
 
+@dataclass
+class _LayerRuns:
+    """A layer's pixels in owner order: fragments [H*W (+ whole rows), 4], row and
+    column indices [H*W], one zero."""
+    frag: torch.Tensor
+    rows: torch.Tensor
+    cols: torch.Tensor
+    zero: torch.Tensor
+
+
+@dataclass
+class _Run:
+    layer: _LayerRuns
+    start: int
+    end: int
+
+    def indices(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+        return (self.layer.zero.expand(self.end - self.start), self.layer.rows[self.start:self.end],
+                self.layer.cols[self.start:self.end])
+
+
+def _join_runs(runs: Sequence[Optional[_Run]]) -> Optional[_Run]:
+    """The runs as one, when they follow one another in the same layer."""
+    if any(r is None for r in runs) or any(a.layer is not b.layer or a.end != b.start for a, b in zip(runs, runs[1:])):
+        return None
+    return _Run(runs[0].layer, runs[0].start, runs[-1].end)
+
+
+def _partition(rast: torch.Tensor, stencils: torch.Tensor, n_owner: int, fragments: bool):
+    from . import _lib
+    from ._lib import check, ptr, stream_of
+    H, W = rast.shape[1], rast.shape[2]
+    N = H * W
+    rast = rast.contiguous()
+    st = stencils.int().contiguous()
+    L = _lib.lib()
+    order = torch.empty(N, dtype=torch.int32, device=rast.device)
+    se = torch.empty(2, n_owner + 1, dtype=torch.int32, device=rast.device)
+    ws_bytes = L.drp_stencil_partition_workspace_size(H, W, n_owner)
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=rast.device)
+    if not fragments:
+        check(L.drp_stencil_partition(stream_of(rast), ptr(rast), H, W, ptr(st), st.numel() - 1, n_owner, ptr(order),
+                                      ptr(se[0]), ptr(se[1]), ptr(ws), ws_bytes), 'stencil partition')
+        return order, se.cpu().t().tolist(), None
+    frag = torch.empty(N + _FRAG_ROW, 4, dtype=torch.float32, device=rast.device)
+    rc = torch.empty(2, N, dtype=torch.int64, device=rast.device)
+    check(L.drp_stencil_fragments(stream_of(rast), ptr(rast), H, W, ptr(st), st.numel() - 1, n_owner, ptr(order),
+                                  ptr(frag), frag.shape[0], ptr(rc[0]), ptr(rc[1]), ptr(se[0]), ptr(se[1]), ptr(ws),
+                                  ws_bytes), 'stencil partition')
+    layer = _LayerRuns(frag, rc[0], rc[1], torch.zeros(1, dtype=torch.int64, device=rast.device))
+    return order, se.cpu().t().tolist(), layer
+
+
 def stencil_partition(rast: torch.Tensor, stencils: torch.Tensor, n_owner: int):
     """Pixels of one layer [1, H, W, 4] grouped by owner = stencils[id]
     (``surface_deferred.py:283-284``): returns (order [H*W] int32 on the device,
     [(start, end)] per owner 0..n_owner on the host), with one host read for
     the whole layer.  Within an owner the pixels are in row-major order."""
-    from . import _lib
-    from ._lib import check, ptr, stream_of
-    H, W = rast.shape[1], rast.shape[2]
-    rast = rast.contiguous()
-    st = stencils.int().contiguous()
-    L = _lib.lib()
-    order = torch.empty(H * W, dtype=torch.int32, device=rast.device)
-    se = torch.empty(2, n_owner + 1, dtype=torch.int32, device=rast.device)
-    ws_bytes = L.drp_stencil_partition_workspace_size(H, W, n_owner)
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=rast.device)
-    check(L.drp_stencil_partition(stream_of(rast), ptr(rast), H, W, ptr(st), st.numel() - 1, n_owner, ptr(order),
-                                  ptr(se[0]), ptr(se[1]), ptr(ws), ws_bytes), 'stencil partition')
-    return order, se.cpu().t().tolist()
+    return _partition(rast, stencils, n_owner, False)[:2]
 
 
 # ----------------------------------------------------------------------------
@@ -399,6 +451,17 @@ class SurfaceDeferredRenderSessionOptions:
             self.max_layers = 32767
 
 
+def _fill_value(default: Sequence[float], dev) -> torch.Tensor:
+    """[C] of ``default`` on the device by fill kernels (copying it from host memory
+    waits for the stream)."""
+    v = torch.full((len(default),), float(default[0]), dtype=torch.float32, device=dev) if default else \
+        torch.empty(0, dtype=torch.float32, device=dev)
+    for i, x in enumerate(default):
+        if x != default[0]:
+            v[i].fill_(float(x))
+    return v
+
+
 _tls = threading.local()
 
 
@@ -452,12 +515,15 @@ class SurfaceDeferredRenderSession:
             if len(w) != 1:
                 raise ValueError(f'custom attribute {k!r} has different widths across objects')
             widths[k] = w.pop()
-        base, tris, stencil = 0, [], [torch.zeros(1, dtype=torch.int64, device=dev)]
+        base, tris = 0, []
+        stencils = torch.zeros(1 + sum(len(o.tris) for o in objs), dtype=torch.int32, device=dev)
+        at = 1
         for i, o in enumerate(objs):
             if o.tris.shape[-1] != 3:
                 raise ValueError('triangles must have 3 vertex indices')
-            tris.append(o.tris + base)
-            stencil.append(torch.full((len(o.tris),), i + 1, dtype=torch.int64, device=dev))
+            tris.append(o.tris + base if base or len(objs) == 1 else o.tris)
+            stencils[at:at + len(o.tris)].fill_(i + 1)
+            at += len(o.tris)
             base += len(o.verts)
 
         def cat(name, width=None):
@@ -478,7 +544,7 @@ class SurfaceDeferredRenderSession:
             verts=cat('verts', 3), normals=cat('normals', 3),
             world_pos=world[0] if len(world) == 1 else torch.cat(world),
             tris=(tris[0] if len(tris) == 1 else torch.cat(tris)).int().contiguous(),
-            stencils=torch.cat(stencil).int().contiguous(),
+            stencils=stencils,
             color=cat('color'), uv=cat('uv', 2), tangents=cat('tangents', 4), custom_attrs=custom)
 
     @_memo
@@ -505,7 +571,9 @@ class SurfaceDeferredRenderSession:
         n_obj = len(self.scene.objects)
         for rast in self.rasterize():
             if self.options.interpolator_impl == 'stencil_masked':
-                order, runs = stencil_partition(rast, vao.stencils, n_obj)
+                # the fragments come with the partition unless a gradient goes through them to rast
+                taped = rast.requires_grad or torch.autograd.forward_ad._current_level >= 0
+                order, runs, layer = _partition(rast, vao.stencils, n_obj, not taped)
             per_obj = []
             for i, obj in enumerate(self.scene.objects):
                 su = SurfaceUniform(obj.M, V, P)
@@ -513,7 +581,11 @@ class SurfaceDeferredRenderSession:
                     si = SurfaceInput(su, vao, FullScreenInterpolator(rast, vao.tris))
                 elif self.options.interpolator_impl == 'stencil_masked':
                     s, e = runs[i + 1]
-                    si = SurfaceInput(su, vao, MaskedSparseInterpolator(rast, vao.tris, pixels=order[s:e]))
+                    if layer is not None:
+                        interp = MaskedSparseInterpolator(rast, vao.tris, run=_Run(layer, s, e))
+                    else:
+                        interp = MaskedSparseInterpolator(rast, vao.tris, pixels=order[s:e])
+                    si = SurfaceInput(su, vao, interp)
                     if len(si.interpolator.indices[0]) == 0:
                         per_obj.append((si, SurfaceOutputStandard()))
                         continue
@@ -532,9 +604,9 @@ class SurfaceDeferredRenderSession:
         C = len(default)
         out = []
         if self.options.interpolator_impl == 'stencil_masked':
-            fill = torch.tensor(default, dtype=torch.float32, device=dev).expand(1, h, w, C)
+            fill = _fill_value(default, dev).expand(1, h, w, C)
             for mats in self.layer_material():
-                idx, vals = [], []
+                idx, vals, runs = [], [], []
                 for si, so in mats:
                     if len(si.interpolator.indices[0]) == 0:
                         continue
@@ -542,12 +614,15 @@ class SurfaceDeferredRenderSession:
                     if v is not None:
                         idx.append(si.interpolator.indices)
                         vals.append(v)
+                        runs.append(getattr(si.interpolator, 'run', None))
                 if not idx:
                     out.append(fill)
                 elif len(idx) == 1:
                     out.append(fill.index_put(idx[0], vals[0]))
                 else:
-                    cat_idx = tuple(torch.cat([ix[d] for ix in idx]) for d in range(len(idx[0])))
+                    joined = _join_runs(runs)
+                    cat_idx = joined.indices() if joined is not None else \
+                        tuple(torch.cat([ix[d] for ix in idx]) for d in range(len(idx[0])))
                     out.append(fill.index_put(cat_idx, torch.cat(vals)))
             return out
         vao = self.vertex_array_object()
@@ -630,12 +705,12 @@ class SurfaceDeferredRenderSession:
 
     @_memo
     def camera_space_normal_layered(self):
-        V = self.camera.V()
+        V = self.camera_V()
         return [normalized(xform_dir(n, V)) for n in self.world_space_normal_layered()]
 
     @_memo
     def depth_layered(self):
-        V = self.camera.V()
+        V = self.camera_V()
         return self.gbuffer_collect(lambda si, so: -xform_affine(si.world_pos, V)[..., 2:3], [0.0])
 
     @_memo

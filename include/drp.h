@@ -216,6 +216,12 @@ int drp_sample3d_bwd(void *stream, const float *tex, int D, int H, int W, int C,
 size_t drp_stencil_partition_workspace_size(int H, int W, int n_owner);
 int drp_stencil_partition(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
                           int32_t *order, int32_t *starts, int32_t *ends, void *workspace, size_t workspace_bytes);
+/* The same, and what a masked interpolation takes per pixel, in `order`'s order:
+ * frag [n_frag,4] the pixels' rast values (n_frag >= H*W, the rows past H*W
+ * zero, so that a run may be read in whole image rows), rows and cols [H*W]. */
+int drp_stencil_fragments(void *stream, const float *rast, int H, int W, const int32_t *stencils, int F, int n_owner,
+                          int32_t *order, float *frag, long long n_frag, int64_t *rows, int64_t *cols, int32_t *starts,
+                          int32_t *ends, void *workspace, size_t workspace_bytes);
 
 /* One step of front-to-back compositing (diffrp blends its peeled layers with
  * torch operators, diffrp/rendering/surface_deferred.py:348-395): with rgba
