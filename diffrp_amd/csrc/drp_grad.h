@@ -33,8 +33,11 @@ __device__ __forceinline__ double drcp(double x) {
 // NDC centre of pixel column c (row r) in double: (2c + 1 - W) / W
 __device__ __forceinline__ double pix_ndc_d(int c, int W) { return (double)(2 * c + 1 - W) / (double)W; }
 
-// px, py: the pixel's NDC centre, pix_ndc_d(c, W), pix_ndc_d(r, H)
-template <bool DB>
+// px, py: the pixel's NDC centre, pix_ndc_d(c, W), pix_ndc_d(r, H).  Z: g may
+// hold a gradient of z/w (an interpolation's grad_rast never does, and without
+// one the whole z/w chain falls away: a sixth of the backward's instructions
+// with the products written as FMAs, which the compiler may not form here).
+template <bool DB, bool Z>
 __device__ __forceinline__ void raster_pixel_grad_at(const TriVerts &v, double px, double py, float4 g, float4 gd,
                                                      float4 out[3]) {
     double X[3], Y[3], wk[3], zk[3], e[3];
@@ -49,11 +52,15 @@ __device__ __forceinline__ void raster_pixel_grad_at(const TriVerts &v, double p
     e[1] = dfma(X[2], Y[0], -(X[0] * Y[2]));
     e[2] = dfma(X[0], Y[1], -(X[1] * Y[0]));
     const double s = (e[0] + e[1]) + e[2];
-    const double zn = dfma(e[0], zk[0], dfma(e[1], zk[1], e[2] * zk[2]));
-    const double wn = dfma(e[0], wk[0], dfma(e[1], wk[1], e[2] * wk[2]));
-    const double inv_s = drcp(s), inv_wn = drcp(wn);
-    const double u = e[0] * inv_s, vv = e[1] * inv_s, zw = zn * inv_wn;
-    double gu = g.x, gv = g.y, gz = g.z;
+    const double inv_s = drcp(s);
+    const double u = e[0] * inv_s, vv = e[1] * inv_s;
+    double zw = 0.0, gzw = 0.0;
+    if (Z) {
+        const double inv_wn = drcp(dfma(e[0], wk[0], dfma(e[1], wk[1], e[2] * wk[2])));
+        zw = dfma(e[0], zk[0], dfma(e[1], zk[1], e[2] * zk[2])) * inv_wn;
+        gzw = (double)g.z * inv_wn;
+    }
+    double gu = g.x, gv = g.y;
     double gX[3] = {0.0, 0.0, 0.0}, gY[3] = {0.0, 0.0, 0.0}, gw[3] = {0.0, 0.0, 0.0}, gs = 0.0;
     if (DB) {
         double ex[3], ey[3];
@@ -79,28 +86,35 @@ __device__ __forceinline__ void raster_pixel_grad_at(const TriVerts &v, double p
         gw[2] += gey[1] * X[0]; gX[0] += gey[1] * wk[2]; gw[0] -= gey[1] * X[2]; gX[2] -= gey[1] * wk[0];
         gw[0] += gey[2] * X[1]; gX[1] += gey[2] * wk[0]; gw[1] -= gey[2] * X[0]; gX[0] -= gey[2] * wk[1];
     }
-    double gzw = gz * inv_wn;
-    double G0 = (gu * (1.0 - u) + gv * (-vv)) * inv_s + gs + gzw * (zk[0] - zw * wk[0]);
-    double G1 = (gu * (-u) + gv * (1.0 - vv)) * inv_s + gs + gzw * (zk[1] - zw * wk[1]);
-    double G2 = (gu * (-u) + gv * (-vv)) * inv_s + gs + gzw * (zk[2] - zw * wk[2]);
-    gX[0] += G2 * Y[1] - G1 * Y[2];
-    gX[1] += G0 * Y[2] - G2 * Y[0];
-    gX[2] += G1 * Y[0] - G0 * Y[1];
-    gY[0] += G1 * X[2] - G2 * X[1];
-    gY[1] += G2 * X[0] - G0 * X[2];
-    gY[2] += G0 * X[1] - G1 * X[0];
+    const double h = dfma(gu, u, gv * vv);
+    double G[3] = {(gu - h) * inv_s, (gv - h) * inv_s, -h * inv_s};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        double ek = e[k];
-        out[k] = make_float4((float)gX[k], (float)gY[k], (float)(gzw * ek),
-                             (float)(gw[k] - px * gX[k] - py * gY[k] - gzw * zw * ek));
+        if (DB) G[k] += gs;
+        if (Z) G[k] = dfma(gzw, dfma(-zw, wk[k], zk[k]), G[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int i = (k + 1) % 3, j = (k + 2) % 3;
+        double x = dfma(G[j], Y[i], -(G[i] * Y[j])), y = dfma(G[i], X[j], -(G[j] * X[i]));
+        if (DB) {
+            x += gX[k];
+            y += gY[k];
+        }
+        double w = dfma(-py, y, -(px * x)), z = 0.0;
+        if (DB) w += gw[k];
+        if (Z) {
+            z = gzw * e[k];
+            w = dfma(-zw, z, w);
+        }
+        out[k] = make_float4((float)x, (float)y, (float)z, (float)w);
     }
 }
 
 template <bool DB>
 __device__ __forceinline__ void raster_pixel_grad(const TriVerts &v, int c, int r, int H, int W, float4 g, float4 gd,
                                                   float4 out[3]) {
-    raster_pixel_grad_at<DB>(v, pix_ndc_d(c, W), pix_ndc_d(r, H), g, gd, out);
+    raster_pixel_grad_at<DB, true>(v, pix_ndc_d(c, W), pix_ndc_d(r, H), g, gd, out);
 }
 
 __device__ __forceinline__ float4 db_grad_scaled(float4 gd, int H, int W) {

@@ -112,25 +112,20 @@ __device__ __forceinline__ void attr_sums(const float4 *w, const float4 *g, cons
             for (int p = p0; p < p1; ++p) {
                 const float4 wp = w[p], gp = gr[p];
                 const float wv[3] = {wp.x, wp.y, wp.z}, gv[4] = {gp.x, gp.y, gp.z, gp.w};
-                float t[3][4];
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) t[j][c] = wv[j] * gv[c];
+                    for (int c = 0; c < 4; ++c) s[j][c] = fma_(wv[j], gv[c], s[j][c]);
                 if (DA) {
                     const float4 a = k[q * kBTP + p], b = k[(NQ + q) * kBTP + p];
                     const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
-                        t[0][c] += av[c];
-                        t[1][c] += bv[c];
-                        t[2][c] -= av[c] + bv[c];
+                        s[0][c] += av[c];
+                        s[1][c] += bv[c];
+                        s[2][c] -= av[c] + bv[c];
                     }
                 }
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) s[j][c] += t[j][c];
             }
             float *o = rec + (long long)sg * nv + 4 * q;
 #pragma unroll
@@ -158,15 +153,19 @@ __device__ __forceinline__ void attr_sums(const float4 *w, const float4 *g, cons
         for (int p = live ? seg_start[sg] + l : 0; p < p1; p += lanes) {
             const float wv = wj[4 * p];
             const float4 gp = gr[p];
-            float t[4] = {wv * gp.x, wv * gp.y, wv * gp.z, wv * gp.w};
+            const float gv[4] = {gp.x, gp.y, gp.z, gp.w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[c] = fma_(wv, gv[c], s[c]);
             if (DA) {
                 const float4 a = k[q * kBTP + p], b = k[(NQ + q) * kBTP + p];
                 const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-                for (int c = 0; c < 4; ++c) t[c] = j == 0 ? t[c] + av[c] : (j == 1 ? t[c] + bv[c] : t[c] - (av[c] + bv[c]));
+                for (int c = 0; c < 4; ++c) {
+                    if (j == 0) s[c] += av[c];
+                    else if (j == 1) s[c] += bv[c];
+                    else s[c] -= av[c] + bv[c];
+                }
             }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] += t[c];
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) s[c] = lanes_sum(s[c], lanes);
@@ -302,9 +301,9 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C, DB>())) k_tile_red
         return;
     }
     // The gradients of narrow attributes and the corners' positions are asked for
-    // before the sort, which hides their latency.  Wider ones would cost registers:
-    // at C = 8, both sums, they spill (456 against 412 us at 64 x 512^2).
-    constexpr bool kEarly = MODE == 1 ? C <= 8 : MODE == 2 && C <= 4;
+    // before the sort, which hides their latency, as far as the registers go: at
+    // C = 8, both sums, 381 us with the gradients at 64 x 512^2, 386 without or with both.
+    constexpr bool kEarly = MODE != 0 && C <= 8;
     constexpr bool kEarlyPos = MODE == 0 || (MODE == 2 && C <= 4);
     float4 early_g[kEarly ? NQ : 1];
     TriVerts tv;
@@ -374,8 +373,8 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C, DB>())) k_tile_red
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
                     if (4 * q + k < C) {
-                        su += gv[k] * (p0[k] - p2[k]);
-                        sv += gv[k] * (p1[k] - p2[k]);
+                        su = fma_(gv[k], p0[k] - p2[k], su);
+                        sv = fma_(gv[k], p1[k] - p2[k], sv);
                     }
             }
             rows[my] = make_float4(u, v, (1.f - u) - v, 0.f);
@@ -432,7 +431,7 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C, DB>())) k_tile_red
         if (MODE == 2) __syncthreads();  // the attribute sums have read the rows
         if (t >= 0) {
             float4 o[3];
-            raster_pixel_grad_at<MODE == 0 && DB>(tv, spx[tid & 15], spy[tid >> 4], g, gd, o);
+            raster_pixel_grad_at<MODE == 0 && DB, MODE == 0>(tv, spx[tid & 15], spy[tid >> 4], g, gd, o);
 #pragma unroll
             for (int q = 0; q < 3; ++q) rows[q * kBTP + my] = o[q];
         }
