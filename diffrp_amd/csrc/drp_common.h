@@ -139,24 +139,18 @@ __device__ __forceinline__ bool load_tri(const float *__restrict__ pos, const in
     return true;
 }
 
-__device__ __forceinline__ long long floor_div16(long long a) {  // floor(a / 16)
-    return a >> 4;
-}
-
 // pixel box (centres inside the snapped vertices' bounding box), clipped to
-// the image; false when empty
+// the image; false when empty.  Snapped coordinates stay within (kGuard + 1) *
+// kMaxRes / 2 * kSubpix of the origin, far inside 32 bits.
 __device__ __forceinline__ bool direct_box(const int X[3], const int Y[3], int H, int W, int &bc0, int &bc1,
                                            int &br0, int &br1) {
-    int mnx = min(X[0], min(X[1], X[2])), mxx = max(X[0], max(X[1], X[2]));
-    int mny = min(Y[0], min(Y[1], Y[2])), mxy = max(Y[0], max(Y[1], Y[2]));
-    long long c0 = -floor_div16(-((long long)mnx - kHalfSub)), c1 = floor_div16((long long)mxx - kHalfSub);
-    long long r0 = -floor_div16(-((long long)mny - kHalfSub)), r1 = floor_div16((long long)mxy - kHalfSub);
-    c0 = c0 < 0 ? 0 : c0;
-    r0 = r0 < 0 ? 0 : r0;
-    c1 = c1 > W - 1 ? W - 1 : c1;
-    r1 = r1 > H - 1 ? H - 1 : r1;
+    const int mnx = min(X[0], min(X[1], X[2])), mxx = max(X[0], max(X[1], X[2]));
+    const int mny = min(Y[0], min(Y[1], Y[2])), mxy = max(Y[0], max(Y[1], Y[2]));
+    // ceil((lo - half) / 16), floor((hi - half) / 16)
+    const int c0 = max((mnx - kHalfSub + kSubpix - 1) >> 4, 0), c1 = min((mxx - kHalfSub) >> 4, W - 1);
+    const int r0 = max((mny - kHalfSub + kSubpix - 1) >> 4, 0), r1 = min((mxy - kHalfSub) >> 4, H - 1);
     if (c0 > c1 || r0 > r1) return false;
-    bc0 = (int)c0; bc1 = (int)c1; br0 = (int)r0; br1 = (int)r1;
+    bc0 = c0; bc1 = c1; br0 = r0; br1 = r1;
     return true;
 }
 

@@ -166,21 +166,28 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
         }
     }
     bool live = valid && s.cls != kCull;
-    int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1, ntiles = 0;
+    // tile edges are powers of two; a tile grid has at most 2048 columns and rows
+    const int sw = __builtin_ctz(tile_w), sh = __builtin_ctz(tile_h);
+    int tx0 = 0, ty0 = 0, ncols = 0, ntiles = 0;
     if (live) {
-        tx0 = s.c0 / tile_w; tx1 = s.c1 / tile_w; ty0 = s.r0 / tile_h; ty1 = s.r1 / tile_h;
-        ntiles = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
+        tx0 = s.c0 >> sw;
+        ty0 = s.r0 >> sh;
+        ncols = (s.c1 >> sw) - tx0 + 1;
+        ntiles = ncols * ((s.r1 >> sh) - ty0 + 1);
     }
     const bool large = live && ntiles > kMaxBinTiles;
     bool spill = large;
     int mine = (live && !spill) ? ntiles : 0;
-    int ncols = tx1 - tx0 + 1;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, t_wave = t - lane;
+    // first tile and columns of a binned triangle (at most kMaxBinTiles = 64): 11, 11 and 7 bits
+    const unsigned first = (unsigned)tx0 | (unsigned)ty0 << 11 | (unsigned)ncols << 22;
+    __shared__ int owner[256];
+    int *own = owner + (threadIdx.x & ~63);  // this wave's
     // The wave's (triangle, tile) pairs are numbered in lane order (lane i's
     // triangle owns pairs [excl, incl)) and inserted 64 per round, so a round
-    // is full whatever the spread of tile counts.  Each lane finds its pair's
-    // triangle by a binary search over the lanes' inclusive counts; the wave
-    // sorts the pairs' (tile, lane) keys; the first lane of each run of one
+    // is full whatever the spread of tile counts.  Each triangle marks its first
+    // pair of the round with its lane, and a running maximum hands the mark to
+    // its other pairs; the wave sorts the pairs' (tile, lane) keys; the first lane of each run of one
     // tile reserves the run's slots with one atomic -- all runs at once -- and
     // every sorted lane writes the triangle of the pair its key came from.  A
     // full bin hands the flag back to the pair's lane, and a triangle with a
@@ -193,18 +200,20 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
     for (int r0 = 0; r0 < total; r0 += 64) {
         const int p = r0 + lane;
         const bool active = p < total;
-        int sl = 0;  // the pair's lane: the number of lanes whose pairs end at or before p
-#pragma unroll
-        for (int step = 32; step >= 1; step >>= 1) {
-            const int v = __shfl(incl, sl + step - 1, 64);
-            if (v <= p) sl += step;
-        }
+        own[lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+        if (mine > 0 && excl < r0 + 64 && incl > r0) own[max(excl - r0, 0)] = lane;
+        __builtin_amdgcn_wave_barrier();
+        const int sl = wave_incl_max(own[lane]);
+        __builtin_amdgcn_wave_barrier();
         const int k = p - __shfl(excl, sl, 64);
-        const int nc = __shfl(ncols, sl, 64), px0 = __shfl(tx0, sl, 64), py0 = __shfl(ty0, sl, 64);
-        const int tp = __shfl(t, sl, 64);
+        const unsigned f = __shfl(first, sl, 64);
         unsigned key = (kNoTile << 6) | (unsigned)lane;  // unique: the sorted lanes are a permutation
         if (active) {
-            const int ty = py0 + k / nc, tx = px0 + k % nc;
+            const int nc = (int)(f >> 22);
+            // k / nc, both at most 64: the quotient is at least 1 / 128 off an integer
+            const int dy = (int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)nc));
+            const int ty = (int)((f >> 11) & 2047) + dy, tx = (int)(f & 2047) + k - dy * nc;
             key = ((unsigned)(ty * d.tiles_x + tx) << 6) | (unsigned)lane;
         }
         const unsigned sk = wave_sort(key);
@@ -222,7 +231,7 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
         int base = 0;
         if (head) base = atomicAdd(&bin_count[d.tile_off + tl], e - lane);
         base = __shfl(base, h, 64);
-        const int tsrc = __shfl(tp, src, 64);
+        const int tsrc = t_wave + __shfl(sl, src, 64);
         bool full = false;
         if (valid) {
             const int slot = base + (lane - h);

@@ -137,6 +137,22 @@ __device__ __forceinline__ int wave_incl_scan(int x) {
     return scan_step<kDppBcast31, 0xc>(x);  // rows 2 and 3 add lane 31
 }
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int max_step(int x) {  // lanes without a source keep theirs (x >= 0)
+    const int y = __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+    return x > y ? x : y;
+}
+
+// largest of the non-negative values of lanes 0 .. this one
+__device__ __forceinline__ int wave_incl_max(int x) {
+    x = max_step<kDppShr1, 0xf>(x);
+    x = max_step<kDppShr2, 0xf>(x);
+    x = max_step<kDppShr4, 0xf>(x);
+    x = max_step<kDppShr8, 0xf>(x);
+    x = max_step<kDppBcast15, 0xa>(x);
+    return max_step<kDppBcast31, 0xc>(x);
+}
+
 // exclusive scan over a block of NT threads; wsum: NT / 64 words of LDS that
 // nothing else uses between this call and the block's next barrier
 template <int NT>
