@@ -572,11 +572,9 @@ __global__ void __launch_bounds__(256, 8) k_aa_fwd(AALaunch L) {
     __shared__ unsigned long long s_mask[2 * kAAH];
     __shared__ int q_n;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // one row of blocks, padded to a multiple of 8; XCD k takes the k-th eighth
-    // of them, whole images in a uniform batch (their vertices and flags stay
-    // in its L2, and a block's upper neighbour follows soon there)
+    // one row of blocks, dealt to the XCDs in groups of neighbours
     AABlock B;
-    if (!aa_block(L, xcd_remap(blockIdx.x, gridDim.x), B)) return;  // uniform per block
+    if (!aa_block(L, xcd_deal(blockIdx.x, L.xcd), B)) return;  // uniform per block
     const AAImg I = aa_img(L, B.img);
     const int H = I.H, W = I.W;
     const int c = B.c0 + lane;
@@ -820,7 +818,7 @@ __global__ void __launch_bounds__(256, 8) k_aa_bwd(AALaunch L) {
     __shared__ unsigned short s_slot[2 * kAAW * kAAH];  // pair slot of each list entry
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     AABlock B;
-    if (!aa_block(L, xcd_remap(blockIdx.x, gridDim.x), B)) return;  // uniform per block
+    if (!aa_block(L, xcd_deal(blockIdx.x, L.xcd), B)) return;  // uniform per block
     const AAImg I = aa_img(L, B.img);
     AASweep<CV> sweep(L, B, I.W);
     sweep.load(B, I.H, I.W, L.grad_out, 0);
@@ -914,12 +912,22 @@ static long long aa_blocks(const AALaunch &L) {
                   : (long long)((L.W + kAAW - 1) / kAAW) * ((L.H + kAAH - 1) / kAAH) * L.n_img;
 }
 
-static int launch_pairs(const AALaunch &L, hipStream_t st) {
+// blocks per XCD turn; the grid they make
+static AALaunch with_groups(const AALaunch &L0, dim3 &grid) {
+    AALaunch L = L0;
     const long long nblk = aa_blocks(L);
+    L.xcd = xcd_group(nblk, L.um.n ? 1 : L.n_img, kXcdPixels);
+    grid = dim3((unsigned)xcd_pad(nblk, L.xcd));
+    return L;
+}
+
+static int launch_pairs(const AALaunch &L0, hipStream_t st) {
+    const long long nblk = aa_blocks(L0);
     if (nblk == 0) return 0;
-    if (nblk >= (1ll << 31) - 8) return -1;
-    if (!L.prepared) launch_orient(L, st);
-    const dim3 grid((unsigned)((nblk + 7) & ~7ll));
+    if (nblk >= (1ll << 31) - 8 * kXcdPixels) return -1;
+    if (!L0.prepared) launch_orient(L0, st);
+    dim3 grid;
+    const AALaunch L = with_groups(L0, grid);
     DRP_AA_DISPATCH(k_aa_fwd)
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
@@ -934,15 +942,16 @@ int launch_antialias_prepare(const AALaunch &L, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_antialias_bwd(const AALaunch &L, hipStream_t st) {
-    const long long nblk = aa_blocks(L);
+int launch_antialias_bwd(const AALaunch &L0, hipStream_t st) {
+    const long long nblk = aa_blocks(L0);
     if (nblk == 0) return 0;
-    if (nblk >= (1ll << 31) - 8) return -1;
+    if (nblk >= (1ll << 31) - 8 * kXcdPixels) return -1;
     // without the forward's state the pairs are evaluated again, for their list alone
-    if (!L.reuse) {
-        if (int rc = launch_pairs(L, st)) return rc;
+    if (!L0.reuse) {
+        if (int rc = launch_pairs(L0, st)) return rc;
     }
-    const dim3 grid((unsigned)((nblk + 7) & ~7ll));
+    dim3 grid;
+    const AALaunch L = with_groups(L0, grid);
     DRP_AA_DISPATCH(k_aa_bwd)
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -12,14 +12,14 @@ struct AttrGather {
     int groups, F, V, nc;
     int ldc, c0;           // channels of grad_attr's rows, first channel of this pass
     int per_output;        // one group per output (else every group sums into output 0)
-    int lanes;
+    int lanes, xcd;        // lanes per (vertex, quad), blocks per XCD turn
     const int *inc_off, *inc;
     float *grad_attr;
 };
 struct PosGather {
     const float4 *partial;  // [n_img, 3 F]
     const unsigned char *live;  // [n_img, F]
-    int n_img, F, V, pos_batched;
+    int n_img, F, V, pos_batched, xcd;
     const int *inc_off, *inc;
     float4 *grad_pos;
 };
@@ -171,16 +171,15 @@ __device__ __forceinline__ void gather_pos(const PosGather &G, int blk, int oimg
     *o = make_float4(cur.x + s.x, cur.y + s.y, cur.z + s.z, cur.w + s.w);
 }
 
-// Grids are padded to a multiple of 8 blocks (x): XCD k takes the k-th eighth of
-// the vertices, whose corners' rows share cache lines.
+// Neighbouring vertices, whose corners' rows share cache lines, on one XCD.
 __global__ void __launch_bounds__(256) k_gather_attr_q(AttrGather A) {
-    gather_attr_q(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
+    gather_attr_q(A, xcd_deal(blockIdx.x, A.xcd), blockIdx.y);
 }
 __global__ void __launch_bounds__(256) k_gather_attr_c(AttrGather A) {
-    gather_attr_c(A, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
+    gather_attr_c(A, xcd_deal(blockIdx.x, A.xcd), blockIdx.y);
 }
 __global__ void __launch_bounds__(256) k_gather_pos(PosGather G) {
-    gather_pos(G, xcd_remap(blockIdx.x, gridDim.x), blockIdx.y);
+    gather_pos(G, xcd_deal(blockIdx.x, G.xcd), blockIdx.y);
 }
 
 // Both gathers of the fused backward (one attribute output), the first
@@ -191,31 +190,40 @@ template <bool QUADS>
 __global__ void __launch_bounds__(256) k_gather_both(AttrGather A, PosGather G, int attr_blocks, int pos_blocks) {
     const int blk = blockIdx.x;
     if (blk < attr_blocks) {
-        if (QUADS) gather_attr_q(A, xcd_remap(blk, attr_blocks), 0);
-        else gather_attr_c(A, xcd_remap(blk, attr_blocks), 0);
+        if (QUADS) gather_attr_q(A, xcd_deal(blk, A.xcd), 0);
+        else gather_attr_c(A, xcd_deal(blk, A.xcd), 0);
         return;
     }
     const int p = blk - attr_blocks, img = p / pos_blocks;
-    gather_pos(G, xcd_remap(p - img * pos_blocks, pos_blocks), img);
+    gather_pos(G, xcd_deal(p - img * pos_blocks, G.xcd), img);
 }
 
+// n_img: images the gathered partials come from (1: an uneven batch)
 static AttrGather attr_gather(const float *partial, const unsigned char *live, int groups, int F, int V, int C,
-                              int ldc, int c0, int per_output, const int *inc_off, const int *inc, float *grad_attr) {
+                              int ldc, int c0, int per_output, const int *inc_off, const int *inc, float *grad_attr,
+                              int n_img, unsigned &blocks) {
     const int per_out = per_output ? 1 : groups;
     const int lanes = per_out >= kAttrLanes ? kAttrLanes : (per_out >= 2 ? 2 : 1);
-    return {partial, live, groups, F, V, C, ldc, c0, per_output, lanes, inc_off, inc, grad_attr};
+    const long long n = ((C % 4 == 0 ? (long long)V * (C / 4) * lanes : (long long)V * C) + 255) / 256;
+    const int xcd = xcd_group(n, n_img, kXcdVerts);
+    blocks = (unsigned)xcd_pad(n, xcd);
+    return {partial, live, groups, F, V, C, ldc, c0, per_output, lanes, xcd, inc_off, inc, grad_attr};
 }
-static unsigned blocks8(long long n) { return (unsigned)(((n + 255) / 256 + 7) & ~7ll); }
-static unsigned attr_blocks(const AttrGather &A) {
-    return blocks8(A.nc % 4 == 0 ? (long long)A.V * (A.nc / 4) * A.lanes : (long long)A.V * A.nc);
+static PosGather pos_gather(const float *partial, const unsigned char *live, int n_img, int F, int V, int pos_batched,
+                            const int *inc_off, const int *inc, float *grad_pos, unsigned &blocks) {
+    const long long n = (V + 255ll) / 256;
+    const int xcd = xcd_group(n, n_img, kXcdVerts);
+    blocks = (unsigned)xcd_pad(n, xcd);
+    return {(const float4 *)partial, live, n_img, F, V, pos_batched, xcd, inc_off, inc, (float4 *)grad_pos};
 }
 
 int launch_gather_attr(const float *partial, const unsigned char *live, int groups, int F, int V, int C, int ldc,
                        int c0, int outs, int per_output, const int *inc_off, const int *inc, float *grad_attr,
                        hipStream_t st) {
     if (V == 0) return 0;
-    const AttrGather A = attr_gather(partial, live, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr);
-    const dim3 grid(attr_blocks(A), outs);
+    unsigned blocks;
+    const AttrGather A = attr_gather(partial, live, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr, groups, blocks);
+    const dim3 grid(blocks, outs);
     if (C % 4 == 0) hipLaunchKernelGGL(k_gather_attr_q, grid, dim3(256), 0, st, A);
     else hipLaunchKernelGGL(k_gather_attr_c, grid, dim3(256), 0, st, A);
     return hipGetLastError() == hipSuccess ? 0 : -2;
@@ -224,8 +232,9 @@ int launch_gather_attr(const float *partial, const unsigned char *live, int grou
 int launch_gather_pos(const float *partial, const unsigned char *live, int n_img, int F, int V, int pos_batched,
                       const int *inc_off, const int *inc, float *grad_pos, hipStream_t st) {
     if (V == 0) return 0;
-    const PosGather G{(const float4 *)partial, live, n_img, F, V, pos_batched, inc_off, inc, (float4 *)grad_pos};
-    hipLaunchKernelGGL(k_gather_pos, dim3(blocks8(V), pos_batched ? n_img : 1), dim3(256), 0, st, G);
+    unsigned blocks;
+    const PosGather G = pos_gather(partial, live, n_img, F, V, pos_batched, inc_off, inc, grad_pos, blocks);
+    hipLaunchKernelGGL(k_gather_pos, dim3(blocks, pos_batched ? n_img : 1), dim3(256), 0, st, G);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -233,11 +242,9 @@ int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const i
                        float *grad_pos, hipStream_t st) {
     if (T.V == 0) return 0;
     const int groups = (T.n_img + T.views_per_block - 1) / T.views_per_block;
-    const AttrGather A =
-        attr_gather(T.partial, T.live, groups, T.F, T.V, C, C, 0, 0, inc_off, inc, grad_attr);
-    const PosGather G{(const float4 *)T.partial_pos, T.live_pos, T.n_img, T.F, T.V, T.b.pos_batched, inc_off, inc,
-                      (float4 *)grad_pos};
-    const unsigned na = attr_blocks(A), np = blocks8(T.V);
+    unsigned na, np;
+    const AttrGather A = attr_gather(T.partial, T.live, groups, T.F, T.V, C, C, 0, 0, inc_off, inc, grad_attr, T.n_img, na);
+    const PosGather G = pos_gather(T.partial_pos, T.live_pos, T.n_img, T.F, T.V, T.b.pos_batched, inc_off, inc, grad_pos, np);
     const unsigned long long blocks = na + (unsigned long long)np * (T.b.pos_batched ? T.n_img : 1);
     if (blocks >= (1ull << 31)) {  // past one launch's blocks
         if (int rc = launch_gather_attr(T.partial, T.live, groups, T.F, T.V, C, C, 0, 1, 0, inc_off, inc, grad_attr, st))

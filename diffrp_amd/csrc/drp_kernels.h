@@ -161,6 +161,7 @@ struct AALaunch {
     float boost;
     UnevenMap um;                // uneven batch (um.n > 0): n_img items, packed; pos / tri global
     int total_blk;               // uneven batch: blocks of all items
+    int xcd;                     // blocks per XCD turn (set at launch)
 };
 
 struct PartitionLaunch {
@@ -206,6 +207,7 @@ struct TriBwdLaunch {
     float *rec_v;
     int *box_slot;           // [boxes, kBoxSlots] record index of the box's first tiles (nullptr: search)
     int tiles_x, tiles_per_img, n_tiles, n_tiles_pad;
+    int xcd_tiles;           // tiles per XCD turn
     UnevenMap um;            // uneven batch (um.n > 0): tiles of all items, one group
     int local_ids;           // uneven batch: rast ids count from each item's first triangle (else global)
 };

@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256, (reduce_waves<MODE, C, DB>())) k_tile_red
     __shared__ unsigned char rank[kBTP];  // sorted place of each pixel's key
     __shared__ double spx[kBT], spy[kBT]; // NDC centres of the tile's columns and rows (position chain)
     const int tid = threadIdx.x;
-    const int tile = xcd_remap(blockIdx.x, L.n_tiles_pad);
+    const int tile = xcd_deal(blockIdx.x, L.xcd_tiles);
     if (tile >= L.n_tiles) return;  // uniform per block
     // the tile's image: arithmetic for a uniform batch, the item map for an uneven one
     int img, lt, H = L.H, W = L.W, tiles_x = L.tiles_x;
@@ -632,11 +632,10 @@ template <int MODE, int C>
 constexpr int gather_waves() { return tile_nv<MODE, C>() <= 16 ? 6 : (tile_nv<MODE, C>() <= 40 ? 4 : 3); }
 
 template <int MODE, int C>
-__global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(TriBwdLaunch L) {
+__global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(TriBwdLaunch L, int xcd) {
     constexpr int NV = tile_nv<MODE, C>();
-    // XCD k takes the k-th eighth of the (group, block) grid (its width a
-    // multiple of 8): neighbouring triangles share their tiles' record lines
-    const int lin = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    // neighbouring triangles, which share their tiles' record lines, on one XCD
+    const int lin = xcd_deal(blockIdx.x + gridDim.x * blockIdx.y, xcd);
     const int grp = lin / gridDim.x;
     const int t = (lin - grp * (int)gridDim.x) * blockDim.x + threadIdx.x;
     if (t >= L.F) return;
@@ -669,9 +668,6 @@ __global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(
     }
 }
 
-// blocks per group of the tile gather: a multiple of 8 (xcd_remap)
-inline unsigned gather_width(int F) { return (unsigned)((((F + 255) / 256) + 7) & ~7); }
-
 template <int MODE, int C, bool DB>
 inline void launch_tiles(const TriBwdLaunch &L, hipStream_t st) {
     const dim3 grid((unsigned)L.n_tiles_pad);
@@ -680,7 +676,9 @@ inline void launch_tiles(const TriBwdLaunch &L, hipStream_t st) {
     else
         hipLaunchKernelGGL((k_tile_reduce<MODE, C, DB, unsigned long long>), grid, dim3(kBTP), 0, st, L);
     const int groups = (L.n_img + L.views_per_block - 1) / L.views_per_block;
-    hipLaunchKernelGGL((k_tile_gather<MODE, C>), dim3(gather_width(L.F), groups), dim3(256), 0, st, L);
+    const long long blocks = (L.F + 255ll) / 256, width = L.um.n || L.n_img < 8 ? xcd_pad(blocks, kXcdVerts) : xcd_pad(blocks, 1);
+    hipLaunchKernelGGL((k_tile_gather<MODE, C>), dim3((unsigned)width, groups), dim3(256), 0, st, L,
+                       xcd_group(width * groups, L.um.n ? 1 : L.n_img, kXcdVerts));
 }
 
 }  // namespace drp

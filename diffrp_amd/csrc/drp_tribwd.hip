@@ -30,7 +30,8 @@ size_t tile_records_bytes(int n_img, int H, int W, int nv, long long n_boxes) {
 
 void tile_records_layout_tiles(TriBwdLaunch &T, void *ws, long long n_tiles, long long n_boxes) {
     T.n_tiles = (int)n_tiles;
-    T.n_tiles_pad = (T.n_tiles + 7) & ~7;
+    T.xcd_tiles = xcd_group(n_tiles, T.um.n ? 1 : T.n_img, kXcdPixels);
+    T.n_tiles_pad = (int)xcd_pad(n_tiles, T.xcd_tiles);
     char *b = (char *)ws;
     T.rec_count = (int *)b;
     b += a256((size_t)n_tiles * 4);
