@@ -134,7 +134,8 @@ __global__ void __launch_bounds__(256) k_sample2d_fwd(const float *__restrict__ 
                                                       const float *__restrict__ uv, long long n, int wrap, int mode,
                                                       float *__restrict__ out) {
     const int Cn = CV > 0 ? CV : C;
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // (neighbouring samples share texels: runs of blocks on one XCD)
+    long long i = (long long)xcd_deal(blockIdx.x, kXcdPixels) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const bool raw = mode == kModeBicubic;
     const TexAxis ax = make_axis(uv[2 * i], W, wrap, false, raw), ay = make_axis(uv[2 * i + 1], H, wrap, true, raw);
@@ -179,6 +180,21 @@ __global__ void __launch_bounds__(256) k_sample2d_fwd(const float *__restrict__ 
         const int x = x0 + (k & 1), y = y0 + (k >> 1);
         in[k] = x >= 0 && x < ax.size && y >= 0 && y < ay.size;
         off[k] = in[k] ? ((long long)texel(ay, y) * W + texel(ax, x)) * Cn : 0;
+    }
+    if (CV > 0) {  // the four texels' loads in flight together (outside: texel 0, not used)
+        float t[4][CV > 0 ? CV : 1];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int c = 0; c < CV; ++c) t[k][c] = tex[off[k] + c];
+#pragma unroll
+        for (int c = 0; c < CV; ++c) {
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s = in[k] ? s + t[k][c] * w[k] : s;
+            o[c] = s;
+        }
+        return;
     }
     for (int c = 0; c < Cn; ++c) {
         float s = 0.f;
@@ -295,12 +311,13 @@ __global__ void __launch_bounds__(256) k_sample2d_bwd(const float *__restrict__ 
     __shared__ int box[4];  // min x, min y, max x, max y
     const int Cn = CV > 0 ? CV : C;
     const int tid = threadIdx.x;
-    long long i = (long long)blockIdx.x * blockDim.x + tid;
+    const long long blk = xcd_deal(blockIdx.x, kXcdPixels);  // neighbouring samples share texels
+    long long i = blk * blockDim.x + tid;
     bool live = i < n;
     if (width > 0) {  // 16 x 16 samples of an image (rows of all images counted on)
         const int tiles_x = (width + 15) / 16;
-        const long long ty = blockIdx.x / tiles_x;
-        const int col = (int)(blockIdx.x - ty * tiles_x) * 16 + (tid & 15);
+        const long long ty = blk / tiles_x;
+        const int col = (int)(blk - ty * tiles_x) * 16 + (tid & 15);
         i = (ty * 16 + (tid >> 4)) * width + col;
         live = col < width && i < n;
     }
@@ -311,7 +328,26 @@ __global__ void __launch_bounds__(256) k_sample2d_bwd(const float *__restrict__ 
     const float *g = gout + il * Cn;
     if (guv && live) {
         float gx = 0.f, gy = 0.f;
-        if (MODE != kModeNearest) {
+        if (MODE == kModeBilinear && CV > 0) {  // the texels' and gradients' loads in flight together
+            float t[ty.N * tx.N][CV > 0 ? CV : 1], gr[CV > 0 ? CV : 1];
+#pragma unroll
+            for (int k = 0; k < ty.N * tx.N; ++k)
+#pragma unroll
+                for (int c = 0; c < CV; ++c)
+                    t[k][c] = tex[((long long)max(ty.at[k / tx.N], 0) * W + max(tx.at[k % tx.N], 0)) * Cn + c];
+#pragma unroll
+            for (int c = 0; c < CV; ++c) gr[c] = g[c];
+#pragma unroll
+            for (int k = 0; k < ty.N * tx.N; ++k) {
+                const int a = k / tx.N, b = k % tx.N;
+                if (ty.at[a] < 0 || tx.at[b] < 0) continue;
+                float dot = 0.f;
+#pragma unroll
+                for (int c = 0; c < CV; ++c) dot += t[k][c] * gr[c];
+                gx += tx.dw[b] * ty.w[a] * dot;
+                gy += tx.w[b] * ty.dw[a] * dot;
+            }
+        } else if (MODE != kModeNearest) {
 #pragma unroll
             for (int a = 0; a < ty.N; ++a)
 #pragma unroll
@@ -478,7 +514,7 @@ __global__ void __launch_bounds__(256) k_sample3d_bwd(const float *__restrict__ 
 int launch_sample2d(const float *tex, int H, int W, int C, const float *uv, long long n, int wrap, int mode,
                     float *out, hipStream_t st) {
     if (n == 0) return 0;
-    dim3 grid((unsigned)((n + 255) / 256));
+    dim3 grid((unsigned)xcd_pad((n + 255) / 256, kXcdPixels));
     DRP_TEX_DISPATCH(k_sample2d_fwd, tex, H, W, C, uv, n, wrap, mode, out)
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
@@ -489,8 +525,8 @@ int launch_sample2d_bwd(const float *tex, int H, int W, int C, const float *uv, 
     long long blocks = (n + 255) / 256;
     if (width < 16) width = 0;  // narrower rows leave most of a 16 x 16 block idle
     else blocks = (long long)((width + 15) / 16) * (((n + width - 1) / width + 15) / 16);
-    if (blocks >= (1ll << 31)) return -1;
-    dim3 grid((unsigned)blocks);
+    if (blocks >= (1ll << 31) - 8 * kXcdPixels) return -1;
+    dim3 grid((unsigned)xcd_pad(blocks, kXcdPixels));
     if (mode == kModeBicubic) DRP_TEX_DISPATCH_M(kModeBicubic, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
     else if (mode == kModeNearest) DRP_TEX_DISPATCH_M(kModeNearest, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
     else DRP_TEX_DISPATCH_M(kModeBilinear, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
