@@ -182,6 +182,64 @@ __global__ void __launch_bounds__(256) k_gather_pos(PosGather G) {
     gather_pos(G, xcd_deal(blockIdx.x, G.xcd), blockIdx.y);
 }
 
+// Both gathers for one image of a large mesh: a thread per vertex reads its
+// corners and their triangles' bytes once for the position and all NQ quads, and
+// leaves a vertex without a live corner alone.  With a lane per quad those reads
+// are most of the work: 262 -> 149 us for 2.6M vertices of 16 channels.  Below
+// kVertexThreads vertices the lanes are needed to fill the GPU.
+constexpr int kVertexThreads = 1 << 18;
+template <int NQ>
+__global__ void __launch_bounds__(256) k_gather_vertex(AttrGather A, PosGather G) {
+    const int v = xcd_deal(blockIdx.x, G.xcd) * (int)blockDim.x + (int)threadIdx.x;
+    if (v >= G.V) return;
+    const int i0 = G.inc_off[v], i1 = G.inc_off[v + 1];
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f), acc[NQ];
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = i0; i < i1; i += 8) {
+        int c[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) c[k] = i + k < i1 ? G.inc[i + k] : -1;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (c[k] >= 0 && !G.live[(unsigned)c[k] / 3u]) c[k] = -1;
+        float4 x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (c[k] >= 0) {
+                x[k] = G.partial[c[k]];
+                any = true;
+            }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (c[k] >= 0) { s.x += x[k].x; s.y += x[k].y; s.z += x[k].z; s.w += x[k].w; }
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (c[k] >= 0) x[k] = reinterpret_cast<const float4 *>(A.partial)[(long long)c[k] * NQ + q];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (c[k] >= 0) {
+                    acc[q].x += x[k].x; acc[q].y += x[k].y; acc[q].z += x[k].z; acc[q].w += x[k].w;
+                }
+        }
+    }
+    if (!any) return;
+    float4 *o = G.grad_pos + v;
+    const float4 cur = *o;
+    *o = make_float4(cur.x + s.x, cur.y + s.y, cur.z + s.z, cur.w + s.w);
+    float *ga = A.grad_attr + (long long)v * (4 * NQ);  // (may lack 16-byte alignment)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        ga[4 * q] += acc[q].x;
+        ga[4 * q + 1] += acc[q].y;
+        ga[4 * q + 2] += acc[q].z;
+        ga[4 * q + 3] += acc[q].w;
+    }
+}
+
 // Both gathers of the fused backward (one attribute output), the first
 // `attr_blocks` blocks for the attributes.  They are independent and each too
 // small to fill the GPU on an ordinary mesh; as two launches they needed a second
@@ -245,6 +303,16 @@ int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const i
     unsigned na, np;
     const AttrGather A = attr_gather(T.partial, T.live, groups, T.F, T.V, C, C, 0, 0, inc_off, inc, grad_attr, T.n_img, na);
     const PosGather G = pos_gather(T.partial_pos, T.live_pos, T.n_img, T.F, T.V, T.b.pos_batched, inc_off, inc, grad_pos, np);
+    if (C % 4 == 0 && T.n_img == 1 && T.V >= kVertexThreads) {
+        const dim3 grid(np);
+        switch (C / 4) {
+            case 1: hipLaunchKernelGGL((k_gather_vertex<1>), grid, dim3(256), 0, st, A, G); break;
+            case 2: hipLaunchKernelGGL((k_gather_vertex<2>), grid, dim3(256), 0, st, A, G); break;
+            case 3: hipLaunchKernelGGL((k_gather_vertex<3>), grid, dim3(256), 0, st, A, G); break;
+            default: hipLaunchKernelGGL((k_gather_vertex<4>), grid, dim3(256), 0, st, A, G); break;
+        }
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    }
     const unsigned long long blocks = na + (unsigned long long)np * (T.b.pos_batched ? T.n_img : 1);
     if (blocks >= (1ull << 31)) {  // past one launch's blocks
         if (int rc = launch_gather_attr(T.partial, T.live, groups, T.F, T.V, C, C, 0, 1, 0, inc_off, inc, grad_attr, st))
