@@ -51,6 +51,9 @@ _SIGS = {
     'drp_batch_interpolate_rasterize_bwd': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_size]),
+    'drp_batch_interpolate_rasterize_bwd_to': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
+                                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                    c_void_p, c_void_p, c_void_p, c_size, c_int]),
     'drp_batch_rasterize_bwd_workspace_size': (c_size, [c_void_p]),
     'drp_batch_rasterize_bwd': (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -90,6 +93,9 @@ _SIGS = {
     'drp_interpolate_rasterize_bwd': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int,
                                               c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                                               c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_size]),
+    'drp_interpolate_rasterize_bwd_to': (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int,
+                                              c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                              c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_size, c_int]),
     'drp_edge_grad_bwd': (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
                                   c_int, c_void_p]),
     'drp_topology_workspace_size': (c_size, [c_int]),

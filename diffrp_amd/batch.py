@@ -404,21 +404,23 @@ class _UInterpolate(torch.autograd.Function):
         ub = fctx.ub
         C = attr.shape[1]
         gout = nvdr._as_f32(gout, 'grad_out')
-        gattr = torch.zeros_like(attr)
         L = _lib.lib()
         if src_pos is not None and fctx.needs_input_grad[4]:
             # the rasterize backward of this interpolation's grad_rast in the same
             # pass, returned as the gradient of the rasterised positions (the
             # rasterize backward, linear in grad_rast, sees only rast's other consumers)
-            gpos = torch.zeros_like(src_pos)
+            some = ub.plan.n_pix > 0 and ub.plan.n_tri > 0 and ub.plan.n_vert > 0
+            new = torch.empty_like if some else torch.zeros_like  # (written whole)
+            gattr, gpos = new(attr), new(src_pos)
             ws_bytes = L.drp_batch_interpolate_rasterize_bwd_workspace_size(ub.plan.host_ptr(), C)
             ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=attr.device)
-            check(L.drp_batch_interpolate_rasterize_bwd(stream_of(attr), ub.plan.host_ptr(), ptr(ub.plan.dev),
+            check(L.drp_batch_interpolate_rasterize_bwd_to(stream_of(attr), ub.plan.host_ptr(), ptr(ub.plan.dev),
                                                         ptr(attr), C, ptr(src_pos), ptr(rast), ptr(ub.tri),
                                                         ptr(gout), ptr(gattr), ptr(gpos), ptr(boxes),
-                                                        ptr(ub.inc[0]), ptr(ub.inc[1]), ptr(ws), ws_bytes),
+                                                        ptr(ub.inc[0]), ptr(ub.inc[1]), ptr(ws), ws_bytes, 3),
                   'batch interpolate + rasterize backward')
             return gattr, None, None, None, gpos
+        gattr = torch.zeros_like(attr)
         grast = torch.empty_like(rast)
         ws_bytes = L.drp_batch_interpolate_bwd_workspace_size(ub.plan.host_ptr(), C)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=attr.device)

@@ -605,11 +605,11 @@ size_t drp_batch_interpolate_rasterize_bwd_workspace_size(const void *plan, int 
            tile_records_bytes_tiles(tiles, tile_record_floats(pass_width(C), true, true), h.n_tri) + 2 * align256((size_t)h.n_tri);
 }
 
-int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr,
+int drp_batch_interpolate_rasterize_bwd_to(void *stream, const void *plan, const void *plan_dev, const float *attr,
                                         int C, const float *pos, const float *rast, const int32_t *tri,
                                         const float *grad_out, float *grad_attr, float *grad_pos,
                                         const int32_t *boxes, const int32_t *inc_off, const int32_t *inc,
-                                        void *workspace, size_t workspace_bytes) {
+                                        void *workspace, size_t workspace_bytes, int overwrite) {
     PlanView v;
     if (int e = plan_view(plan, plan_dev, v)) return e;
     if (C < 1 || C > kMaxPassChannels)
@@ -662,9 +662,17 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
     T.local_ids = 0;
     tile_records_layout_tiles(T, records, v.bt16, F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, st);
+    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, overwrite & 1, overwrite & 2, st);
     if (rc) return fail(rc, "batch fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
+}
+
+int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const void *plan_dev, const float *attr,
+                                        int C, const float *pos, const float *rast, const int32_t *tri,
+                                        const float *grad_out, float *grad_attr, float *grad_pos,
+                                        const int32_t *boxes, const int32_t *inc_off, const int32_t *inc,
+                                        void *workspace, size_t workspace_bytes) {
+    return drp_batch_interpolate_rasterize_bwd_to(stream, plan, plan_dev, attr, C, pos, rast, tri, grad_out, grad_attr, grad_pos, boxes, inc_off, inc, workspace, workspace_bytes, 0);
 }
 
 size_t drp_batch_rasterize_bwd_workspace_size(const void *plan) {
@@ -978,11 +986,11 @@ size_t drp_interpolate_rasterize_bwd_workspace_size(int n_img, int H, int W, int
            align256(groups * (size_t)F) + align256((size_t)n_img * (size_t)F);
 }
 
-int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
+int drp_interpolate_rasterize_bwd_to(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
                                   int W, const int32_t *tri, int F, const float *pos, int pos_batched,
                                   const float *grad_out, float *grad_attr, float *grad_rast, float *grad_pos,
                                   const int32_t *boxes, int views_per_group, const int32_t *inc_off,
-                                  const int32_t *inc, void *workspace, size_t workspace_bytes) {
+                                  const int32_t *inc, void *workspace, size_t workspace_bytes, int overwrite) {
     if (int e = check_dims(n_img, H, W)) return e;
     if (n_img == 0) return 0;
     if (C < 1 || C > kMaxPassChannels)
@@ -1034,9 +1042,17 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
     T.views_per_block = vpg;
     tile_records_layout(T, records, n_img, H, W, (long long)n_img * F);
     int rc = launch_tri_bwd_fused(T, C, st);
-    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, st);
+    if (!rc) rc = launch_gather_both(T, C, inc_off, inc, grad_attr, grad_pos, overwrite & 1, overwrite & 2, st);
     if (rc) return fail(rc, "fused backward launch failed: %s", hipGetErrorString(hipGetLastError()));
     return 0;
+}
+
+int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
+                                  int W, const int32_t *tri, int F, const float *pos, int pos_batched,
+                                  const float *grad_out, float *grad_attr, float *grad_rast, float *grad_pos,
+                                  const int32_t *boxes, int views_per_group, const int32_t *inc_off,
+                                  const int32_t *inc, void *workspace, size_t workspace_bytes) {
+    return drp_interpolate_rasterize_bwd_to(stream, attr, n_img, V, C, rast, H, W, tri, F, pos, pos_batched, grad_out, grad_attr, grad_rast, grad_pos, boxes, views_per_group, inc_off, inc, workspace, workspace_bytes, 0);
 }
 
 int drp_edge_grad_bwd(void *stream, const float *grad_out, const float *rgb, int H, int W, int C, const float *rast,

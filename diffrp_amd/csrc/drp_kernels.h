@@ -235,7 +235,7 @@ int launch_gather_pos(const float *partial, const unsigned char *live, int n_img
                       const int *inc_off, const int *inc, float *grad_pos, hipStream_t st);
 // both, after launch_tri_bwd_fused(T, C, ..)
 int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const int *inc, float *grad_attr,
-                       float *grad_pos, hipStream_t st);
+                       float *grad_pos, int set_attr, int set_pos, hipStream_t st);
 // floats of a tile record with the attribute and position sums
 int tile_record_floats(int C, bool attr, bool pos);
 // workspace of the tile records for nv floats per record and n_boxes pixel

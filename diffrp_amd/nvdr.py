@@ -506,7 +506,6 @@ class _InterpolateFunc(torch.autograd.Function):
         F = tri.shape[0]
         nd = fctx.nd
         dy = _as_f32(dy, 'grad_out')
-        gattr = torch.zeros_like(attr)
         L = _lib.lib()
         aa_gpos = _take_aa_pos(fctx)
         if src_pos is not None and fctx.needs_input_grad[6]:
@@ -514,16 +513,21 @@ class _InterpolateFunc(torch.autograd.Function):
             # pass, returned as the gradient of the rasterised positions; grad_rast
             # itself is neither written nor returned, so the rasterize backward
             # (linear in its grad_rast) sees only what rast's other consumers send
-            gpos = aa_gpos if aa_gpos is not None else torch.zeros_like(src_pos)  # (accumulated into)
+            # (attributes' and, without an antialias's share to add to, positions' gradients written whole)
+            new = torch.empty_like if n > 0 and V > 0 else torch.zeros_like
+            gattr = new(attr)
+            gpos = aa_gpos if aa_gpos is not None else new(src_pos)
             off, inc = incidence(tri, V)
             vpg = _views_per_group(n, F)
             ws_bytes = L.drp_interpolate_rasterize_bwd_workspace_size(n, H, W, F, C, vpg)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=attr.device)
-            rc = L.drp_interpolate_rasterize_bwd(stream_of(attr), ptr(attr), n, V, C, ptr(rast), H, W, ptr(tri), F,
+            rc = L.drp_interpolate_rasterize_bwd_to(stream_of(attr), ptr(attr), n, V, C, ptr(rast), H, W, ptr(tri), F,
                                                  ptr(src_pos), int(src_pos.dim() == 3), ptr(dy), ptr(gattr), None,
-                                                 ptr(gpos), ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws_bytes)
+                                                 ptr(gpos), ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws_bytes,
+                                                    1 if aa_gpos is not None else 3)
             check(rc, 'interpolate + rasterize backward')
             return gattr, None, None, None, None, None, gpos
+        gattr = torch.zeros_like(attr)
         grast = torch.empty_like(rast)
         gdb = torch.empty_like(rast) if nd else None
         dda = _as_f32(dda, 'grad_da') if (nd and dda is not None) else None

@@ -158,6 +158,14 @@ int drp_batch_interpolate_rasterize_bwd(void *stream, const void *plan, const vo
                                         const float *grad_out, float *grad_attr, float *grad_pos,
                                         const int32_t *boxes, const int32_t *inc_off, const int32_t *inc,
                                         void *workspace, size_t workspace_bytes);
+/* The same; overwrite bit 0: grad_attr, bit 1: grad_pos is written whole instead
+ * of accumulated into (no zero-fill before).  Nothing is written when the batch
+ * has no pixel, triangle or vertex. */
+int drp_batch_interpolate_rasterize_bwd_to(void *stream, const void *plan, const void *plan_dev, const float *attr,
+                                        int C, const float *pos, const float *rast, const int32_t *tri,
+                                        const float *grad_out, float *grad_attr, float *grad_pos,
+                                        const int32_t *boxes, const int32_t *inc_off, const int32_t *inc,
+                                        void *workspace, size_t workspace_bytes, int overwrite);
 size_t drp_batch_antialias_workspace_size(const void *plan);
 int drp_batch_antialias_fwd(void *stream, const void *plan, const void *plan_dev, const float *color, int C,
                             const float *rast, const float *pos, const int32_t *tri, const int32_t *opp, float *out,
@@ -298,6 +306,13 @@ int drp_interpolate_rasterize_bwd(void *stream, const float *attr, int n_img, in
                                   const float *grad_out, float *grad_attr, float *grad_rast, float *grad_pos,
                                   const int32_t *boxes, int views_per_group, const int32_t *inc_off,
                                   const int32_t *inc, void *workspace, size_t workspace_bytes);
+/* The same; overwrite bit 0: grad_attr, bit 1: grad_pos is written whole instead
+ * of accumulated into (no zero-fill before).  Nothing is written when n_img is 0. */
+int drp_interpolate_rasterize_bwd_to(void *stream, const float *attr, int n_img, int V, int C, const float *rast, int H,
+                                  int W, const int32_t *tri, int F, const float *pos, int pos_batched,
+                                  const float *grad_out, float *grad_attr, float *grad_rast, float *grad_pos,
+                                  const int32_t *boxes, int views_per_group, const int32_t *inc_off,
+                                  const int32_t *inc, void *workspace, size_t workspace_bytes, int overwrite);
 
 /* ---- antialias -----------------------------------------------------------
  * Topology table for antialias: replaces dr.antialias_construct_topology_hash

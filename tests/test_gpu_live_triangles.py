@@ -63,3 +63,37 @@ def test_gradients_with_hidden_triangles(cuda, n, views, C):
     op = oracle.rasterize_bwd(pos.numpy(), tri.numpy(), r, orr)
     _close(ga, oa, 1e-5, 'grad attr')
     _close(gp, op, 1e-4, 'grad pos')
+
+
+@pytest.mark.parametrize('views', [1, 9])
+@pytest.mark.parametrize('C', [3, 8])
+def test_accumulating_and_overwriting_calls(cuda, views, C):
+    """The fused call adds to the gradients given; its overwriting form replaces them."""
+    from diffrp_amd import _lib
+    from diffrp_amd._lib import check, ptr, stream_of
+    pos, tri, g = _cones(40, views)
+    H, W = 45, 70
+    V, F = pos.shape[1], tri.shape[0]
+    p, t = pos.cuda().requires_grad_(True), tri.cuda()
+    a, go = torch.rand(V, C, generator=g).cuda(), torch.randn(views, H, W, C, generator=g).cuda()
+    rast, _ = nvdr.rasterize(nvdr.RasterizeCudaContext(), p, t, (H, W), grad_db=False)
+    boxes, (off, inc), r, p = rast._drp_boxes[0], nvdr.incidence(t, V), rast.detach(), p.detach()
+    L, vpg = _lib.lib(), nvdr._views_per_group(views, F)
+    ws = torch.empty(L.drp_interpolate_rasterize_bwd_workspace_size(views, H, W, F, C, vpg), dtype=torch.uint8, device='cuda')
+
+    def call(ga, gp, overwrite):
+        args = [stream_of(a), ptr(a), views, V, C, ptr(r), H, W, ptr(t), F, ptr(p), 1, ptr(go), ptr(ga), None, ptr(gp),
+                ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws.numel()]
+        if overwrite is None:
+            check(L.drp_interpolate_rasterize_bwd(*args), 'add')
+        else:
+            check(L.drp_interpolate_rasterize_bwd_to(*args, overwrite), 'to')
+        return ga, gp
+    z, one = call(torch.zeros_like(a), torch.zeros_like(p), None), (torch.ones_like(a), torch.ones_like(p))
+    nan = (torch.full_like(a, float('nan')), torch.full_like(p, float('nan')))
+    assert z[0].abs().sum() > 0 and z[1].abs().sum() > 0
+    for overwrite in (None, 0, 1, 2, 3):
+        bits = overwrite or 0
+        ga, gp = call((nan if bits & 1 else one)[0].clone(), (nan if bits & 2 else one)[1].clone(), overwrite)
+        assert torch.equal(ga, z[0] if bits & 1 else z[0] + 1)
+        assert torch.equal(gp, z[1] if bits & 2 else z[1] + 1)
