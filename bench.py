@@ -242,12 +242,11 @@ STEP_OPS = ('rasterize_fwd', 'interpolate_fwd', 'antialias_fwd', 'antialias_bwd'
 OP_KERNELS = {
     'rasterize_fwd': ['k_zero_i32', 'k_setup_bin', 'k_fine', 'k_fine_split'],
     'interpolate_fwd': ['k_interp_fwd'],
-    'antialias_fwd': ['k_aa_project', 'k_aa_orient', 'k_aa_silhouette', 'k_aa_pairs', 'k_aa_gather'],
-    'antialias_bwd': ['k_aa_pairs_bwd', 'k_aa_gather_bwd'],
-    'interpolate_bwd': ['k_tile_reduce<1,C>', 'k_tile_gather<1,C>', 'k_gather_attr'],
+    'antialias_fwd': ['k_aa_orient', 'k_aa_silhouette', 'k_aa_fwd'],
+    'antialias_bwd': ['k_aa_bwd'],
+    'interpolate_bwd': ['k_tile_reduce<1,C>', 'k_tile_gather<1,C>', 'k_gather_attr_q'],
     'rasterize_bwd': ['k_tile_reduce<0>', 'k_tile_gather<0>', 'k_gather_pos'],
-    'interpolate_rasterize_bwd': ['k_corner_slots_clear', 'k_corner_slots', 'k_tile_reduce<2,C>',
-                                  'k_tile_gather<2,C>', 'k_gather_attr', 'k_gather_pos'],
+    'interpolate_rasterize_bwd': ['k_tile_reduce<2,C>', 'k_tile_gather<2,C>', 'k_gather_both'],
 }
 
 TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'profiles', 'traffic_64view_512.txt')

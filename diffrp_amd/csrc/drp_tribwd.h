@@ -11,15 +11,16 @@
 // rows and not 3 C / 4, and the products live in no register across the sort.
 // Tiles without a covered pixel leave before the sort.  64 views of 82k
 // triangles at 512^2, C = 8, both sums: 483 us with 36 staged terms per pixel,
-// 412 us so.  What remains is instruction issue: the sort, the double chain,
-// the sums.
+// 412 us so, 381 with the sums as FMAs and no z/w chain where none can arrive.
+// What remains is instruction issue: the sort, the double chain, the sums.
 //
 // k_tile_gather, one thread per (image [group], triangle) that won a pixel
 // in the forward: the triangle's pixel box names the tiles it touches; the
 // tile pass stored the record index of the box's first kBoxSlots tiles per
 // box, further tiles' records are binary-searched, and the thread adds them in
 // tile order.  All sums run in a fixed order, so results are reproducible bit
-// for bit.
+// for bit.  (Four lanes per triangle, to read a record in whole lines, repeat
+// that search per lane: 150 -> 259 us at 64 views.)
 //
 //   POS  (12 floats): d rast (u, v, z/w [, db]) -> d clip (x, y, z, w) of the 3
 //        corners (double-precision chain, drp_grad.h); partial [n, 3F] float4,
@@ -646,7 +647,9 @@ __global__ void __launch_bounds__(256, (gather_waves<MODE, C>())) k_tile_gather(
     const int v0 = grp * VB, v1 = min(v0 + VB, L.n_img);
     // Only triangles that won a pixel have sums: the others' partials are neither
     // written here nor read by the vertex gathers, which look at one byte each
-    // (half of a mesh faces away, and a dense one hides most of the rest).
+    // (half of a mesh faces away, and a dense one hides most of the rest): 64
+    // views of 82k triangles 255 -> 150 us, one view of 5.2M 920 -> 240 us with
+    // the triangles dealt to the XCDs.
     const bool hit = MODE == 2 ? gather_records_fused<rec_attr<MODE, C>()>(L, t, v0, v1, acc)
                                : gather_records<NV>(L, t, v0, v1, acc);
     const long long gt = (long long)grp * L.F + t;

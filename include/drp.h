@@ -360,8 +360,7 @@ int drp_antialias_fwd_prepared(void *stream, const float *color, int n_img, int 
  * zero-fills; may be null to skip), scaled by pos_gradient_boost.
  * reuse_forward != 0: the workspace still holds what drp_antialias_fwd left
  * there for the same rast, pos and tri (colour may differ), so the pair
- * search is not repeated (ignored for F >= 2^27 - 1, where the forward keeps
- * no pair decisions). */
+ * search is not repeated. */
 int drp_antialias_bwd(void *stream, const float *color, int n_img, int H, int W, int C, const float *rast,
                       const float *pos, int V, int pos_batched, const int32_t *tri, int F, const int32_t *opp,
                       const float *grad_out, float *grad_color, float *grad_pos, float pos_gradient_boost,
