@@ -294,9 +294,14 @@ __device__ __forceinline__ int xcd_deal(int bid, int group) {
 // images, or an uneven batch: an eighth may lie in an empty band of the image or
 // on the hidden side of the mesh, and its XCD idles (at one 2048^2 view of 5.2M
 // triangles the tile gather took 529 us in eighths and 240 us dealt), so short
-// runs are dealt: 32 blocks of pixels, 16 of vertices or triangles.
+// runs are dealt: 32 blocks of pixels, 16 of vertices or triangles, shorter ones
+// where an XCD would get fewer than four.
 constexpr int kXcdPixels = 32, kXcdVerts = 16;
-inline int xcd_group(long long blocks, int n_img, int few) { return n_img >= 8 ? (int)((blocks + 7) / 8) : few; }
+inline int xcd_group(long long blocks, int n_img, int few) {
+    if (n_img >= 8) return (int)((blocks + 7) / 8);
+    const long long turn = blocks / 32;
+    return turn < 1 ? 1 : (turn < few ? (int)turn : few);
+}
 inline long long xcd_pad(long long blocks, int group) {
     const long long unit = 8ll * group;
     return (blocks + unit - 1) / unit * unit;

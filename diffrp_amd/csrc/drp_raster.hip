@@ -30,7 +30,7 @@ constexpr int kListCount = 0x7fffffff;  // spill-list count's value bits; the to
 constexpr int kQueuePerLane = 2;  // fine raster: covered-pixel queue entries per lane and pass
 constexpr int kFineWavesPerEU = 6;  // occupancy target of k_fine (VGPR budget 512 / 6)
 constexpr int kMaxFineNT = 256;     // largest tile (pixels)
-constexpr int kFineXcdGroup = 16;   // fine raster: consecutive tiles per XCD turn when tiles are dealt
+constexpr int kFineXcdGroup = 64;   // fine raster: consecutive tiles per XCD turn when tiles are dealt
 
 __device__ __forceinline__ int2 pack_box(int c0, int c1, int r0, int r1) {
     return make_int2(c0 | (c1 << 16), r0 | (r1 << 16));
@@ -996,9 +996,11 @@ static void launch_fine_c(const RasterLaunch &L, hipStream_t st) {
     // Eight or more images of one size: each XCD takes one contiguous eighth of
     // the tiles (whole images, so its L2 holds one image's triangles and setup
     // records at a time).  Otherwise groups of kFineXcdGroup tiles are dealt
-    // round robin, so no XCD is left with the heavy images or the heavy band.
-    const bool eighths = L.b.descs == nullptr && L.b.n_img >= 8;
-    const int group = eighths ? max(1, (L.n_tiles + 7) / 8) : kFineXcdGroup;
+    // round robin, so no XCD is left with the heavy images or the heavy band:
+    // about a row of tiles, whose triangles' records and vertices the next tiles
+    // share (three views of 733 x 1019: 92 us in groups of 16, 72 in 64; one
+    // 2048^2 view of 5.2M triangles 724 and 687 us).
+    const int group = xcd_group(L.n_tiles, L.b.descs ? 1 : L.b.n_img, kFineXcdGroup);
     const long long unit = 8ll * group;
     const int pad = (int)((L.n_tiles + unit - 1) / unit * unit);
     hipLaunchKernelGGL((k_fine<TW, TH, PEEL, DB, CULL>), dim3(pad), dim3(TW * TH), 0, st, L.b, L.pos, L.tri,

@@ -679,9 +679,13 @@ inline void launch_tiles(const TriBwdLaunch &L, hipStream_t st) {
     else
         hipLaunchKernelGGL((k_tile_reduce<MODE, C, DB, unsigned long long>), grid, dim3(kBTP), 0, st, L);
     const int groups = (L.n_img + L.views_per_block - 1) / L.views_per_block;
-    const long long blocks = (L.F + 255ll) / 256, width = L.um.n || L.n_img < 8 ? xcd_pad(blocks, kXcdVerts) : xcd_pad(blocks, 1);
+    // a row of blocks per group of images, padded so that the turns divide all of them
+    const bool eighths = !L.um.n && L.n_img >= 8;
+    const long long blocks = (L.F + 255ll) / 256;
+    const int few = eighths ? 1 : xcd_group(blocks, 1, kXcdVerts);
+    const long long width = xcd_pad(blocks, few);
     hipLaunchKernelGGL((k_tile_gather<MODE, C>), dim3((unsigned)width, groups), dim3(256), 0, st, L,
-                       xcd_group(width * groups, L.um.n ? 1 : L.n_img, kXcdVerts));
+                       eighths ? (int)(width * groups / 8) : few);
 }
 
 }  // namespace drp
