@@ -423,10 +423,12 @@ __device__ __forceinline__ unsigned long long readlane64(unsigned long long v, i
            (unsigned)__builtin_amdgcn_readlane((int)v, lane);
 }
 
-// channel chunk handled by one thread: 4 (one float4) when C is a multiple of 4
+// channel chunk handled by one thread: 4 (one float4) when C is a multiple of 4.
+// CV > 0: compile-time channel count; 0: runtime; kAnyQuads: runtime, a multiple of 4
+constexpr int kAnyQuads = -4;
 template <int CV>
 struct AAChunk {
-    static constexpr int CH = (CV > 0 && CV % 4 == 0) ? 4 : 1;
+    static constexpr int CH = CV != 0 && CV % 4 == 0 ? 4 : 1;
 };
 
 template <int CH>
@@ -891,7 +893,9 @@ __global__ void __launch_bounds__(256, 8) k_aa_bwd(AALaunch L) {
         case 4: hipLaunchKernelGGL(KERNEL<4>, grid, dim3(256), 0, st, L); break;   \
         case 8: hipLaunchKernelGGL(KERNEL<8>, grid, dim3(256), 0, st, L); break;   \
         case 16: hipLaunchKernelGGL(KERNEL<16>, grid, dim3(256), 0, st, L); break; \
-        default: hipLaunchKernelGGL(KERNEL<0>, grid, dim3(256), 0, st, L); break;  \
+        default:                                                                   \
+            if (L.C % 4 == 0) hipLaunchKernelGGL(KERNEL<kAnyQuads>, grid, dim3(256), 0, st, L); \
+            else hipLaunchKernelGGL(KERNEL<0>, grid, dim3(256), 0, st, L);         \
     }
 
 static void launch_orient(const AALaunch &L, hipStream_t st) {
