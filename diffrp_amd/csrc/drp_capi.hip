@@ -762,7 +762,6 @@ static int batch_aa_common(AALaunch &L, const PlanView &v, const float *color, i
     L.V = (int)v.h.n_vert;
     L.F = (int)v.h.n_tri;
     L.pos_batched = 0;
-    L.cv = (C == 1 || C == 3 || C == 4 || C == 8 || C == 16) ? C : 0;
     aa_pointers(L, workspace, (size_t)v.h.n_vert, (size_t)v.h.n_tri, (size_t)v.h.n_pix);
     L.um = v.um;
     L.total_blk = (int)v.blk;
@@ -1291,7 +1290,6 @@ static int aa_common(AALaunch &L, void *stream, const float *color, int n_img, i
     L.V = V;
     L.F = F;
     L.pos_batched = pos_batched;
-    L.cv = (C == 1 || C == 3 || C == 4 || C == 8 || C == 16) ? C : 0;
     aa_layout(L, workspace, n_img, H, W, V, F, pos_batched);
     (void)stream;
     return 0;

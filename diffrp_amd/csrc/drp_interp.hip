@@ -33,7 +33,8 @@ __device__ __forceinline__ InterpPix interp_pix(const float4 *__restrict__ rast,
 // four consecutive lanes, so that a wave's loads of vertex rows and its stores
 // cover whole cache lines: one lane per pixel stored 16 bytes in every 64 at 16
 // channels, 81 us for 8 x 512^2, 35 us so.  At 8 channels two lanes are slower
-// than one (213 against 194 us for 64 x 512^2).
+// than one (213 against 194 us for 64 x 512^2).  Counts below 8 are compiled: the
+// rows of 5 channels then load in two accesses (3 x 733 x 1019: 29 -> 16 us).
 template <int CV, bool QUADS>
 constexpr int interp_lanes() { return !QUADS || CV == 4 || CV == 8 ? 1 : 4; }
 
@@ -191,7 +192,10 @@ int launch_interpolate(const InterpLaunch &L, hipStream_t st) {
         case 8: launch_fwd<8, true>(L, st); break;
         case 16: launch_fwd<16, true>(L, st); break;
         default:
-            if (L.C % 4 == 0 && aligned) launch_fwd<0, true>(L, st);
+            if (L.C == 5) launch_fwd<5, false>(L, st);
+            else if (L.C == 6) launch_fwd<6, false>(L, st);
+            else if (L.C == 7) launch_fwd<7, false>(L, st);
+            else if (L.C % 4 == 0 && aligned) launch_fwd<0, true>(L, st);
             else launch_fwd<0, false>(L, st);
     }
     return hipGetLastError() == hipSuccess ? 0 : -2;

@@ -146,7 +146,6 @@ struct AALaunch {
     const float *color, *rast, *pos;
     const int *tri, *opp;
     int n_img, H, W, C, V, F, pos_batched;
-    int cv;           // compiled channel variant (0 = generic loop)
     double2 *proj;               // [n_proj, V] pixel coordinates (NaN: w <= 0)
     signed char *orient;
     unsigned char *silh;

@@ -31,7 +31,7 @@ def _rel(a, b, rtol, what):
     assert err <= rtol, f'{what}: {err:.3e} > {rtol}'
 
 
-@pytest.mark.parametrize('C', [1, 3, 4, 5, 8, 12, 16])
+@pytest.mark.parametrize('C', [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 16])
 def test_blocks(cuda, C):
     pos, tri = random_soup(40, 3)
     pos2, _ = random_soup(40, 4)
