@@ -454,11 +454,11 @@ class SurfaceDeferredRenderSessionOptions:
 def _fill_value(default: Sequence[float], dev) -> torch.Tensor:
     """[C] of ``default`` on the device by fill kernels (copying it from host memory
     waits for the stream)."""
-    v = torch.full((len(default),), float(default[0]), dtype=torch.float32, device=dev) if default else \
-        torch.empty(0, dtype=torch.float32, device=dev)
-    for i, x in enumerate(default):
-        if x != default[0]:
-            v[i].fill_(float(x))
+    vals = [float(x) for x in default]
+    v = torch.full((len(vals),), vals[0] if vals else 0.0, dtype=torch.float32, device=dev)
+    for i, x in enumerate(vals):
+        if x != vals[0]:
+            v[i].fill_(x)
     return v
 
 
