@@ -11,9 +11,10 @@ import threading
 
 import torch
 
-from .build_ext import LIB_PATH
+from .build_ext import AUTOGRAD_LIB_PATH, LIB_PATH
 
 _lib = None
+_grad_observed = None
 _lock = threading.Lock()
 
 c_void_p = ctypes.c_void_p
@@ -142,6 +143,24 @@ def lib() -> ctypes.CDLL:
                     f.argtypes = args
                 _lib = L
     return _lib
+
+
+def grad_observed(fctx, i: int) -> bool:
+    """Within a Function's backward: whether anything besides the node that made
+    the i-th tensor argument sees the gradient returned for it -- a hook of the
+    tensor or of that node, ``retain_grad``, or the running pass, when it was
+    asked for that gradient (``torch.autograd.grad``, ``backward(inputs=...)``)."""
+    global _grad_observed
+    if _grad_observed is None:
+        with _lock:
+            if _grad_observed is None:
+                if not os.path.exists(AUTOGRAD_LIB_PATH):
+                    raise RuntimeError(f'{AUTOGRAD_LIB_PATH} is missing: build it with `python -m diffrp_amd.build_ext` '
+                                       '(or __graft_entry__.build())')
+                f = ctypes.PyDLL(AUTOGRAD_LIB_PATH).drp_grad_observed  # (keeps the interpreter lock)
+                f.restype, f.argtypes = c_int, [ctypes.py_object, c_int]
+                _grad_observed = f
+    return _grad_observed(fctx, i) != 0
 
 
 def check(rc: int, what: str):

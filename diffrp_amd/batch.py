@@ -39,7 +39,7 @@ import numpy as np
 import torch
 
 from . import _lib, nvdr
-from ._lib import check, ptr, stream_of, require_device
+from ._lib import check, grad_observed, ptr, require_device, stream_of
 
 _c_ll = ctypes.c_longlong
 
@@ -405,10 +405,11 @@ class _UInterpolate(torch.autograd.Function):
         C = attr.shape[1]
         gout = nvdr._as_f32(gout, 'grad_out')
         L = _lib.lib()
-        if src_pos is not None and fctx.needs_input_grad[4]:
+        if src_pos is not None and fctx.needs_input_grad[4] and not grad_observed(fctx, 1):
             # the rasterize backward of this interpolation's grad_rast in the same
             # pass, returned as the gradient of the rasterised positions (the
-            # rasterize backward, linear in grad_rast, sees only rast's other consumers)
+            # rasterize backward, linear in grad_rast, sees only rast's other consumers;
+            # where a hook or the caller sees rast's gradient, it goes through rast)
             some = ub.plan.n_pix > 0 and ub.plan.n_tri > 0 and ub.plan.n_vert > 0
             new = torch.empty_like if some else torch.zeros_like  # (written whole)
             gattr, gpos = new(attr), new(src_pos)

@@ -33,7 +33,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import ptr, check, stream_of, require_device
+from ._lib import ptr, check, grad_observed, stream_of, require_device
 
 __all__ = [
     'RasterizeCudaContext', 'RasterizeGLContext', 'RasterizeHipContext', 'DepthPeeler', 'rasterize',
@@ -508,11 +508,13 @@ class _InterpolateFunc(torch.autograd.Function):
         dy = _as_f32(dy, 'grad_out')
         L = _lib.lib()
         aa_gpos = _take_aa_pos(fctx)
-        if src_pos is not None and fctx.needs_input_grad[6]:
+        if src_pos is not None and fctx.needs_input_grad[6] and not grad_observed(fctx, 1):
             # the rasterize backward of this interpolation's grad_rast in the same
             # pass, returned as the gradient of the rasterised positions; grad_rast
             # itself is neither written nor returned, so the rasterize backward
-            # (linear in its grad_rast) sees only what rast's other consumers send
+            # (linear in its grad_rast) sees only what rast's other consumers send.
+            # (Where a hook or the caller sees rast's gradient, it is written and
+            # goes through rast.)
             # (attributes' and, without an antialias's share to add to, positions' gradients written whole)
             new = torch.empty_like if n > 0 and V > 0 else torch.zeros_like
             gattr = new(attr)
