@@ -454,10 +454,11 @@ class SurfaceDeferredRenderSessionOptions:
 def _fill_value(default: Sequence[float], dev) -> torch.Tensor:
     """[C] of ``default`` on the device by fill kernels (copying it from host memory
     waits for the stream)."""
-    vals = [float(x) for x in default]
+    host = torch.tensor([float(x) for x in default], dtype=torch.float32)  # (past float32's range: infinite)
+    vals, bits = host.tolist(), host.view(torch.int32).tolist()
     v = torch.full((len(vals),), vals[0] if vals else 0.0, dtype=torch.float32, device=dev)
     for i, x in enumerate(vals):
-        if x != vals[0]:
+        if bits[i] != bits[0]:  # (0.0 and -0.0 differ)
             v[i].fill_(x)
     return v
 
