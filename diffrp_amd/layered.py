@@ -120,9 +120,10 @@ def _compose(rgba, rast, out, trans):
             and rgba.device == rast.device and rast.is_contiguous()
             and (out is None or (out.dtype == torch.float32 and out.is_contiguous() and trans.is_contiguous()))
             and torch.autograd.forward_ad._current_level < 0):
-        # a slice of a wider buffer is copied out: what is kept for the backward must not hold the buffer
-        if (not rgba.is_contiguous() or rgba.data_ptr() % 16
-                or rgba.untyped_storage().nbytes() > 2 * rgba.numel() * rgba.element_size()):
+        # kept for the backward: a copy, as the operators keep (shade may write to its buffer again, and a
+        # slice would hold the whole of a wider one)
+        kept = torch.is_grad_enabled() and (rgba.requires_grad or (trans is not None and trans.requires_grad))
+        if kept or not rgba.is_contiguous() or rgba.data_ptr() % 16:
             rgba = rgba.clone(memory_format=torch.contiguous_format)
         return _Compose.apply(rgba, rast, out, trans)
     return _blend(rgba, rast, out, trans)
