@@ -130,7 +130,9 @@ class MaskedSparseInterpolator:
         self.run = run
         if run is not None:  # an owner's run of a partitioned layer
             self.indices = run.indices()
-            self.vi_data = run.layer.frag[run.start:run.end]
+            # (.data: a material may write to its fragments without touching the version of the others')
+            self.vi_data = run.layer.frag[run.start:run.end].data
+            self._from_run = self.vi_data, self.indices
         elif pixels is None:
             self.indices = mask.nonzero(as_tuple=True)
             self.vi_data = rast[self.indices]
@@ -152,7 +154,8 @@ class MaskedSparseInterpolator:
         if P == 0:
             return values.new_zeros(0, C)
         rows = -(-P // _FRAG_ROW)
-        if self.run is not None and not (torch.is_grad_enabled() and values.requires_grad):
+        if (self.run is not None and self.vi_data is self._from_run[0]
+                and not (torch.is_grad_enabled() and values.requires_grad)):
             # whole rows of the layer's fragments: what follows the run (other owners' fragments, then
             # zeros) is interpolated and cut off
             s = self.run.start
@@ -165,6 +168,12 @@ class MaskedSparseInterpolator:
         frag = frag.view(1, rows, -1, 4)
         out, _ = nvdr.interpolate(values.float().contiguous(), frag, self.tris)
         return out.view(-1, C)[:P]
+
+    def pixel_run(self) -> Optional['_Run']:
+        """The run ``indices`` are, unless they or the fragments were replaced since."""
+        if self.run is None or self.vi_data is not self._from_run[0] or self.indices is not self._from_run[1]:
+            return None
+        return self.run
 
 
 @dataclass
@@ -184,8 +193,8 @@ class _Run:
     end: int
 
     def indices(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-        return (self.layer.zero.expand(self.end - self.start), self.layer.rows[self.start:self.end],
-                self.layer.cols[self.start:self.end])
+        return (self.layer.zero.expand(self.end - self.start), self.layer.rows[self.start:self.end].data,
+                self.layer.cols[self.start:self.end].data)
 
 
 def _join_runs(runs: Sequence[Optional[_Run]]) -> Optional[_Run]:
@@ -615,7 +624,8 @@ class SurfaceDeferredRenderSession:
                     if v is not None:
                         idx.append(si.interpolator.indices)
                         vals.append(v)
-                        runs.append(getattr(si.interpolator, 'run', None))
+                        run_of = getattr(si.interpolator, 'pixel_run', None)  # (a material may bring its own)
+                        runs.append(run_of() if run_of is not None else None)
                 if not idx:
                     out.append(fill)
                 elif len(idx) == 1:
