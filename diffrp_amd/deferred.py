@@ -178,12 +178,24 @@ class MaskedSparseInterpolator:
 
 @dataclass
 class _LayerRuns:
-    """A layer's pixels in owner order: fragments [H*W (+ whole rows), 4], row and
-    column indices [H*W], one zero."""
+    """A layer's pixels in owner order, from the ``first``: fragments [n (+ whole
+    rows), 4], row and column indices [n], one zero."""
     frag: torch.Tensor
     rows: torch.Tensor
     cols: torch.Tensor
     zero: torch.Tensor
+    first: int = 0
+
+    def covered(self, background: int) -> '_LayerRuns':
+        """For the interpolators, which live as long as the session and take no
+        background (the first pixels): without it where it is most of the layer."""
+        if 2 * background <= self.rows.numel():
+            return self
+        return _LayerRuns(self.frag[background:].clone(), self.rows[background:].clone(),
+                          self.cols[background:].clone(), self.zero, background)
+
+    def run(self, start: int, end: int) -> '_Run':
+        return _Run(self, start - self.first, end - self.first) if end > start else _Run(self, 0, 0)
 
 
 @dataclass
@@ -584,6 +596,7 @@ class SurfaceDeferredRenderSession:
                 # the fragments come with the partition unless a gradient goes through them to rast
                 taped = rast.requires_grad or torch.autograd.forward_ad._current_level >= 0
                 order, runs, layer = _partition(rast, vao.stencils, n_obj, not taped)
+                layer = None if layer is None else layer.covered(runs[0][1])
             per_obj = []
             for i, obj in enumerate(self.scene.objects):
                 su = SurfaceUniform(obj.M, V, P)
@@ -592,7 +605,7 @@ class SurfaceDeferredRenderSession:
                 elif self.options.interpolator_impl == 'stencil_masked':
                     s, e = runs[i + 1]
                     if layer is not None:
-                        interp = MaskedSparseInterpolator(rast, vao.tris, run=_Run(layer, s, e))
+                        interp = MaskedSparseInterpolator(rast, vao.tris, run=layer.run(s, e))
                     else:
                         interp = MaskedSparseInterpolator(rast, vao.tris, pixels=order[s:e])
                     si = SurfaceInput(su, vao, interp)
