@@ -299,6 +299,7 @@ __device__ __forceinline__ int xcd_deal(int bid, int group) {
 constexpr int kXcdPixels = 32, kXcdVerts = 16;
 inline int xcd_group(long long blocks, int n_img, int few) {
     if (n_img >= 8) return (int)((blocks + 7) / 8);
+    if (blocks > (1ll << 24) - 1024) return 1;  // a turn's padding could take 256-thread blocks past 2^32 threads
     const long long turn = blocks / 32;
     return turn < 1 ? 1 : (turn < few ? (int)turn : few);
 }
@@ -306,5 +307,10 @@ inline long long xcd_pad(long long blocks, int group) {
     const long long unit = 8ll * group;
     return (blocks + unit - 1) / unit * unit;
 }
+
+// Blocks of 256 threads along a grid's x: a launch takes fewer than 2^32 threads
+// in one dimension, with room here for an XCD deal's padding.  More work goes in
+// several launches, or along another dimension.
+constexpr long long kMaxBlocks = 1ll << 23;
 
 }  // namespace drp

@@ -185,11 +185,12 @@ __device__ __forceinline__ void gather_pos(const PosGather &G, int blk, int oimg
 }
 
 // Neighbouring vertices, whose corners' rows share cache lines, on one XCD.
+// (Grid: blocks, outputs, further blocks.)
 __global__ void __launch_bounds__(256) k_gather_attr_q(AttrGather A) {
-    gather_attr_q(A, xcd_deal(blockIdx.x, A.xcd), blockIdx.y);
+    gather_attr_q(A, xcd_deal(blockIdx.x + gridDim.x * blockIdx.z, A.xcd), blockIdx.y);
 }
 __global__ void __launch_bounds__(256) k_gather_attr_c(AttrGather A) {
-    gather_attr_c(A, xcd_deal(blockIdx.x, A.xcd), blockIdx.y);
+    gather_attr_c(A, xcd_deal(blockIdx.x + gridDim.x * blockIdx.z, A.xcd), blockIdx.y);
 }
 __global__ void __launch_bounds__(256) k_gather_pos(PosGather G) {
     gather_pos(G, xcd_deal(blockIdx.x, G.xcd), blockIdx.y);
@@ -296,15 +297,20 @@ static PosGather pos_gather(const float *partial, const unsigned char *live, int
     return {(const float4 *)partial, live, n_img, F, V, pos_batched, xcd, inc_off, inc, (float4 *)grad_pos, 0};
 }
 
+static void launch_attr(const AttrGather &A, unsigned blocks, int outs, hipStream_t st) {
+    const unsigned x = blocks < kMaxBlocks ? blocks : (unsigned)kMaxBlocks;
+    const dim3 grid(x, outs, (blocks + x - 1) / x);
+    if (A.nc % 4 == 0) hipLaunchKernelGGL(k_gather_attr_q, grid, dim3(256), 0, st, A);
+    else hipLaunchKernelGGL(k_gather_attr_c, grid, dim3(256), 0, st, A);
+}
+
 int launch_gather_attr(const float *partial, const unsigned char *live, int groups, int F, int V, int C, int ldc,
                        int c0, int outs, int per_output, const int *inc_off, const int *inc, float *grad_attr,
                        hipStream_t st) {
     if (V == 0) return 0;
     unsigned blocks;
     const AttrGather A = attr_gather(partial, live, groups, F, V, C, ldc, c0, per_output, inc_off, inc, grad_attr, groups, blocks);
-    const dim3 grid(blocks, outs);
-    if (C % 4 == 0) hipLaunchKernelGGL(k_gather_attr_q, grid, dim3(256), 0, st, A);
-    else hipLaunchKernelGGL(k_gather_attr_c, grid, dim3(256), 0, st, A);
+    launch_attr(A, blocks, outs, st);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -340,9 +346,8 @@ int launch_gather_both(const TriBwdLaunch &T, int C, const int *inc_off, const i
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }
     const unsigned long long blocks = na + (unsigned long long)np * (T.b.pos_batched ? T.n_img : 1);
-    if (blocks >= (1ull << 31)) {  // past one launch's blocks
-        if (C % 4 == 0) hipLaunchKernelGGL(k_gather_attr_q, dim3(na), dim3(256), 0, st, A);
-        else hipLaunchKernelGGL(k_gather_attr_c, dim3(na), dim3(256), 0, st, A);
+    if (blocks >= (unsigned long long)kMaxBlocks) {  // past one launch's blocks
+        launch_attr(A, na, 1, st);
         hipLaunchKernelGGL(k_gather_pos, dim3(np, T.b.pos_batched ? T.n_img : 1), dim3(256), 0, st, G);
         return hipGetLastError() == hipSuccess ? 0 : -2;
     }

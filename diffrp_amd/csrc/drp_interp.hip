@@ -43,7 +43,8 @@ constexpr int interp_lanes() { return !QUADS || CV == 4 || CV == 8 ? 1 : 4; }
 template <int CV, bool QUADS>
 __global__ void __launch_bounds__(256) k_interp_fwd(const float *__restrict__ attr, int V, int C, int attr_batched,
                                                     const float4 *__restrict__ rast, const int *__restrict__ tri,
-                                                    int F, long long total_pix, long long pix_per_img,
+                                                    int F, long long first_pix, long long total_pix,
+                                                    long long pix_per_img,
                                                     float *__restrict__ out, const float4 *__restrict__ rast_db,
                                                     const int *__restrict__ diff_idx, int n_diff,
                                                     float *__restrict__ out_da) {
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(256) k_interp_fwd(const float *__restrict__ at
     const int NC = CV > 0 ? CV : C;
     // groups of blocks dealt to the XCDs: neighbouring pixels share their vertices' rows in one L2
     const long long gt = (long long)xcd_deal(blockIdx.x, kXcdPixels) * blockDim.x + threadIdx.x;
-    const long long gid = gt / LP;
+    const long long gid = first_pix + gt / LP;
     const int lane = (int)(gt % LP);
     if (gid >= total_pix) return;
     InterpPix p = interp_pix(rast, tri, gid, F, V);
@@ -174,10 +175,14 @@ __global__ void __launch_bounds__(256) k_interp_bwd(const float *__restrict__ at
 
 template <int CV, bool QUADS>
 static void launch_fwd(const InterpLaunch &L, hipStream_t st) {
-    const long long blocks = (L.total_pix * interp_lanes<CV, QUADS>() + 255) / 256;
-    hipLaunchKernelGGL((k_interp_fwd<CV, QUADS>), dim3((unsigned)xcd_pad(blocks, kXcdPixels)), dim3(256), 0, st, L.attr, L.V,
-                       L.C, L.attr_batched, (const float4 *)L.rast, L.tri, L.F, L.total_pix, L.pix_per_img, L.out,
-                       (const float4 *)L.rast_db, L.diff_idx, L.n_diff, L.out_da);
+    constexpr long long most = kMaxBlocks * 256 / interp_lanes<CV, QUADS>();  // pixels of a launch
+    for (long long first = 0; first < L.total_pix; first += most) {
+        const long long end = first + most < L.total_pix ? first + most : L.total_pix;
+        const long long blocks = ((end - first) * interp_lanes<CV, QUADS>() + 255) / 256;
+        hipLaunchKernelGGL((k_interp_fwd<CV, QUADS>), dim3((unsigned)xcd_pad(blocks, kXcdPixels)), dim3(256), 0, st,
+                           L.attr, L.V, L.C, L.attr_batched, (const float4 *)L.rast, L.tri, L.F, first, end,
+                           L.pix_per_img, L.out, (const float4 *)L.rast_db, L.diff_idx, L.n_diff, L.out_da);
+    }
 }
 
 int launch_interpolate(const InterpLaunch &L, hipStream_t st) {

@@ -513,23 +513,31 @@ __global__ void __launch_bounds__(256) k_sample3d_bwd(const float *__restrict__ 
 
 int launch_sample2d(const float *tex, int H, int W, int C, const float *uv, long long n, int wrap, int mode,
                     float *out, hipStream_t st) {
-    if (n == 0) return 0;
-    dim3 grid((unsigned)xcd_pad((n + 255) / 256, kXcdPixels));
-    DRP_TEX_DISPATCH(k_sample2d_fwd, tex, H, W, C, uv, n, wrap, mode, out)
+    const long long most = kMaxBlocks * 256;  // samples of a launch
+    for (; n > 0; n -= most, uv += 2 * most, out += (long long)C * most) {
+        const long long k = n < most ? n : most;
+        dim3 grid((unsigned)xcd_pad((k + 255) / 256, kXcdPixels));
+        DRP_TEX_DISPATCH(k_sample2d_fwd, tex, H, W, C, uv, k, wrap, mode, out)
+    }
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 int launch_sample2d_bwd(const float *tex, int H, int W, int C, const float *uv, long long n, int width, int wrap,
                         int mode, const float *gout, float *gtex, float *guv, hipStream_t st) {
-    if (n == 0) return 0;
-    long long blocks = (n + 255) / 256;
-    if (width < 16) width = 0;  // narrower rows leave most of a 16 x 16 block idle
-    else blocks = (long long)((width + 15) / 16) * (((n + width - 1) / width + 15) / 16);
-    if (blocks >= (1ll << 31) - 8 * kXcdPixels) return -1;
-    dim3 grid((unsigned)xcd_pad(blocks, kXcdPixels));
-    if (mode == kModeBicubic) DRP_TEX_DISPATCH_M(kModeBicubic, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
-    else if (mode == kModeNearest) DRP_TEX_DISPATCH_M(kModeNearest, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
-    else DRP_TEX_DISPATCH_M(kModeBilinear, tex, H, W, C, uv, n, width, wrap, gout, gtex, guv)
+    const long long most = kMaxBlocks * 256;  // samples of a launch
+    long long tiles = 0;
+    if (width >= 16) {  // narrower rows leave most of a 16 x 16 block idle
+        tiles = (long long)((width + 15) / 16) * (((n + width - 1) / width + 15) / 16);
+        if (tiles > kMaxBlocks) tiles = 0;
+    }
+    if (!tiles) width = 0;
+    for (; n > 0; n -= most, uv += 2 * most, gout += (long long)C * most, guv = guv ? guv + 2 * most : nullptr) {
+        const long long k = tiles || n < most ? n : most;
+        dim3 grid((unsigned)xcd_pad(tiles ? tiles : (k + 255) / 256, kXcdPixels));
+        if (mode == kModeBicubic) DRP_TEX_DISPATCH_M(kModeBicubic, tex, H, W, C, uv, k, width, wrap, gout, gtex, guv)
+        else if (mode == kModeNearest) DRP_TEX_DISPATCH_M(kModeNearest, tex, H, W, C, uv, k, width, wrap, gout, gtex, guv)
+        else DRP_TEX_DISPATCH_M(kModeBilinear, tex, H, W, C, uv, k, width, wrap, gout, gtex, guv)
+    }
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -64,7 +64,7 @@ class _SampleFunc(torch.autograd.Function):
         C = tex_c.shape[-1]
         L = _lib.lib()
         if dims == 2:
-            width = tc.shape[-2] if tc.dim() > 2 else 0  # samples of an image: its row width
+            width = tc.shape[-2] if tc.dim() > 2 and tc.shape[-2] < 1 << 31 else 0  # samples of an image: its row width
             rc = L.drp_sample2d_image_bwd(stream_of(tex_c), ptr(tex_c), tex_c.shape[0], tex_c.shape[1], C, ptr(tc), n,
                                           width, wrap, mode, ptr(g), ptr(gtex), ptr(gtc))
         else:
