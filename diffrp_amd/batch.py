@@ -384,7 +384,9 @@ class _URasterize(torch.autograd.Function):
         return _rasterize_bwd(ub.plan, pos, ub.tri, rast, False, grast, None, boxes, ub.inc), None
 
 
-_FUSED_C = (1, 2, 3, 4, 8, 16)  # channel counts of the fused attribute + position backward (tests switch it off)
+# channel counts of the fused attribute + position backward: those that the batch's own attribute
+# backward takes, which runs instead where rast's gradient is seen (tests switch the fused one off)
+_FUSED_C = (1, 2, 3, 4, 8, 16)
 
 
 class _UInterpolate(torch.autograd.Function):
