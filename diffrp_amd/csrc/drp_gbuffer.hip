@@ -51,6 +51,7 @@ __device__ __forceinline__ void wave_owners(const PartitionLaunch &L, long long 
             const int first = __ffsll((long long)left) - 1, o = __builtin_amdgcn_readlane(own[i], first);
             const unsigned long long m = __ballot(own[i] == o);
             if (lane == first) cnt[o] += __popcll(m);
+            wave_lds_sync();  // another lane may count this owner next
             left &= ~m;
         }
     }
@@ -130,10 +131,12 @@ __global__ void __launch_bounds__(256) k_owner_place(PartitionLaunch L, int n_bl
             const int first = __ffsll((long long)left) - 1, o = __builtin_amdgcn_readlane(own[i], first);
             const unsigned long long m = __ballot(own[i] == o);
             const int base = next[o];
+            wave_lds_sync();  // read by every lane, then moved on by one
             const int rank = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
             if (own[i] == o) place_pixel(L, base + rank, p0 + i * 64 + lane);
             if (lane == first) next[o] = base + __popcll(m);
+            wave_lds_sync();
             left &= ~m;
         }
     }

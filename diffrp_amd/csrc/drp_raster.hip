@@ -203,11 +203,11 @@ __global__ void __launch_bounds__(256) k_setup_bin(Batch b, const float *__restr
         const int p = r0 + lane;
         const bool active = p < total;
         own[lane] = 0;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         if (mine > 0 && excl < r0 + 64 && incl > r0) own[max(excl - r0, 0)] = lane;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         const int sl = wave_incl_max(own[lane]);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         const int k = p - __shfl(excl, sl, 64);
         const unsigned f = __shfl(first, sl, 64);
         unsigned key = (kNoTile << 6) | (unsigned)lane;  // unique: the sorted lanes are a permutation

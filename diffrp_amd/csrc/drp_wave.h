@@ -56,6 +56,16 @@ __device__ __forceinline__ float group_max(float x) {
     return x;
 }
 
+// LDS words handed from lane to lane within a wave, without a block barrier: the
+// loads after see the stores before.  (The hardware keeps a wave's LDS accesses in
+// order; the fences keep the compiler to it, which may otherwise move or keep a
+// lane's load across another lane's store.)
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // lanes that keep the minimum in the bitonic step (size, stride)
 constexpr unsigned long long bitonic_min_mask(int size, int stride) {
     unsigned long long m = 0;
