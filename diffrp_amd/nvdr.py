@@ -471,6 +471,20 @@ def _views_per_group(n, F):
 
 
 _FUSED_C = tuple(range(1, 17))  # channel counts of the fused attribute + position backward
+_TILE_C = (1, 2, 3, 4, 8, 16)    # counts whose separate attribute backward is always the tile passes
+
+
+def _pixel_atomics(px, F, groups, C, nd):
+    """Whether the attribute backward of another channel count, or with derivative
+    gradients (nd), is cheaper by one atomic per pixel, corner and channel than by
+    the tile passes, which touch every triangle and vertex once per pass of up to
+    16 channels (4 with derivatives).  5.2M triangles, 5 channels, us by atomics
+    and by passes: 87 and 199 at 64^2, 106 and 227 at 256^2, 856 and 310 at 1024^2;
+    40 channels: 199 and 835, 504 and 919, 6304 and 1395; 3 channels with
+    derivatives: 95 and 149, 124 and 165, 1031 and 232.  The line lies where an image
+    covered to about a half costs the same either way."""
+    passes = -(-C // (4 if nd else 16))
+    return 12 * px * C * (2 if nd else 1) < groups * F * (passes + C / 8)
 
 
 class _InterpolateFunc(torch.autograd.Function):
@@ -536,10 +550,13 @@ class _InterpolateFunc(torch.autograd.Function):
         if nd and dda is None:
             dda = torch.zeros((n, H, W, 2 * nd), dtype=torch.float32, device=attr.device)
         off = inc = ws = None
-        ws_bytes = vpg = 0
+        ws_bytes = 0
+        vpg = _views_per_group(n, F)
+        groups = n if batched else -(-n // vpg)
+        if boxes is not None and (nd or C not in _TILE_C) and _pixel_atomics(n * H * W, F, groups, C, nd):
+            boxes = None
         if boxes is not None:
             off, inc = incidence(tri, V)
-            vpg = _views_per_group(n, F)
             ws_bytes = L.drp_interpolate_bwd_workspace_size(n, H, W, F, C, batched, vpg)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=attr.device)
         rc = L.drp_interpolate_bwd(stream_of(attr), ptr(attr), n, V, batched, C, ptr(rast), H, W, ptr(tri), F,
