@@ -412,17 +412,17 @@ class _UInterpolate(torch.autograd.Function):
             # pass, returned as the gradient of the rasterised positions (the
             # rasterize backward, linear in grad_rast, sees only rast's other consumers;
             # where a hook or the caller sees rast's gradient, it goes through rast)
-            some = ub.plan.n_pix > 0 and ub.plan.n_tri > 0 and ub.plan.n_vert > 0
-            new = torch.empty_like if some else torch.zeros_like  # (written whole)
-            gattr, gpos = new(attr), new(src_pos)
-            ws_bytes = L.drp_batch_interpolate_rasterize_bwd_workspace_size(ub.plan.host_ptr(), C)
-            ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=attr.device)
-            check(L.drp_batch_interpolate_rasterize_bwd_to(stream_of(attr), ub.plan.host_ptr(), ptr(ub.plan.dev),
-                                                        ptr(attr), C, ptr(src_pos), ptr(rast), ptr(ub.tri),
-                                                        ptr(gout), ptr(gattr), ptr(gpos), ptr(boxes),
-                                                        ptr(ub.inc[0]), ptr(ub.inc[1]), ptr(ws), ws_bytes, 3),
-                  'batch interpolate + rasterize backward')
-            return gattr, None, None, None, gpos
+            ws = nvdr._scratch(max(L.drp_batch_interpolate_rasterize_bwd_workspace_size(ub.plan.host_ptr(), C), 1),
+                               attr.device)
+            if ws is not None:  # (else the separate passes, which need less at a time)
+                some = ub.plan.n_pix > 0 and ub.plan.n_tri > 0 and ub.plan.n_vert > 0
+                new = torch.empty_like if some else torch.zeros_like  # (written whole)
+                gattr, gpos = new(attr), new(src_pos)
+                check(L.drp_batch_interpolate_rasterize_bwd_to(
+                    stream_of(attr), ub.plan.host_ptr(), ptr(ub.plan.dev), ptr(attr), C, ptr(src_pos), ptr(rast),
+                    ptr(ub.tri), ptr(gout), ptr(gattr), ptr(gpos), ptr(boxes), ptr(ub.inc[0]), ptr(ub.inc[1]), ptr(ws),
+                    ws.numel(), 3), 'batch interpolate + rasterize backward')
+                return gattr, None, None, None, gpos
         gattr = torch.zeros_like(attr)
         grast = torch.empty_like(rast)
         ws_bytes = L.drp_batch_interpolate_bwd_workspace_size(ub.plan.host_ptr(), C)

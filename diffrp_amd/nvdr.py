@@ -474,6 +474,19 @@ _FUSED_C = tuple(range(1, 17))  # channel counts of the fused attribute + positi
 _TILE_C = (1, 2, 3, 4, 8, 16)    # counts whose separate attribute backward is always the tile passes
 
 
+def _new_scratch(nbytes, device):
+    return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
+def _scratch(nbytes, device):
+    """Scratch of a route that another one can stand in for: None where the device
+    has no room for it."""
+    try:
+        return _new_scratch(nbytes, device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _pixel_atomics(px, F, groups, C, nd):
     """Whether the attribute backward of another channel count, or with derivative
     gradients (nd), is cheaper by one atomic per pixel, corner and channel than by
@@ -529,20 +542,20 @@ class _InterpolateFunc(torch.autograd.Function):
             # (linear in its grad_rast) sees only what rast's other consumers send.
             # (Where a hook or the caller sees rast's gradient, it is written and
             # goes through rast.)
-            # (attributes' and, without an antialias's share to add to, positions' gradients written whole)
-            new = torch.empty_like if n > 0 and V > 0 else torch.zeros_like
-            gattr = new(attr)
-            gpos = aa_gpos if aa_gpos is not None else new(src_pos)
-            off, inc = incidence(tri, V)
             vpg = _views_per_group(n, F)
-            ws_bytes = L.drp_interpolate_rasterize_bwd_workspace_size(n, H, W, F, C, vpg)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=attr.device)
-            rc = L.drp_interpolate_rasterize_bwd_to(stream_of(attr), ptr(attr), n, V, C, ptr(rast), H, W, ptr(tri), F,
-                                                 ptr(src_pos), int(src_pos.dim() == 3), ptr(dy), ptr(gattr), None,
-                                                 ptr(gpos), ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws_bytes,
-                                                    1 if aa_gpos is not None else 3)
-            check(rc, 'interpolate + rasterize backward')
-            return gattr, None, None, None, None, None, gpos
+            ws = _scratch(L.drp_interpolate_rasterize_bwd_workspace_size(n, H, W, F, C, vpg), attr.device)
+            if ws is not None:  # (else the separate passes, which need less at a time)
+                # attributes' and, without an antialias's share to add to, positions' gradients written whole
+                new = torch.empty_like if n > 0 and V > 0 else torch.zeros_like
+                gattr = new(attr)
+                gpos = aa_gpos if aa_gpos is not None else new(src_pos)
+                off, inc = incidence(tri, V)
+                rc = L.drp_interpolate_rasterize_bwd_to(
+                    stream_of(attr), ptr(attr), n, V, C, ptr(rast), H, W, ptr(tri), F, ptr(src_pos),
+                    int(src_pos.dim() == 3), ptr(dy), ptr(gattr), None, ptr(gpos), ptr(boxes), vpg, ptr(off), ptr(inc),
+                    ptr(ws), ws.numel(), 1 if aa_gpos is not None else 3)
+                check(rc, 'interpolate + rasterize backward')
+                return gattr, None, None, None, None, None, gpos
         gattr = torch.zeros_like(attr)
         grast = torch.empty_like(rast)
         gdb = torch.empty_like(rast) if nd else None
@@ -553,12 +566,16 @@ class _InterpolateFunc(torch.autograd.Function):
         ws_bytes = 0
         vpg = _views_per_group(n, F)
         groups = n if batched else -(-n // vpg)
-        if boxes is not None and (nd or C not in _TILE_C) and _pixel_atomics(n * H * W, F, groups, C, nd):
+        either = nd or C not in _TILE_C  # by tile passes or by atomics
+        if boxes is not None and either and _pixel_atomics(n * H * W, F, groups, C, nd):
             boxes = None
         if boxes is not None:
-            off, inc = incidence(tri, V)
             ws_bytes = L.drp_interpolate_bwd_workspace_size(n, H, W, F, C, batched, vpg)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=attr.device)
+            ws = (_scratch if either else _new_scratch)(ws_bytes, attr.device)
+            if ws is None:
+                boxes, ws_bytes = None, 0
+            else:
+                off, inc = incidence(tri, V)
         rc = L.drp_interpolate_bwd(stream_of(attr), ptr(attr), n, V, batched, C, ptr(rast), H, W, ptr(tri), F,
                                    ptr(rast_db), ptr(diff_idx), nd, ptr(dy), ptr(dda), ptr(gattr), ptr(grast),
                                    ptr(gdb), ptr(boxes), vpg, ptr(off), ptr(inc), ptr(ws), ws_bytes)
