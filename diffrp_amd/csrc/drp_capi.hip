@@ -1068,7 +1068,7 @@ int drp_edge_grad_bwd(void *stream, const float *grad_out, const float *rgb, int
 
 int drp_compose_layer_fwd(void *stream, const float *rgba, const float *rast,
                           const float *out_prev, const float *trans_prev, long long n_pix, float *out, float *trans) {
-    if (n_pix < 0 || n_pix >= (1ll << 39)) return fail(-1, "pixel count out of range");
+    if (n_pix < 0 || n_pix > kMaxBlocks * 256) return fail(-1, "pixel count out of range");  // of one launch
     if (n_pix == 0) return 0;
     if (!rgba || !rast || !out || !trans || !out_prev != !trans_prev) return fail(-1, "null pointer argument");
     if (!aligned16(rgba)) return fail(-1, "rgba must be 16-byte aligned");
@@ -1080,7 +1080,7 @@ int drp_compose_layer_fwd(void *stream, const float *rgba, const float *rast,
 int drp_compose_layer_bwd(void *stream, const float *rgba, const float *rast,
                           const float *trans_prev, long long n_pix, const float *grad_out, const float *grad_trans,
                           float *grad_rgba, float *grad_trans_prev) {
-    if (n_pix < 0 || n_pix >= (1ll << 39)) return fail(-1, "pixel count out of range");
+    if (n_pix < 0 || n_pix > kMaxBlocks * 256) return fail(-1, "pixel count out of range");  // of one launch
     if (n_pix == 0) return 0;
     if (!rgba || !rast || !grad_rgba || (grad_trans_prev && !trans_prev)) return fail(-1, "null pointer argument");
     if (!aligned16(rgba) || !aligned16(grad_rgba)) return fail(-1, "rgba and grad_rgba must be 16-byte aligned");

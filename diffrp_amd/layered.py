@@ -113,11 +113,14 @@ class _Compose(torch.autograd.Function):
         return grgba, None, go if out is not None else None, gtrans
 
 
+_COMPOSE_PIXELS = 1 << 31  # pixels of one launch
+
+
 def _compose(rgba, rast, out, trans):
     # the kernel takes plain float32 buffers; what shade returns otherwise (another type or shape, a
     # subclass, a forward-mode dual) goes through the operators
     if (type(rgba) is torch.Tensor and rgba.dtype == torch.float32 and rgba.shape == rast.shape
-            and rgba.device == rast.device and rast.is_contiguous()
+            and rgba.device == rast.device and rast.is_contiguous() and rast.numel() <= 4 * _COMPOSE_PIXELS
             and (out is None or (out.dtype == torch.float32 and out.is_contiguous() and trans.is_contiguous()))
             and torch.autograd.forward_ad._current_level < 0):
         # kept for the backward: a copy, as the operators keep (shade may write to its buffer again, and a

@@ -235,8 +235,8 @@ int drp_stencil_fragments(void *stream, const float *rast, int H, int W, const i
  * torch operators, diffrp/rendering/surface_deferred.py:348-395): with rgba
  * masked by the layer's coverage (rast [n_pix,4], id > 0) and T = trans_prev,
  * out = out_prev + (T a) rgb and trans = T (1 - a); out_prev and trans_prev are
- * both NULL at the first layer (0 and 1).  rgba [n_pix,4], 16-byte aligned;
- * out [n_pix,3], trans [n_pix].  Backward:
+ * both NULL at the first layer (0 and 1).  n_pix is at most 2^31; rgba
+ * [n_pix,4] 16-byte aligned; out [n_pix,3], trans [n_pix].  Backward:
  * grad_rgba [n_pix,4] and grad_trans_prev [n_pix] (nullable) written; the
  * gradient of out_prev is grad_out.  grad_out, grad_trans nullable (zero). */
 int drp_compose_layer_fwd(void *stream, const float *rgba, const float *rast,
