@@ -15,7 +15,9 @@ composed images are flipped to top row first; background takes the G-buffer
 default value with alpha 0; a session caches every query (one camera, one
 scene snapshot).
 """
+import ctypes
 import functools
+import math
 import threading
 from dataclasses import dataclass, field
 from typing import Callable, Dict, List, Optional, Sequence, Tuple, Union
@@ -179,20 +181,26 @@ class MaskedSparseInterpolator:
 @dataclass
 class _LayerRuns:
     """A layer's pixels in owner order, from the ``first``: fragments [n (+ whole
-    rows), 4], row and column indices [n], one zero."""
+    rows), 4], row and column indices [2, n], one zero."""
     frag: torch.Tensor
-    rows: torch.Tensor
-    cols: torch.Tensor
+    rc: torch.Tensor
     zero: torch.Tensor
     first: int = 0
+
+    @property
+    def rows(self) -> torch.Tensor:
+        return self.rc[0]
+
+    @property
+    def cols(self) -> torch.Tensor:
+        return self.rc[1]
 
     def covered(self, background: int) -> '_LayerRuns':
         """For the interpolators, which live as long as the session and take no
         background (the first pixels): without it where it is most of the layer."""
-        if 2 * background <= self.rows.numel():
+        if 2 * background <= self.rc.shape[1]:
             return self
-        return _LayerRuns(self.frag[background:].clone(), self.rows[background:].clone(),
-                          self.cols[background:].clone(), self.zero, background)
+        return _LayerRuns(self.frag[background:].clone(), self.rc[:, background:].clone(), self.zero, background)
 
     def run(self, start: int, end: int) -> '_Run':
         return _Run(self, start - self.first, end - self.first) if end > start else _Run(self, 0, 0)
@@ -205,8 +213,8 @@ class _Run:
     end: int
 
     def indices(self) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-        return (self.layer.zero.expand(self.end - self.start), self.layer.rows[self.start:self.end].data,
-                self.layer.cols[self.start:self.end].data)
+        rows, cols = self.layer.rc[:, self.start:self.end].unbind()
+        return self.layer.zero.expand(self.end - self.start), rows.data, cols.data
 
 
 def _join_runs(runs: Sequence[Optional[_Run]]) -> Optional[_Run]:
@@ -237,7 +245,7 @@ def _partition(rast: torch.Tensor, stencils: torch.Tensor, n_owner: int, fragmen
     check(L.drp_stencil_fragments(stream_of(rast), ptr(rast), H, W, ptr(st), st.numel() - 1, n_owner, ptr(order),
                                   ptr(frag), frag.shape[0], ptr(rc[0]), ptr(rc[1]), ptr(se[0]), ptr(se[1]), ptr(ws),
                                   ws_bytes), 'stencil partition')
-    layer = _LayerRuns(frag, rc[0], rc[1], torch.zeros(1, dtype=torch.int64, device=rast.device))
+    layer = _LayerRuns(frag, rc, torch.zeros(1, dtype=torch.int64, device=rast.device))
     return order, se.cpu().t().tolist(), layer
 
 
@@ -475,11 +483,10 @@ class SurfaceDeferredRenderSessionOptions:
 def _fill_value(default: Sequence[float], dev) -> torch.Tensor:
     """[C] of ``default`` on the device by fill kernels (copying it from host memory
     waits for the stream)."""
-    host = torch.tensor([float(x) for x in default], dtype=torch.float32)  # (past float32's range: infinite)
-    vals, bits = host.tolist(), host.view(torch.int32).tolist()
+    vals = [ctypes.c_float(float(x)).value for x in default]  # (past float32's range: infinite)
     v = torch.full((len(vals),), vals[0] if vals else 0.0, dtype=torch.float32, device=dev)
     for i, x in enumerate(vals):
-        if bits[i] != bits[0]:  # (0.0 and -0.0 differ)
+        if x != vals[0] or math.copysign(1.0, x) != math.copysign(1.0, vals[0]):  # (0.0 and -0.0 differ)
             v[i].fill_(x)
     return v
 
