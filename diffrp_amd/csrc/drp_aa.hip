@@ -288,11 +288,6 @@ __device__ __forceinline__ PairRes eval_pair(const AAImg &I, const int *__restri
     return res;
 }
 
-// signed pair weight: > 0 b receives from a, < 0 a receives from b
-__device__ __forceinline__ float signed_w(const PairRes &p) {
-    return p.recv < 0 ? 0.f : (p.recv == 1 ? p.wgt : -p.wgt);
-}
-
 __device__ __forceinline__ AAImg aa_img(const AALaunch &L, int img) {
     AAImg I;
     if (L.um.n) {  // uneven batch: the item's pixels; vertices and triangles are global
@@ -426,7 +421,8 @@ __device__ __forceinline__ unsigned long long readlane64(unsigned long long v, i
 // Channels handled by one thread: 4 (one float4) when C is a multiple of 4, a whole
 // pixel below 8 channels (a wave's accesses still cover whole lines, and the
 // pixel's weights are read once: 24 views of 361 x 641 x 3, 126 -> 115 us; 3 of 733 x
-// 1019 x 5, 52 -> 37 us forward and 54 -> 44 backward), else 1.
+// 1019 x 5, 52 -> 37 us forward and 54 -> 44 backward), else 1 (9 channels and more that are
+// no whole quads: whole pixels were not tried there).
 // CV > 0: compile-time channel count; 0: runtime; kAnyQuads: runtime, a multiple of 4
 constexpr int kAnyQuads = -4;
 template <int CV>
@@ -720,10 +716,12 @@ __global__ void __launch_bounds__(256, 8) k_aa_fwd(AALaunch L) {
 // Per-block accumulation of vertex gradients before the global atomics.
 // Device-scope float atomics on a multi-XCD GPU are performed beyond the
 // per-XCD L2 caches, so every one is a memory transaction; neighbouring
-// silhouette pairs share vertices, and summing them per 32 x 32 tile first
+// silhouette pairs share vertices, and summing them per 64 x 8 block first
 // leaves one atomic per distinct vertex and component.
 constexpr int kAAHashBits = 9;
-constexpr int kAAHash = 1 << kAAHashBits;  // table slots per tile (a 32 x 32 tile touches ~50-100 vertices)
+// table slots per block: its pairs touch 41 vertices on average at 512^2 with 82k triangles (119 at most), 163 at
+// 361 x 641 with 328k (309 at most)
+constexpr int kAAHash = 1 << kAAHashBits;
 
 struct VertexAcc {
     int key[kAAHash];
@@ -834,6 +832,8 @@ __device__ __forceinline__ void pair_grad_add(VertexAcc &A, float *GP, const Pai
 // in the block's table and flushed with one atomic request per vertex.  One
 // kernel for both, so that the pairs find output gradients in the caches: 343 us
 // at 64 x 512^2 x 8, against 430 for a colour and a position kernel side by side.
+// Eight waves per SIMD as the forward (at 16 channels two VGPRs spill for it, 12
+// bytes of scratch a lane).
 template <int CV>
 __global__ void __launch_bounds__(256, 8) k_aa_bwd(AALaunch L) {
     __shared__ VertexAcc A;

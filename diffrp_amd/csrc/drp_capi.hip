@@ -292,8 +292,8 @@ static size_t plan_desc_off() { return (sizeof(BatchPlanHeader) + 15) & ~(size_t
 static size_t plan_t2i_off(int n_img) { return plan_desc_off() + (size_t)n_img * sizeof(ImageDesc); }
 // item map (UnevenMap) after the tile -> image table: pixel prefix (int64), the
 // vertex, triangle, 16 x 16 tile, 64 x 8 block and 32 x 32 tile prefixes
-// (int32, n + 1 each; no kernel reads the last, it holds the format), then
-// (H, W) per item
+// (int32, n + 1 each; no kernel reads the last, it holds the format, and it
+// never exceeds the 16 x 16 one), then (H, W) per item
 static size_t plan_map_off(int n_img, long long n_tiles) {
     return (plan_t2i_off(n_img) + sizeof(int32_t) * (size_t)n_tiles + 15) & ~(size_t)15;
 }
@@ -374,7 +374,7 @@ int drp_batch_plan(const int32_t *items, int n_img, int tile_w, int tile_h, void
             k += (long long)((W + kAAW - 1) / kAAW) * ((H + kAAH - 1) / kAAH);
             c += (long long)((W + 31) / 32) * ((H + 31) / 32);
         }
-        if (a > 0x7fffffffll || k > 0x7fffffffll || c > 0x7fffffffll) return fail(-1, "batch too large");
+        if (a > 0x7fffffffll || k > 0x7fffffffll) return fail(-1, "batch too large");
     }
     vb = fb = pb = tb = sb = 0;
     for (int i = 0; i < n_img; ++i) {

@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256) k_sample2d_fwd(const float *__restrict__ 
 // atomic per tap and channel, 0.151 ms so.  What remains is the LDS atomics
 // (12 per covered sample) and the scattered texel reads of the coordinate
 // gradient.
-constexpr int kTexTile = 4096;  // floats (16 KiB: ten blocks per CU)
+constexpr int kTexTile = 4096;  // floats (16 KiB and the box: the eight blocks that a CU's wave slots hold fit its LDS)
 
 struct TexGrad {
     float *tile;        // LDS box, or nullptr

@@ -122,16 +122,6 @@ __device__ __forceinline__ unsigned long long wave_sort(unsigned long long k) { 
     return k;
 }
 
-// sum over the wave, in every lane
-__device__ __forceinline__ float wave_sum(float x) {
-    x += lane_xor<1>(x);
-    x += lane_xor<2>(x);
-    x += lane_xor<4>(x);
-    x += lane_xor<8>(x);
-    x += lane_xor<16>(x);
-    return x + lane_xor<32>(x);
-}
-
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int scan_step(int x) {  // lanes without a source add 0
     return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);

@@ -129,7 +129,7 @@ int drp_rasterize_batch_fwd(void *stream, const float *pos, const int32_t *tri, 
  * table (drp_topology_build), boxes from the rasterize call, inc_off / inc the
  * incidence table of tri (drp_incidence_build).  Gradients are summed in fixed
  * orders without atomics, except the antialias position gradient (one float
- * atomic per vertex component and 32 x 32 tile).  grad_attr, grad_pos are
+ * atomic per vertex component and 64 x 8 block).  grad_attr, grad_pos are
  * accumulated (caller zero-fills); grad_rast, grad_color written.  The
  * interpolate backward takes C in {1, 2, 3, 4, 8, 16}.  The rasterize
  * backward also takes the item-local ids of global_ids = 0 (local_ids = 1),
