@@ -2,10 +2,18 @@
 the gradient of its intermediate: a function of the fused form (the gradient of
 y = 2 x left out, that of x returned on a side input in its place) gives every
 caller what the unfused one gives."""
+import os
+
 import pytest
 import torch
 
-from diffrp_amd import _lib
+from diffrp_amd import _lib, build_ext
+
+
+@pytest.fixture(scope='module', autouse=True)
+def built():
+    if not os.path.exists(build_ext.AUTOGRAD_LIB_PATH):
+        build_ext.build()
 
 
 class _Double(torch.autograd.Function):
