@@ -47,8 +47,9 @@ constexpr int kAttrLanes = 4;
 // incident corners, channel counts that are whole quads, with `lanes` lanes per
 // (vertex, four channels) (1, 2 or 4: up to the groups each output sums): lane
 // s takes groups s, s + lanes, ... (a group's corner rows in flight together,
-// summed in corner order), and the lanes' sums are added in a fixed tree.  (One lane per (vertex, quad) left the 64-view grid at barely one
-// wave per SIMD waiting on its loads.)
+// summed in corner order), and the lanes' sums are added in a fixed tree.  (One
+// lane per (vertex, quad) left the 64-view grid at barely one wave per SIMD
+// waiting on its loads.)
 __device__ __forceinline__ void gather_attr_q(const AttrGather &A, int blk, int out) {
     const float *__restrict__ partial = A.partial;
     const int *__restrict__ inc_off = A.inc_off, *__restrict__ inc = A.inc;
